@@ -525,22 +525,40 @@ __device__ __forceinline__ void count_work(unsigned long long* work, bool live, 
 
 // Forward with one lane per pair slot (the reverse's slot order) and the aux records of the reverse
 // (centre-grouped, wave-uniform): block (s, g) of the 2-D grid (ceil(N / kFwdRecs), pair groups)
-// sums the pair slots [g kFwdPairs, (g + 1) kFwdPairs) against the kFwdRecs aux slots from
-// s kFwdRecs on. The record blocks (x) run fastest, so the workgroups dispatched together share
+// sums the `pairs` pair slots from g `pairs` on against the kFwdRecs aux slots from s kFwdRecs
+// on. The record blocks (x) run fastest, so the workgroups dispatched together share
 // their pair slots (read once into L2) and differ only in their aux records. (One dimension of a
 // grid holds at most 2^32 - 1 work-items: a 1-D grid of both would pass that at 20 M pairs.) The centre-dependent terms (d, Ah d, q0..q2)
 // are formed once per centre and shared by its exponent scales, and the wave's node screen acts on
 // 64 pairs in precision band + Morton order. Each lane keeps its running sums of coef_a F(P, a) for
-// the block's records in LDS; at the end the 256 lane sums of each record are added in lane order
-// and scaled by KN_P (the record's u): partial[g * N + slot]. Twelve records per block keep the
+// the block's records in LDS; at the end the 256 lane sums of each record are added in a fixed
+// order and scaled by KN_P (the record's u): partial[g * N + slot]. Twelve records per block keep the
 // LDS at 26 KB, so six workgroups (six waves per SIMD, within the kernel's 60 registers) share a
 // CU; 16 records (34 KB, four waves per SIMD) were 1.9% slower and 8 or 10 records 0.9% and 1.6%.
-// The sums do not depend on the block size: each lane adds its pairs to a record's sum in the
-// same order, and the lanes are added in lane order.
+// The sums do not depend on the records per block: each lane adds its pairs to a record's sum in
+// the same order.
 constexpr int kFwdRecs = 12;
 constexpr int64_t kFwdPairs = 8192;
 
-__global__ __launch_bounds__(256) void k_gamma_fwd_pairs(int64_t n,
+// Pair slots per forward block: kFwdPairs while the launch has kFwdBlocks blocks or more, else
+// halved (to 256 at least, and to no fewer than N / 8, so that the block sums, ceil(n / pairs) N
+// doubles, stay within the dead pair records' 16 n). A CU holds six blocks, so 1536 are one round
+// of the chip; a small system has fewer (CO2, 504 aux x 7893 pairs: 42 blocks of 8192 slots left
+// the chip idle, 857 us against 88 us with 1302 blocks of 256), and many rounds keep the uneven
+// last one short (2400 aux x 167 k pairs: 4200 blocks against 32800, the step 2% faster; 2434 x
+// 260 k: gamma 6%). At 33000 blocks and more the size makes no difference.
+constexpr int64_t kFwdBlocks = 32768;
+inline int64_t fwd_pairs(int64_t N, int64_t n) {
+    const int64_t nrb = (N + kFwdRecs - 1) / kFwdRecs;
+    int64_t p = kFwdPairs;
+    while (p > 256 && p / 2 >= N / 8 && nrb * ((n + p - 1) / p) < kFwdBlocks) p /= 2;
+    return p;
+}
+inline int64_t fwd_groups(int64_t N, int64_t n) {
+    return n > 0 ? (n + fwd_pairs(N, n) - 1) / fwd_pairs(N, n) : 1;
+}
+
+__global__ __launch_bounds__(256) void k_gamma_fwd_pairs(int64_t n, int64_t pairs,
                                                          const double* __restrict__ rec,
                                                          int64_t N,
                                                          const double* __restrict__ aux,
@@ -554,8 +572,8 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_pairs(int64_t n,
     __syncthreads();
     const int64_t q0 = (int64_t)blockIdx.x * kFwdRecs, g = blockIdx.y;
     const int nrec = (int)min((int64_t)kFwdRecs, N - q0);
-    const int64_t a_begin = g * kFwdPairs;
-    const int64_t a_end = min(n, a_begin + kFwdPairs);
+    const int64_t a_begin = g * pairs;
+    const int64_t a_end = min(n, a_begin + pairs);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const double c256 = vgpr_const(kNegC256);
     uint64_t lane_nodes = 0;                 // profiling: node evaluations over live lanes
@@ -637,12 +655,15 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_pairs(int64_t n,
     }
     if (work && (threadIdx.x & 63) == 0) atomicAdd(work, (unsigned long long)lane_nodes);
     __syncthreads();
-    if ((int)threadIdx.x < nrec) {
-        double sum = 0.0;
-        for (int l = 0; l < 256; ++l) sum += acc[threadIdx.x][l];
-        partial[g * N + q0 + threadIdx.x] =
-            sum * aux[kAuxRec * (q0 + threadIdx.x) + 3];
-    }
+    // sixteen lanes per record: each adds sixteen of the 256 lane sums, then a butterfly
+    static_assert(kFwdRecs <= 16, "one record per sixteen lanes of the block");
+    const int j = threadIdx.x >> 4, part = threadIdx.x & 15;
+    double sum = 0.0;
+    if (j < nrec)
+        for (int l = 0; l < 16; ++l) sum += acc[j][16 * l + part];
+    for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    if (j < nrec && part == 0)
+        partial[g * N + q0 + j] = sum * aux[kAuxRec * (q0 + j) + 3];
 }
 
 // gamma[p] = sum over pair groups of partial[g * N + slot(p)], in group order.
@@ -652,6 +673,7 @@ __global__ void k_slot_sum(int64_t N, int64_t G, int64_t groups, const double* _
     if (p >= N) return;
     const int64_t q = aux_slot(p, N, G);
     double s = 0.0;
+#pragma unroll 8
     for (int64_t g = 0; g < groups; ++g) s += partial[g * N + q];
     gamma[p] = s;
 }
@@ -1953,12 +1975,13 @@ int layout_gamma(Arena& ar, int64_t M, int64_t N, int64_t n, bool reverse, Gamma
     w->q = ar.take<double>(n + 1);
     w->partial = w->aux = w->acc = w->contrib = w->rec_sorted = w->rec = nullptr;
     if (!reverse) {
-        w->rec = ar.take<double>(kRec * n + kRec);
-        const int64_t groups = n > 0 ? (n + kFwdPairs - 1) / kFwdPairs : 1;
+        // the unsorted pair records are dead once gathered into slot order, before any block sum
+        // is written, so both occupy one slice
+        w->rec = ar.take<double>(std::max(kRec * n + kRec, fwd_groups(N, n) * N + 1));
         w->aux = ar.take<double>(kAuxRec * N + kAuxRec);
         w->rec_sorted = ar.take<double>(kRec * n + kRec);
         GSDFT_TRY(pair_order_layout(ar, n, &w->pair_order));
-        w->partial = ar.take<double>(groups * N + 1);
+        w->partial = w->rec_sorted && w->pair_order.sort_tmp ? w->rec : nullptr;
     } else {
         // at least as many slabs as bwd_split's, which the nuclear pass launches with; the
         // unsorted pair records are dead once gathered into slot order, before any moment is
@@ -2821,14 +2844,14 @@ int gamma_run(int64_t M, const double* quat, const double* log_scale, const doub
     k_rec_gather<<<blocks_for(n * kRec, 256), 256, 0, s>>>(n, w.pair_order.perm, w.rec,
                                                             w.rec_sorted);
     GSDFT_HIP(hipGetLastError());
-    const int64_t groups = (n + kFwdPairs - 1) / kFwdPairs;
+    const int64_t groups = fwd_groups(N, n);
     const int64_t nrb = (N + kFwdRecs - 1) / kFwdRecs;
     if (nrb * 256 > (int64_t)UINT32_MAX || groups > kMaxGridY)
         return fail(GSDFT_ERR_ARG, "gsdft_gamma: N_aux = %lld or n = %lld too large for one launch",
                     (long long)N, (long long)n);
     const dim3 grid((unsigned)nrb, (unsigned)groups);
     if (profile) profile_begin(kProfGammaFwd, s);
-    k_gamma_fwd_pairs<<<grid, 256, 0, s>>>(n, w.rec_sorted, N, w.aux, w.partial,
+    k_gamma_fwd_pairs<<<grid, 256, 0, s>>>(n, fwd_pairs(N, n), w.rec_sorted, N, w.aux, w.partial,
                                            profile ? profile_work_counter(kProfGammaFwd)
                                                    : nullptr);
     if (profile) profile_end(kProfGammaFwd, s);
