@@ -203,9 +203,15 @@ def main() -> int:
     integrals = float(N) * float(n)
     fwd_tf = integrals * FLOPS_FWD / (fwd_ms * 1e-3)
     bwd_tf = integrals * FLOPS_BWD / (bwd_ms * 1e-3)
-    # What the kernels executed: the node screen leaves out nodes whose terms are below e^-36.
-    fwd_exec_tf = (integrals * FWD_PER_INTEGRAL + fwd_nodes * FWD_PER_NODE) / (fwd_ms * 1e-3)
-    bwd_exec_tf = (integrals * BWD_PER_INTEGRAL + bwd_nodes * BWD_PER_NODE) / (bwd_ms * 1e-3)
+    # What the kernels executed: the node screen leaves out nodes whose terms are below e^-36, and
+    # from 32768 pairs on the exponent scales of a centre share one node list (its centre terms
+    # once, each forward node added to every scale's sum).
+    scales = min(len(s.scales), 4) if n >= 32768 else 1
+    fwd_share, bwd_share = (scales if scales > 2 else 1), scales
+    fwd_fixed, bwd_fixed = FWD_PER_INTEGRAL / fwd_share, BWD_PER_INTEGRAL / bwd_share
+    fwd_node = FWD_PER_NODE + 2 * (fwd_share - 1)
+    fwd_exec_tf = (integrals * fwd_fixed + fwd_nodes * fwd_node) / (fwd_ms * 1e-3)
+    bwd_exec_tf = (integrals * bwd_fixed + bwd_nodes * BWD_PER_NODE) / (bwd_ms * 1e-3)
     fwd_node_frac = fwd_nodes / (NODES * integrals)
     bwd_node_frac = bwd_nodes / (NODES * integrals)
     log(f"E_J={E.item():.12e} step {wall * 1e3:.1f} ms; three-centre fwd {fwd_ms:.1f} ms "
@@ -215,10 +221,10 @@ def main() -> int:
         f"solves {solve_ms / max(args.steps, 1):.2f} ms")
     if bwd_ms >= fwd_ms:
         dom = ("reverse", "k_gamma_bwd", bwd_ms, FLOPS_BWD, bwd_tf, bwd_exec_tf, bwd_node_frac,
-               BWD_PER_INTEGRAL, BWD_PER_NODE)
+               bwd_fixed, BWD_PER_NODE)
     else:
         dom = ("forward", "k_gamma_fwd", fwd_ms, FLOPS_FWD, fwd_tf, fwd_exec_tf, fwd_node_frac,
-               FWD_PER_INTEGRAL, FWD_PER_NODE)
+               fwd_fixed, fwd_node)
     # HBM bytes of the dominant kernel from the copy-calibrated counter runs of this workload,
     # stored per step together with the kernel's launches per step (the reverse runs its aux
     # slabs in several launches when their moments do not fit one launch's budget).
@@ -315,7 +321,8 @@ def main() -> int:
                              "peak 78.6 TFLOP/s, no MFMA: the work is elementwise). achieved "
                              "counts the work the kernel has to do: flops_per_integral for "
                              "every (P, a) plus flops_per_evaluated_node for each node the "
-                             "e^-36 screen keeps (the kernel's own node counter); "
+                             "e^-36 screen keeps (the kernel's own node counter; the scales of "
+                             "a centre share one node list); "
                              "algorithmic_* credit all 20 nodes of every integral, skipped ones "
                              "included, and so can pass 1; fp64_counters holds the hardware "
                              "FP64 VALU instruction rate of the same kernel at this workload "

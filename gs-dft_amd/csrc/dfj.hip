@@ -473,8 +473,6 @@ __device__ __forceinline__ bool new_centre(const double* __restrict__ x) {
 // `scale` multiplies the weight (the record's u, for the reverse pass that folds it in). Stored
 // node-major from offset 8 (node t at 8 + 4 t): the four values a node reads are one 32-byte run,
 // a single scalar load, and two nodes share a cache line.
-constexpr double kExpMinusHalf = 0x1.368b2fc6f960ap-1;     // e^(-1/2), correctly rounded
-
 __host__ __device__ constexpr int rec_s(int t) { return 8 + 4 * t; }
 __host__ __device__ constexpr int rec_wh(int t) { return 8 + 4 * t + 1; }
 __host__ __device__ constexpr int rec_s2(int t) { return 8 + 4 * t + 2; }
@@ -499,6 +497,12 @@ __device__ __forceinline__ void put_fwd_node_consts(double* o, int t, double s, 
     o[rec_lw(t)] = fold_weight(wp / sqrt(s) * (kExpMinusHalf / kExpPolyK), &S);
     o[rec_S(t)] = S;
     o[rec_is(t)] = 1.0 / s;
+}
+
+// A wave-uniform read-only pointer in the constant address space: its loads are scalar loads.
+typedef const __attribute__((address_space(4))) double* UniformPtr;
+__device__ __forceinline__ UniformPtr uniform_ptr(const double* p) {
+    return (UniformPtr)(uintptr_t)p;
 }
 
 // body(std::integral_constant<int, t>) for t = 0, 1, ..., kN - 1 until it returns true: a fully
@@ -666,16 +670,138 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_pairs(int64_t n, int64_t pair
         partial[g * N + q0 + j] = sum * aux[kAuxRec * (q0 + j) + 3];
 }
 
-// gamma[p] = sum over pair groups of partial[g * N + slot(p)], in group order.
+// The forward on shared node lists (nodeset.hip): one list per centre serves the NB exponent scales
+// there, so a node is evaluated once and added to NB sums with the NB weights of the list. Blocks,
+// pair slots, the lanes' sums in LDS and their reduction are k_gamma_fwd_pairs'; the block's
+// kFwdRecs records are kFwdRecs / NB groups. Bound by its VALU instructions like
+// k_gamma_fwd_pairs: 26.5 a node (22 + NB; the weights' signs no longer let one ride in the
+// exponent) against 22 for each node of each scale, for about half the nodes (C20H42, 590 k pairs,
+// four scales: 44.5 -> 37.9 ms; water octamer 6.05 -> 4.36). One node a step, with its constants
+// moved between register sets, took 39.1 and 4.62. partial[g * N + slot] is the sum without KN_P
+// (k_slot_sum multiplies it in).
+template <int NB>
+__global__ __launch_bounds__(256) void k_gamma_fwd_sets(int64_t n, int64_t pairs,
+                                                        const double* __restrict__ rec, int64_t N,
+                                                        int64_t G, int64_t per_centre,
+                                                        int64_t ngroups, int64_t stride,
+                                                        const double* __restrict__ sets,
+                                                        double* __restrict__ partial,
+                                                        unsigned long long* __restrict__ work) {
+    constexpr int kGroups = kFwdRecs / NB, kNd = set_node_doubles(NB);
+    __shared__ double tab[256];
+    __shared__ double acc[kFwdRecs][256];
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) tab[i] = exp2_frac_lead(i);
+#pragma unroll
+    for (int j = 0; j < kFwdRecs; ++j) acc[j][threadIdx.x] = 0.0;
+    __syncthreads();
+    const int64_t gr0 = (int64_t)blockIdx.x * kGroups, g = blockIdx.y;
+    const int ngr = (int)min((int64_t)kGroups, ngroups - gr0);
+    const int64_t a_begin = g * pairs;
+    const int64_t a_end = min(n, a_begin + pairs);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    uint64_t lane_nodes = 0;                 // profiling: node evaluations over live lanes
+    for (int64_t a0 = a_begin + 64 * wave; a0 < a_end; a0 += 256) {      // wave-uniform
+        const int64_t a = a0 + lane;
+        const bool live = a < a_end;
+        const uint64_t lanes = __builtin_popcountll(__builtin_amdgcn_ballot_w64(live));
+        const double* __restrict__ r = rec + kRec * (live ? a : a0);
+        const double I1 = r[0], I2 = r[1], I3 = r[2];
+        const double xx = r[3], yy = r[4], zz = r[5], xy = r[6], xz = r[7], yz = r[8];
+        const double Px = live ? r[9] : kFarAway, Py = live ? r[10] : kFarAway,
+                     Pz = live ? r[11] : kFarAway;
+        const double coef = live ? r[12] : 0.0;
+        for (int j = 0; j < ngr; ++j) {
+            UniformPtr x = uniform_ptr(sets + stride * (gr0 + j));
+            bool last;
+            do {                                     // wave-uniform; once unless centres differ
+                const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
+                const int count = (int)(uint32_t)head;
+                last = (head >> 32) != 0;
+                const double dx = x[0] - Px, dy = x[1] - Py, dz = x[2] - Pz;
+                const double ax = __builtin_fma(xx, dx, __builtin_fma(xy, dy, xz * dz));
+                const double ay = __builtin_fma(xy, dx, __builtin_fma(yy, dy, yz * dz));
+                const double az = __builtin_fma(xz, dx, __builtin_fma(yz, dy, zz * dz));
+                const double q0d = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+                const double q1 = __builtin_fma(dx, ax, __builtin_fma(dy, ay, dz * az));
+                const double q2 = __builtin_fma(ax, ax, __builtin_fma(ay, ay, az * az));
+                const double X0 = I3 * q0d;
+                const double rr = __builtin_fma(I1, q1, -q2);
+                const double cf = (q0d == q0d) ? coef : q0d;      // a NaN centre propagates
+                double F[NB];
+#pragma unroll
+                for (int b = 0; b < NB; ++b) F[b] = 0.0;
+                UniformPtr y = x + kSetHeader;
+                x = y + kNd * count;
+                // Two nodes a step (lists are padded to an even length): one's latencies are filled
+                // by the other's instructions, and the screen is tested once, on the second (the
+                // larger exponent). The next two nodes' constants are read meanwhile (the slots
+                // after a full list are readable too).
+                struct Node {
+                    double s, is, w[NB];
+                };
+                auto read = [](UniformPtr z) {
+                    Node c;
+                    c.s = z[0];
+                    c.is = z[1];
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) c.w[b] = z[2 + b];
+                    return c;
+                };
+                Node n0 = read(y), n1 = read(y + kNd);
+                int t = 0;
+                bool done;
+                do {
+                    const Node c0 = n0, c1 = n1;
+                    y += 2 * kNd;
+                    n0 = read(y);
+                    n1 = read(y + kNd);
+                    __builtin_amdgcn_sched_barrier(0);     // issued here, not beside the table's
+                    const double P0 = __builtin_fma(c0.is, I3, __builtin_fma(c0.s, I1 + c0.s, I2));
+                    const double P1 = __builtin_fma(c1.is, I3, __builtin_fma(c1.s, I1 + c1.s, I2));
+                    const double Q0 = __builtin_fma(c0.s, __builtin_fma(c0.s, q1, rr), X0);
+                    const double Q1 = __builtin_fma(c1.s, __builtin_fma(c1.s, q1, rr), X0);
+                    const NodeArgH v0 = node_arg_h(P0, Q0), v1 = node_arg_h(P1, Q1);
+                    const double f0 = v0.y0 * exp_neg_tab_k<true>(v0.arg, tab);
+                    const double f1 = v1.y0 * exp_neg_tab_k<true>(v1.arg, tab);
+#pragma unroll
+                    for (int b = 0; b < NB; ++b)
+                        F[b] = __builtin_fma(c1.w[b], f1, __builtin_fma(c0.w[b], f0, F[b]));
+                    t += 2;
+                    done = (t >= count) | wave_all_beyond_h(v1.arg);
+                } while (!done);
+                lane_nodes += lanes * (uint64_t)t;
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    acc[NB * j + b][threadIdx.x] =
+                        __builtin_fma(F[b], cf, acc[NB * j + b][threadIdx.x]);
+            } while (!last);
+        }
+    }
+    if (work && (threadIdx.x & 63) == 0) atomicAdd(work, (unsigned long long)lane_nodes);
+    __syncthreads();
+    const int j = threadIdx.x >> 4, part = threadIdx.x & 15;
+    double sum = 0.0;
+    if (j < kFwdRecs)
+        for (int l = 0; l < 16; ++l) sum += acc[j][16 * l + part];
+    for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    if (part == 0 && j < NB * ngr) {
+        int64_t slot0;
+        const int nb = set_group(gr0 + j / NB, G, per_centre, &slot0);
+        if (j % NB < nb) partial[g * N + slot0 + j % NB] = sum;
+    }
+}
+
+// gamma[p] = sum over pair groups of partial[g * N + slot(p)], in group order, times kn[p] (null:
+// the blocks have multiplied it in).
 __global__ void k_slot_sum(int64_t N, int64_t G, int64_t groups, const double* __restrict__ partial,
-                           double* __restrict__ gamma) {
+                           const double* __restrict__ kn, double* __restrict__ gamma) {
     const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (p >= N) return;
     const int64_t q = aux_slot(p, N, G);
     double s = 0.0;
 #pragma unroll 8
     for (int64_t g = 0; g < groups; ++g) s += partial[g * N + q];
-    gamma[p] = s;
+    gamma[p] = kn ? s * kn[p] : s;
 }
 
 // ------------------------------------------------------------------ reverse
@@ -814,14 +940,17 @@ constexpr int kAtomChunk = 64;
 
 // The nuclear-force form (kAtomF) is held to four waves per SIMD (128 registers, a 20-byte spill
 // outside the node loop): 1.6% faster than the three its 134 registers allowed. The other forms
-// keep their allocation (for kLaneU four waves cost a 32-byte spill and 2.6%).
-template <bool kLaneU, bool kAtomF = false, bool kFold = false, int kN = kNodes>
-__global__ __launch_bounds__(256, kAtomF ? 4 : 1) void k_gamma_bwd(
+// keep their allocation (for kLaneU four waves cost a 32-byte spill and 2.6%); kSet with
+// its two nodes a step fits four waves (12 bytes spilled outside the node loop; equal to three).
+template <bool kLaneU, bool kAtomF = false, bool kFold = false, int kN = kNodes, bool kSet = false>
+__global__ __launch_bounds__(256, kAtomF || kSet ? 4 : 1) void k_gamma_bwd(
     int64_t n, const double* __restrict__ rec, int64_t N, const double* __restrict__ aux,
     int64_t per_slab, double* __restrict__ partial, unsigned long long* __restrict__ work,
     const double* __restrict__ ut, int64_t ldu, double* __restrict__ atom_part,
     const int32_t* __restrict__ uperm, const int32_t* __restrict__ uptr,
-    const int64_t* __restrict__ n_live, int ugroup = 0, int64_t slab0 = 0, int acc_first = -1) {
+    const int64_t* __restrict__ n_live, int ugroup = 0, int64_t slab0 = 0, int acc_first = -1,
+    int64_t set_stride = 0) {
+    static_assert(!kSet || (kFold && !kLaneU && !kAtomF), "");
     // whole workgroups past the real slots leave at once (workgroup-uniform, before any barrier)
     if (n_live && (int64_t)blockIdx.x * blockDim.x >= *n_live) return;
     __shared__ double tab[256];
@@ -901,6 +1030,81 @@ __global__ __launch_bounds__(256, kAtomF ? 4 : 1) void k_gamma_bwd(
     const int64_t p0 = slab * per_slab;
     const int64_t p1 = min(N, p0 + per_slab);
     uint32_t nodes = 0;
+    // the centre-dependent terms of a new centre
+    auto centre = [&](double Rx, double Ry, double Rz) {
+        flush();
+        const int l = threadIdx.x;
+        const double xx = geo[0][l], yy = geo[1][l], zz = geo[2][l], xy = geo[3][l],
+                     xz = geo[4][l], yz = geo[5][l];
+        d[0] = Rx - geo[6][l]; d[1] = Ry - geo[7][l]; d[2] = Rz - geo[8][l];
+        const double ax = __builtin_fma(xx, d[0], __builtin_fma(xy, d[1], xz * d[2]));
+        const double ay = __builtin_fma(xy, d[0], __builtin_fma(yy, d[1], yz * d[2]));
+        const double az = __builtin_fma(xz, d[0], __builtin_fma(yz, d[1], zz * d[2]));
+        q0 = __builtin_fma(d[0], d[0], __builtin_fma(d[1], d[1], d[2] * d[2]));
+        q1 = __builtin_fma(d[0], ax, __builtin_fma(d[1], ay, d[2] * az));
+        const double q2 = __builtin_fma(ax, ax, __builtin_fma(ay, ay, az * az));
+        X0 = I3 * q0;
+        rr = __builtin_fma(I1, q1, -q2);
+        if constexpr (kAtomF) {
+            ad[0] = ax; ad[1] = ay; ad[2] = az;
+            a2d[0] = __builtin_fma(xx, ax, __builtin_fma(xy, ay, xz * az));
+            a2d[1] = __builtin_fma(xy, ax, __builtin_fma(yy, ay, yz * az));
+            a2d[2] = __builtin_fma(xz, ax, __builtin_fma(yz, ay, zz * az));
+        }
+    };
+    // one node's terms added to the node sums; returns z - 1/2
+    auto add_node = [&](double st, double wh, double s2, double is) {
+        const double Pr = __builtin_fma(is, I3, __builtin_fma(st, I1 + st, I2));
+        const double Qn = __builtin_fma(st, __builtin_fma(st, q1, rr), X0);
+        const NodeValH v = node_val_h(Pr, Qn);
+        const double f = (wh * v.y0) * exp_neg_tab_k<kSet>(v.arg, tab);
+        F += f;
+        const double G = f * v.ip;                  // g s
+        const double Gh = G * v.zh;                 // s df/dPn
+        dP0 = __builtin_fma(Gh, is, dP0);
+        dP1 += Gh;
+        dP2 = __builtin_fma(Gh, st, dP2);
+        gs1 += G;
+        gs2 = __builtin_fma(G, st, gs2);
+        gs3 = __builtin_fma(G, s2, gs3);
+        return v.zh;
+    };
+    // kSet: the records are groups of shared node lists (nodeset.hip), each list's weights the sum
+    // of its functions' cotangents, so a centre costs one list whatever its number of scales
+    // (C20H42, four scales: 68.4 -> 50.5 ms; water octamer 9.09 -> 5.86; 52.3 and 6.07 with one node
+    // a step)
+    if constexpr (kSet) {
+        for (int64_t p = p0; p < p1; ++p) {
+            UniformPtr x = uniform_ptr(aux + set_stride * p);
+            bool last;
+            do {                                     // wave-uniform; once unless centres differ
+                const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
+                const int count = (int)(uint32_t)head;
+                last = (head >> 32) != 0;
+                centre(x[0], x[1], x[2]);
+                UniformPtr y = x + kSetHeader;
+                x = y + 4 * count;
+                // two nodes a step, as in k_gamma_fwd_sets
+                double s0 = y[0], w0 = y[1], ss0 = y[2], i0 = y[3];
+                double s1 = y[4], w1 = y[5], ss1 = y[6], i1 = y[7];
+                int t = 0;
+                bool done;
+                do {
+                    const double cs0 = s0, cw0 = w0, css0 = ss0, ci0 = i0;
+                    const double cs1 = s1, cw1 = w1, css1 = ss1, ci1 = i1;
+                    y += 8;
+                    s0 = y[0]; w0 = y[1]; ss0 = y[2]; i0 = y[3];
+                    s1 = y[4]; w1 = y[5]; ss1 = y[6]; i1 = y[7];
+                    __builtin_amdgcn_sched_barrier(0);     // issued here, not beside the table's
+                    add_node(cs0, cw0, css0, ci0);
+                    const double zh = add_node(cs1, cw1, css1, ci1);
+                    t += 2;
+                    done = (t >= count) | wave_all_beyond_h(zh);
+                } while (!done);
+                nodes += t;
+            } while (!last);
+        }
+    }
     // kLaneU: the lane's summed cotangents of the next kUb records, fetched kUb records at a time
     // (16-byte loads, half a cache line per row, when the rows and the slab start are 16-byte
     // aligned) and shifted down one record per step; each sum adds the rows in order, as one
@@ -917,12 +1121,12 @@ __global__ __launch_bounds__(256, kAtomF ? 4 : 1) void k_gamma_bwd(
     // record's start.
     double c_x = 0, c_y = 0, c_z = 0, c_u = 0, c_s = 0, c_wh = 0, c_s2 = 0, c_is = 0;
     uint64_t c_new = 1;                                  // the flag's bits, tested when used
-    if (p0 < p1) {
+    if (!kSet && p0 < p1) {
         const double* __restrict__ xf = aux + kAuxRec * p0;
         c_x = xf[0]; c_y = xf[1]; c_z = xf[2]; c_u = xf[3];
         c_s = xf[rec_s(0)]; c_wh = xf[rec_wh(0)]; c_s2 = xf[rec_s2(0)]; c_is = xf[rec_is(0)];
     }
-    for (int64_t p = p0; p < p1; ++p) {
+    for (int64_t p = p0; !kSet && p < p1; ++p) {
         const double* __restrict__ x = aux + kAuxRec * p;
         const double Rx = c_x, Ry = c_y, Rz = c_z;
         double u = c_u;
@@ -962,27 +1166,7 @@ __global__ __launch_bounds__(256, kAtomF ? 4 : 1) void k_gamma_bwd(
 #pragma unroll
             for (int j = 0; j + 1 < kUb; ++j) ub[j] = ub[j + 1];
         }
-        if (fresh) {                                     // wave-uniform
-            flush();
-            const int l = threadIdx.x;
-            const double xx = geo[0][l], yy = geo[1][l], zz = geo[2][l], xy = geo[3][l],
-                         xz = geo[4][l], yz = geo[5][l];
-            d[0] = Rx - geo[6][l]; d[1] = Ry - geo[7][l]; d[2] = Rz - geo[8][l];
-            const double ax = __builtin_fma(xx, d[0], __builtin_fma(xy, d[1], xz * d[2]));
-            const double ay = __builtin_fma(xy, d[0], __builtin_fma(yy, d[1], yz * d[2]));
-            const double az = __builtin_fma(xz, d[0], __builtin_fma(yz, d[1], zz * d[2]));
-            q0 = __builtin_fma(d[0], d[0], __builtin_fma(d[1], d[1], d[2] * d[2]));
-            q1 = __builtin_fma(d[0], ax, __builtin_fma(d[1], ay, d[2] * az));
-            const double q2 = __builtin_fma(ax, ax, __builtin_fma(ay, ay, az * az));
-            X0 = I3 * q0;
-            rr = __builtin_fma(I1, q1, -q2);
-            if constexpr (kAtomF) {
-                ad[0] = ax; ad[1] = ay; ad[2] = az;
-                a2d[0] = __builtin_fma(xx, ax, __builtin_fma(xy, ay, xz * az));
-                a2d[1] = __builtin_fma(xy, ax, __builtin_fma(yy, ay, yz * az));
-                a2d[2] = __builtin_fma(xz, ax, __builtin_fma(yz, ay, zz * az));
-            }
-        }
+        if (fresh) centre(Rx, Ry, Rz);                   // wave-uniform
         if constexpr (!kFold) {
             F = 0; dP0 = 0; dP1 = 0; dP2 = 0; gs1 = 0; gs2 = 0; gs3 = 0;
         }
@@ -997,23 +1181,11 @@ __global__ __launch_bounds__(256, kAtomF ? 4 : 1) void k_gamma_bwd(
                 n_s2 = x[rec_s2(t + 1)];
                 n_is = x[rec_is(t + 1)];
             }
-            const double Pr = __builtin_fma(is, I3, __builtin_fma(st, I1 + st, I2));
-            const double Qn = __builtin_fma(st, __builtin_fma(st, q1, rr), X0);
-            const NodeValH v = node_val_h(Pr, Qn);
-            const double f = (wh * v.y0) * exp_neg_tab_k(v.arg, tab);
-            F += f;
-            const double G = f * v.ip;                  // g s
-            const double Gh = G * v.zh;                 // s df/dPn
-            dP0 = __builtin_fma(Gh, is, dP0);
-            dP1 += Gh;
-            dP2 = __builtin_fma(Gh, st, dP2);
-            gs1 += G;
-            gs2 = __builtin_fma(G, st, gs2);
-            gs3 = __builtin_fma(G, s2, gs3);
+            const double zh = add_node(st, wh, s2, is);
             // keep the next node's loads ahead of the early exit (not sunk past it)
             if constexpr (t + 1 < kN)
                 asm volatile("" ::"s"(n_s), "s"(n_wh), "s"(n_s2), "s"(n_is));
-            return screen_after<kN>(t) && wave_all_beyond_h(v.zh);
+            return screen_after<kN>(t) && wave_all_beyond_h(zh);
         };
         nodes += node_loop<0, kN>(node);
         if constexpr (kFold) continue;
@@ -1961,6 +2133,19 @@ int64_t bwd_slabs_per_launch(int64_t N, int64_t n) {
     return r < sp.slabs ? r : sp.slabs;
 }
 
+// Whether a DF-J pass takes the shared node lists (nodeset.hip). Choosing them costs ~0.15 ms, or
+// 0.25 us a centre, which a centre's nodes saved earn back from ~32,000 pairs on (four scales, step
+// in ms, plain / shared: 17 k pairs 0.93 / 0.98, 37 k 2.02 / 1.87, 167 k 16.1 / 11.8, 590 k 117 /
+// 93; 7.9 k 0.48 / 0.64). One scale leaves 18 of 20 nodes, less than the loop over a list costs
+// (2203 functions, 560 k pairs: 78.9 / 79.2); two leave 32 of 40, of use to the reverse only,
+// whose node costs no more for a second function (gamma 9.69 / 9.77 ms; step of 17 k pairs 1.845 /
+// 1.785).
+constexpr int64_t kSetMinPairs = 32768;
+constexpr int64_t kSetSlack = 16;       // the passes read two nodes past a list
+inline bool use_node_sets(int64_t n, int64_t G, bool reverse) {
+    return n >= kSetMinPairs && G >= (reverse ? 2 : 3);
+}
+
 struct GammaWs {
     double *A6, *Nrm, *beta, *kn, *q, *rec, *partial;
     double *aux, *acc, *contrib, *rec_sorted;
@@ -2836,27 +3021,49 @@ int gamma_run(int64_t M, const double* quat, const double* log_scale, const doub
     GSDFT_TRY(gamma_prologue(M, quat, log_scale, centers, k, C, occ, N, log_alpha, n, pi, pj,
                              weight, w, s));
     const int64_t G = (N % M == 0) ? N / M : 1;          // scales per centre of a product aux
-    k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
-                                                      nullptr, kAuxForward, coulomb_table(),
-                                                      w.aux);
-    GSDFT_HIP(hipGetLastError());
+    const int64_t groups = fwd_groups(N, n);
+    const NodeSets ns = node_sets(N, G, false);
+    const bool sets = use_node_sets(n, G, false) &&
+                      ns.stride * ns.groups + kSetSlack + groups * N <= kRec * n;
+    if (sets) {
+        GSDFT_TRY(launch_pair_box(n, nullptr, w.rec, kRec, w.q, s));
+    } else {
+        k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
+                                                          nullptr, kAuxForward, coulomb_table(),
+                                                          w.aux);
+        GSDFT_HIP(hipGetLastError());
+    }
     GSDFT_TRY(launch_pair_order(n, w.rec, kRec, w.pair_order, s));
     k_rec_gather<<<blocks_for(n * kRec, 256), 256, 0, s>>>(n, w.pair_order.perm, w.rec,
                                                             w.rec_sorted);
     GSDFT_HIP(hipGetLastError());
-    const int64_t groups = fwd_groups(N, n);
-    const int64_t nrb = (N + kFwdRecs - 1) / kFwdRecs;
+    // the node lists take the dead pair records' slice as the block sums do, before them
+    double* const set_area = w.rec;
+    double* const partial = sets ? w.rec + ns.stride * ns.groups + kSetSlack : w.partial;
+    if (sets)
+        GSDFT_TRY(launch_node_sets(N, G, false, w.beta, w.kn, aux_centers, nullptr, nullptr, w.q,
+                                   set_area, s));
+    const int64_t per_block = sets ? kFwdRecs / std::min<int64_t>(G, kMaxSetScales) : kFwdRecs;
+    const int64_t nrb = ((sets ? ns.groups : N) + per_block - 1) / per_block;
     if (nrb * 256 > (int64_t)UINT32_MAX || groups > kMaxGridY)
         return fail(GSDFT_ERR_ARG, "gsdft_gamma: N_aux = %lld or n = %lld too large for one launch",
                     (long long)N, (long long)n);
     const dim3 grid((unsigned)nrb, (unsigned)groups);
+    const int64_t pairs = fwd_pairs(N, n);
+    unsigned long long* work = profile ? profile_work_counter(kProfGammaFwd) : nullptr;
     if (profile) profile_begin(kProfGammaFwd, s);
-    k_gamma_fwd_pairs<<<grid, 256, 0, s>>>(n, fwd_pairs(N, n), w.rec_sorted, N, w.aux, w.partial,
-                                           profile ? profile_work_counter(kProfGammaFwd)
-                                                   : nullptr);
+    if (!sets)
+        k_gamma_fwd_pairs<<<grid, 256, 0, s>>>(n, pairs, w.rec_sorted, N, w.aux, partial, work);
+    else if (G == 3)
+        k_gamma_fwd_sets<3><<<grid, 256, 0, s>>>(n, pairs, w.rec_sorted, N, G, ns.per_centre,
+                                                 ns.groups, ns.stride, set_area, partial, work);
+    else
+        k_gamma_fwd_sets<4><<<grid, 256, 0, s>>>(n, pairs, w.rec_sorted, N, G, ns.per_centre,
+                                                 ns.groups, ns.stride, set_area, partial, work);
     if (profile) profile_end(kProfGammaFwd, s);
     GSDFT_HIP(hipGetLastError());
-    k_slot_sum<<<blocks_for(N, 256), 256, 0, s>>>(N, G, groups, w.partial, gamma);
+    k_slot_sum<<<blocks_for(N, 256), 256, 0, s>>>(N, G, groups, partial, sets ? w.kn : nullptr,
+                                                  gamma);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
 }
@@ -2946,23 +3153,42 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
                              weight, w, s));
     if (n > 0) {
         const int64_t G = (N % M == 0) ? N / M : 1;      // scales per centre of a product aux
-        k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers,
-                                                          dgamma, dgamma_scale, kAuxFoldU,
-                                                          coulomb_table(),
-                                                          w.aux);
+        const NodeSets ns = node_sets(N, G, true);
+        const bool sets = use_node_sets(n, G, true) &&
+                          ns.stride * ns.groups + kSetSlack <= kAuxRec * N + kAuxRec;
+        if (sets) {
+            GSDFT_TRY(launch_pair_box(n, nullptr, w.rec, kRec, w.q, s));
+            GSDFT_TRY(launch_node_sets(N, G, true, w.beta, w.kn, aux_centers, dgamma, dgamma_scale,
+                                       w.q, w.aux, s));
+        } else {
+            k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers,
+                                                              dgamma, dgamma_scale, kAuxFoldU,
+                                                              coulomb_table(), w.aux);
+            GSDFT_HIP(hipGetLastError());
+        }
         GSDFT_TRY(launch_pair_order(n, w.rec, kRec, w.pair_order, s));
         k_rec_gather<<<blocks_for(n * kRec, 256), 256, 0, s>>>(n, w.pair_order.perm, w.rec,
                                                                 w.rec_sorted);
-        const Split sp = bwd_split_records(N, n);
+        // the slabs of groups that hold bwd_split_records' records: never more slabs than those
+        Split sp = bwd_split_records(N, n);
+        if (sets) {
+            sp.per_slab = (sp.per_slab + ns.nb - 1) / ns.nb;
+            sp.slabs = (ns.groups + sp.per_slab - 1) / sp.per_slab;
+        }
         const int64_t per_launch = bwd_slabs_per_launch(N, n);
         profile_begin(kProfGammaBwd, s);
         for (int64_t sl = 0; sl < sp.slabs; sl += per_launch) {
             const int64_t r = std::min(per_launch, sp.slabs - sl);
             dim3 grid((unsigned)((n + 255) / 256), (unsigned)r);
-            k_gamma_bwd<false, false, true><<<grid, 256, 0, s>>>(
-                n, w.rec_sorted, N, w.aux, sp.per_slab, w.acc,
-                profile_work_counter(kProfGammaBwd), nullptr, 0, nullptr, nullptr, nullptr,
-                nullptr, 0, sl, sl == 0 ? 1 : 0);
+            unsigned long long* work = profile_work_counter(kProfGammaBwd);
+            if (sets)
+                k_gamma_bwd<false, false, true, kNodes, true><<<grid, 256, 0, s>>>(
+                    n, w.rec_sorted, ns.groups, w.aux, sp.per_slab, w.acc, work, nullptr, 0,
+                    nullptr, nullptr, nullptr, nullptr, 0, sl, sl == 0 ? 1 : 0, ns.stride);
+            else
+                k_gamma_bwd<false, false, true><<<grid, 256, 0, s>>>(
+                    n, w.rec_sorted, N, w.aux, sp.per_slab, w.acc, work, nullptr, 0, nullptr,
+                    nullptr, nullptr, nullptr, 0, sl, sl == 0 ? 1 : 0);
             GSDFT_HIP(hipGetLastError());
             if (r > 1) {
                 k_slab_fold<<<blocks_for(n * kAcc, 256), 256, 0, s>>>(n, r, w.acc);

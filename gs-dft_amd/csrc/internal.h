@@ -156,6 +156,17 @@ int launch_pair_groups(int64_t M, int64_t n, const int32_t* pi, const int32_t* p
                        size_t scan_bytes, int32_t* ent_group, int32_t* ent_pos,
                        int32_t* grp_first, int32_t* grp_rep, int64_t* n_groups, hipStream_t s);
 
+// nodeset.hip: the reach and widths of n pair records (the first 12 doubles as for
+// launch_pair_order; n_live as there) into scratch[0..7], scratch holding node_set_box_doubles();
+// and one node list per group of aux functions (layout: common.h), its weights plain (`fold`
+// false; dgamma, dscale and kn unread) or carrying dgamma_P dscale kn_P summed over the group.
+size_t node_set_box_doubles();
+int launch_pair_box(int64_t n, const int64_t* n_live, const double* rec, int rec_stride,
+                    double* scratch, hipStream_t s);
+int launch_node_sets(int64_t N, int64_t G, bool fold, const double* beta, const double* kn,
+                     const double* R, const double* dgamma, const double* dscale,
+                     const double* box, double* out, hipStream_t s);
+
 // dfj.hip: the three-centre passes of the screened exchange. Charts, aux quantities and pair
 // records (q_a = w_a) in list order. The entries of the list are grouped by their unordered splat
 // pair {i, j} (live entries only; each dead entry is a group of its own): the entries of a group

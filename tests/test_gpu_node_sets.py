@@ -1,0 +1,68 @@
+"""Shared node lists of the DF-J passes (lists of 32,768 pairs and more, aux with two and more scales
+per centre): gamma and its reverse pass against the oracle's twenty nodes per function.
+
+The cases are the forms the lists can take: 2 to 6 scales per centre (groups of four, the last one
+ragged), exponents over six decades, aux far from every pair, and aux whose functions do not share
+a centre although their count is a multiple of the splats' (every function then keeps its own nodes).
+One list is a single pair short, so it takes the plain records.
+
+Tolerance: each (P|a) agrees with the oracle's to 1e-12 of itself (the parity bar for gamma, which
+the lists' own error of a few 1e-15 does not move), so gamma differs by at most 1e-12 of the sum of
+its terms' magnitudes, and each gradient row by 1e-9 of the largest (the parity bar).
+"""
+import numpy as np
+import pytest
+import torch
+
+from conftest import rel_max
+
+pytestmark = pytest.mark.gpu
+
+N_MIN = 32768
+
+
+def _case(wl, name):
+    s = wl.make_small(30, 6, n_atoms=4, seed=11, spread=4.0)
+    rng = np.random.default_rng(5)
+    G = {"two": 2, "three": 3, "four": 4, "five": 5, "six": 6}.get(name, 4)
+    la = np.log(rng.uniform(0.1, 12.0, s.M))[None] + np.log(np.geomspace(0.5, 4.0, G))[:, None]
+    ac = np.repeat((s.centers + rng.normal(0.0, 0.2, (s.M, 3)))[None], G, 0)
+    if name == "decades":
+        la = rng.uniform(np.log(1e-3), np.log(1e3), (G, s.M))
+    if name == "far":
+        ac = ac + np.array([45.0, 30.0, -20.0])
+    if name == "moved":            # one function of each second group stands elsewhere
+        ac[2, ::2] += 0.25
+    n = N_MIN - 1 if name == "short" else N_MIN + 77
+    a = rng.integers(0, s.M * s.M, n)
+    i, j = (a // s.M).astype(np.int32), (a % s.M).astype(np.int32)
+    w = rng.uniform(0.5, 2.0, n)
+    w[::7] = 0.0
+    return s, la.ravel(), ac.reshape(-1, 3), i, j, w
+
+
+@pytest.mark.parametrize("name", ["two", "three", "four", "five", "six", "decades", "far", "moved",
+                                  "short"])
+def test_gamma_and_reverse_match_oracle(g, wl, orc, cuda, name):
+    s, la, ac, i, j, w = _case(wl, name)
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    basis = g.Splat(quat=t(s.quat), log_scale=t(s.log_scale), centers=t(s.centers))
+    C = t(s.C)
+    gam = g.df_coulomb_gamma_screened(basis, C, s.occ, g.IsotropicSplat(log_alpha=la, centers=ac),
+                                      torch.tensor(i), torch.tensor(j), valid=torch.tensor(w))
+    got = gam.detach().cpu().numpy()
+    ref = orc.gamma(s.quat, s.log_scale, s.centers, s.C, s.occ, la, ac, i, j, w)
+    # the terms' magnitudes, bounded: every orbital product by the largest one's
+    big = np.full((s.M, 1), np.sqrt(np.abs((s.C * s.occ) @ s.C.T).max()))
+    unit = orc.gamma(s.quat, s.log_scale, s.centers, big, np.ones(1), la, ac, i, j, w)
+    print(f"[sets] {name}: N={len(la)} n={len(i)} gamma error / bound "
+          f"{np.max(np.abs(got - ref) / (1e-12 * unit)):.2e}", flush=True)
+    assert np.all(np.abs(got - ref) <= 1e-12 * unit)
+    v = np.random.default_rng(3).normal(size=len(la)) / unit
+    grads = torch.autograd.grad(gam, [basis.quat, basis.log_scale, basis.centers, C],
+                                torch.tensor(v, device="cuda"))
+    back = orc.gamma_vjp(s.quat, s.log_scale, s.centers, s.C, s.occ, la, ac, i, j, w, v)
+    for what, a, b in zip(("quat", "log_scale", "centers", "C"), grads, back[-4:]):
+        err = rel_max(a.cpu().numpy(), b)
+        print(f"[sets] {name}: d{what} {err:.2e}", flush=True)
+        assert err < 1e-9
