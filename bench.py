@@ -686,8 +686,13 @@ def run_exchange(args) -> int:
     _lib.profile_enable(False)
     # the three-centre passes run once per unordered splat pair (the list is symmetric)
     groups = int(((pi <= pj) & (w != 0)).sum().item())
-    blk_exec = float(groups) * N * FWD_PER_INTEGRAL + blk_nodes * FWD_PER_NODE
-    rev_exec = float(groups) * N * BWD_PER_INTEGRAL + bwd_nodes * BWD_PER_NODE
+    # scales in fours share one node list per centre from 32768 list entries on: its centre terms
+    # once, each node's weight formed from (or added to) four functions
+    share = 4 if len(s.scales) % 4 == 0 and n >= 32768 else 1
+    blk_exec = (float(groups) * N * FWD_PER_INTEGRAL / share
+                + blk_nodes * (FWD_PER_NODE + 2 * (share - 1)))
+    rev_exec = (float(groups) * N * BWD_PER_INTEGRAL / share
+                + bwd_nodes * (BWD_PER_NODE + 2 * (share - 1)))
     per_step = {kid: prof[kid][0] / args.steps for kid in ids}
     blk_ms, rev_ms = per_step[_lib.PROF_EXCH_BLOCK], per_step[_lib.PROF_EXCH_BWD]
     trsm_ms, gemm_ms = per_step[_lib.PROF_EXCH_TRSM], per_step[_lib.PROF_EXCH_GEMM]

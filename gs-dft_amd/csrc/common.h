@@ -514,14 +514,19 @@ constexpr double kExpMinusHalf = 0x1.368b2fc6f960ap-1;     // e^(-1/2), correctl
 // Layout of the node lists that k_node_sets (nodeset.hip) writes and the three-centre passes read.
 // The aux functions are taken in groups of at most kMaxSetScales consecutive slots of one centre.
 // A group holds sub-records (one, unless its functions do not share a centre): a header R (3),
-// bits (node count, even | last << 32), then per node, in ascending s, either s, 1/s and the weight of
-// each function (forward) or s, weight, s^2, 1/s with the functions' cotangents folded into the
-// one weight (reverse). Weights carry s^(-1/2) e^(-1/2) / 24 (exp_quartic).
+// bits (node count, even | last << 32), then per node, in ascending s: s, 1/s and the weight of
+// each function (kSetForward); s, weight, s^2, 1/s with the functions' cotangents folded into the
+// one weight (kSetFold); or s, 1/s, the four functions' weights times KN_P, s^2 and a pad
+// (kSetExchange). Weights carry s^(-1/2) e^(-1/2) / 24 (exp_quartic).
 constexpr int kMaxSetScales = 4;
 constexpr int kSetHeader = 4;
 
-// Forward node size for NB functions: 2 + NB, an even count of doubles.
-__host__ __device__ constexpr int set_node_doubles(int NB) { return NB <= 2 ? 4 : 6; }
+enum SetForm { kSetForward = 0, kSetFold = 1, kSetExchange = 2 };
+
+// Node size of a list for NB functions, an even count of doubles.
+__host__ __device__ constexpr int set_node_doubles(int NB, SetForm form = kSetForward) {
+    return form == kSetExchange ? 8 : form == kSetFold ? 4 : NB <= 2 ? 4 : 6;
+}
 
 struct NodeSets {
     int nb;                 // functions per group: 2 or 4 (3 are padded)
@@ -531,12 +536,12 @@ struct NodeSets {
 };
 
 // N aux functions, G >= 2 scales per centre.
-__host__ __device__ inline NodeSets node_sets(int64_t N, int64_t G, bool fold) {
+__host__ __device__ inline NodeSets node_sets(int64_t N, int64_t G, SetForm form) {
     NodeSets ns;
     ns.nb = G == 2 ? 2 : kMaxSetScales;
     ns.per_centre = (G + kMaxSetScales - 1) / kMaxSetScales;
     ns.groups = N / G * ns.per_centre;
-    ns.stride = ns.nb * (kSetHeader + (int64_t)kNodes * (fold ? 4 : set_node_doubles(ns.nb)));
+    ns.stride = ns.nb * (kSetHeader + (int64_t)kNodes * set_node_doubles(ns.nb, form));
     return ns;
 }
 

@@ -943,14 +943,14 @@ constexpr int kAtomChunk = 64;
 // keep their allocation (for kLaneU four waves cost a 32-byte spill and 2.6%); kSet with
 // its two nodes a step fits four waves (12 bytes spilled outside the node loop; equal to three).
 template <bool kLaneU, bool kAtomF = false, bool kFold = false, int kN = kNodes, bool kSet = false>
-__global__ __launch_bounds__(256, kAtomF || kSet ? 4 : 1) void k_gamma_bwd(
+__global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kAtomF || kSet ? 4 : 1) void k_gamma_bwd(
     int64_t n, const double* __restrict__ rec, int64_t N, const double* __restrict__ aux,
     int64_t per_slab, double* __restrict__ partial, unsigned long long* __restrict__ work,
     const double* __restrict__ ut, int64_t ldu, double* __restrict__ atom_part,
     const int32_t* __restrict__ uperm, const int32_t* __restrict__ uptr,
     const int64_t* __restrict__ n_live, int ugroup = 0, int64_t slab0 = 0, int acc_first = -1,
     int64_t set_stride = 0) {
-    static_assert(!kSet || (kFold && !kLaneU && !kAtomF), "");
+    static_assert(!kSet || (kFold && !kAtomF), "");
     // whole workgroups past the real slots leave at once (workgroup-uniform, before any barrier)
     if (n_live && (int64_t)blockIdx.x * blockDim.x >= *n_live) return;
     __shared__ double tab[256];
@@ -1069,42 +1069,6 @@ __global__ __launch_bounds__(256, kAtomF || kSet ? 4 : 1) void k_gamma_bwd(
         gs3 = __builtin_fma(G, s2, gs3);
         return v.zh;
     };
-    // kSet: the records are groups of shared node lists (nodeset.hip), each list's weights the sum
-    // of its functions' cotangents, so a centre costs one list whatever its number of scales
-    // (C20H42, four scales: 68.4 -> 50.5 ms; water octamer 9.09 -> 5.86; 52.3 and 6.07 with one node
-    // a step)
-    if constexpr (kSet) {
-        for (int64_t p = p0; p < p1; ++p) {
-            UniformPtr x = uniform_ptr(aux + set_stride * p);
-            bool last;
-            do {                                     // wave-uniform; once unless centres differ
-                const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
-                const int count = (int)(uint32_t)head;
-                last = (head >> 32) != 0;
-                centre(x[0], x[1], x[2]);
-                UniformPtr y = x + kSetHeader;
-                x = y + 4 * count;
-                // two nodes a step, as in k_gamma_fwd_sets
-                double s0 = y[0], w0 = y[1], ss0 = y[2], i0 = y[3];
-                double s1 = y[4], w1 = y[5], ss1 = y[6], i1 = y[7];
-                int t = 0;
-                bool done;
-                do {
-                    const double cs0 = s0, cw0 = w0, css0 = ss0, ci0 = i0;
-                    const double cs1 = s1, cw1 = w1, css1 = ss1, ci1 = i1;
-                    y += 8;
-                    s0 = y[0]; w0 = y[1]; ss0 = y[2]; i0 = y[3];
-                    s1 = y[4]; w1 = y[5]; ss1 = y[6]; i1 = y[7];
-                    __builtin_amdgcn_sched_barrier(0);     // issued here, not beside the table's
-                    add_node(cs0, cw0, css0, ci0);
-                    const double zh = add_node(cs1, cw1, css1, ci1);
-                    t += 2;
-                    done = (t >= count) | wave_all_beyond_h(zh);
-                } while (!done);
-                nodes += t;
-            } while (!last);
-        }
-    }
     // kLaneU: the lane's summed cotangents of the next kUb records, fetched kUb records at a time
     // (16-byte loads, half a cache line per row, when the rows and the slab start are 16-byte
     // aligned) and shifted down one record per step; each sum adds the rows in order, as one
@@ -1114,8 +1078,92 @@ __global__ __launch_bounds__(256, kAtomF || kSet ? 4 : 1) void k_gamma_bwd(
     double ub[kUb];
 #pragma unroll
     for (int j = 0; j < kUb; ++j) ub[j] = 0.0;
-    const bool uvec = kLaneU && (ldu % 2 == 0) && (p0 % 2 == 0) &&
+    const bool uvec = kLaneU && (ldu % 2 == 0) && (kSet || p0 % 2 == 0) &&
                       (reinterpret_cast<uintptr_t>(ut) % 16 == 0);
+    // fills ub with the cotangents of records p .. p + kUb - 1 (0 from `end` on)
+    auto fetch = [&](int64_t p, int64_t end) {
+#pragma unroll
+        for (int j = 0; j < kUb; ++j) ub[j] = 0.0;
+        if (uvec && p + kUb <= end) {
+            for (int e = 0; e < utn; ++e) {
+                const double2* row = reinterpret_cast<const double2*>(ut + (ut0 + e) * ldu + p);
+#pragma unroll
+                for (int j = 0; j < kUb / 2; ++j) {
+                    const double2 v = row[j];
+                    ub[2 * j] += v.x;
+                    ub[2 * j + 1] += v.y;
+                }
+            }
+        } else {
+            for (int e = 0; e < utn; ++e) {
+                const double* row = ut + (ut0 + e) * ldu;
+#pragma unroll
+                for (int j = 0; j < kUb; ++j)
+                    if (p + j < end) ub[j] += row[p + j];
+            }
+        }
+    };
+    // kSet: the records are groups of shared node lists (nodeset.hip). With one cotangent per aux
+    // function each list's weights are already the sum of its functions' (C20H42, four scales:
+    // 68.4 -> 50.5 ms; water octamer 9.09 -> 5.86; 52.3 and 6.07 with one node a step), with kLaneU
+    // the lane forms them node by node from its four cotangents.
+    if constexpr (kSet) {
+        for (int64_t p = p0; p < p1; ++p) {
+            UniformPtr x = uniform_ptr(aux + set_stride * p);
+            double u0 = 0, u1 = 0, u2 = 0, u3 = 0;
+            if constexpr (kLaneU) {
+                if (((p - p0) % (kUb / 4)) == 0) fetch(4 * p, 4 * p1);
+                u0 = ub[0] * uscale; u1 = ub[1] * uscale; u2 = ub[2] * uscale; u3 = ub[3] * uscale;
+#pragma unroll
+                for (int j = 0; j + 4 < kUb; ++j) ub[j] = ub[j + 4];
+            }
+            bool last;
+            do {                                     // wave-uniform; once unless centres differ
+                const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
+                const int count = (int)(uint32_t)head;
+                last = (head >> 32) != 0;
+                centre(x[0], x[1], x[2]);
+                constexpr int kNd = kLaneU ? 8 : 4;
+                UniformPtr y = x + kSetHeader;
+                x = y + kNd * count;
+                // two nodes a step, as in k_gamma_fwd_sets
+                struct Node {
+                    double c[kNd];
+                };
+                auto read = [](UniformPtr z) {
+                    Node v;
+#pragma unroll
+                    for (int j = 0; j < kNd; ++j) v.c[j] = z[j];
+                    return v;
+                };
+                auto add = [&](const Node& v) {
+                    if constexpr (kLaneU) {
+                        const double w = __builtin_fma(
+                            v.c[5], u3,
+                            __builtin_fma(v.c[4], u2, __builtin_fma(v.c[3], u1, v.c[2] * u0)));
+                        return add_node(v.c[0], w, v.c[6], v.c[1]);
+                    } else {
+                        return add_node(v.c[0], v.c[1], v.c[2], v.c[3]);
+                    }
+                };
+                Node n0 = read(y), n1 = read(y + kNd);
+                int t = 0;
+                bool done;
+                do {
+                    const Node c0 = n0, c1 = n1;
+                    y += 2 * kNd;
+                    n0 = read(y);
+                    n1 = read(y + kNd);
+                    __builtin_amdgcn_sched_barrier(0);     // issued here, not beside the table's
+                    add(c0);
+                    const double zh = add(c1);
+                    t += 2;
+                    done = (t >= count) | wave_all_beyond_h(zh);
+                } while (!done);
+                nodes += t;
+            } while (!last);
+        }
+    }
     // Each record's centre, u, new-centre flag and node-0 constants are read one record ahead
     // (the first record's here), so their scalar loads overlap a node loop instead of stalling the
     // record's start.
@@ -1139,29 +1187,7 @@ __global__ __launch_bounds__(256, kAtomF || kSet ? 4 : 1) void k_gamma_bwd(
             c_new = __builtin_bit_cast(uint64_t, xn[5]);
         }
         if constexpr (kLaneU) {
-            if (((p - p0) % kUb) == 0) {                 // wave-uniform
-#pragma unroll
-                for (int j = 0; j < kUb; ++j) ub[j] = 0.0;
-                if (uvec && p + kUb <= p1) {
-                    for (int e = 0; e < utn; ++e) {
-                        const double2* row = reinterpret_cast<const double2*>(
-                            ut + (ut0 + e) * ldu + p);
-#pragma unroll
-                        for (int j = 0; j < kUb / 2; ++j) {
-                            const double2 v = row[j];
-                            ub[2 * j] += v.x;
-                            ub[2 * j + 1] += v.y;
-                        }
-                    }
-                } else {
-                    for (int e = 0; e < utn; ++e) {
-                        const double* row = ut + (ut0 + e) * ldu;
-#pragma unroll
-                        for (int j = 0; j < kUb; ++j)
-                            if (p + j < p1) ub[j] += row[p + j];
-                    }
-                }
-            }
+            if (((p - p0) % kUb) == 0) fetch(p, p1);     // wave-uniform
             u *= ub[0] * uscale;
 #pragma unroll
             for (int j = 0; j + 1 < kUb; ++j) ub[j] = ub[j + 1];
@@ -2055,6 +2081,111 @@ __global__ __launch_bounds__(256) void k_exch_block_pairs(int64_t n,
     }
 }
 
+// The same on shared node lists (nodeset.hip, kSetExchange) of four functions each: the sixteen
+// aux slots of a block are four groups, and each node is added to the four functions' sums with
+// the list's weights (KN_P folded in). C20H42: 51.8 -> 44.9 ms a step, the reverse on the same
+// lists 83.8 -> 70.4 ms (three waves per SIMD: 168 registers).
+template <bool kPair>
+__global__ __launch_bounds__(256) void k_exch_block_sets(int64_t n, const double* __restrict__ rec,
+                                                         const int32_t* __restrict__ perm,
+                                                         int64_t groups, int64_t stride,
+                                                         const double* __restrict__ sets,
+                                                         int64_t ldb, double* __restrict__ Bt,
+                                                         unsigned long long* __restrict__ work,
+                                                         const int64_t* __restrict__ n_live) {
+    // whole workgroups past the real slots leave at once (workgroup-uniform, before any barrier)
+    if (n_live && (int64_t)blockIdx.x * blockDim.x >= *n_live) return;
+    constexpr int kGroups = kBlockRecs / 4, kNd = set_node_doubles(4, kSetExchange);
+    __shared__ double tab[256];
+    __shared__ double val[kBlockRecs][256];
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) tab[i] = exp2_frac_lead(i);
+    __syncthreads();
+    const int64_t slot = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const bool live = slot < (n_live ? *n_live : n);   // n_live: a device count of real slots
+    const double* __restrict__ r = rec + kRec * (live ? slot : 0);
+    const double I1 = r[0], I2 = r[1], I3 = r[2];
+    const double xx = r[3], yy = r[4], zz = r[5], xy = r[6], xz = r[7], yz = r[8];
+    const double Px = live ? r[9] : kFarAway, Py = live ? r[10] : kFarAway,
+                 Pz = live ? r[11] : kFarAway;
+    const double coef = r[12];
+    const int64_t g0 = (int64_t)blockIdx.y * kGroups;
+    const int ngr = (int)min((int64_t)kGroups, groups - g0);
+    uint32_t nodes = 0;
+    for (int j = 0; j < ngr; ++j) {
+        UniformPtr x = uniform_ptr(sets + stride * (g0 + j));
+        double V[4] = {0.0, 0.0, 0.0, 0.0};
+        bool last;
+        do {                                     // wave-uniform; once unless centres differ
+            const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
+            const int count = (int)(uint32_t)head;
+            last = (head >> 32) != 0;
+            const double dx = x[0] - Px, dy = x[1] - Py, dz = x[2] - Pz;
+            const double ax = xx * dx + xy * dy + xz * dz;
+            const double ay = xy * dx + yy * dy + yz * dz;
+            const double az = xz * dx + yz * dy + zz * dz;
+            const double q0d = dx * dx + dy * dy + dz * dz;
+            const double q1 = dx * ax + dy * ay + dz * az;
+            const double q2 = ax * ax + ay * ay + az * az;
+            const double X0 = I3 * q0d;
+            const double rr = I1 * q1 - q2;
+            const double cf = (q0d == q0d) ? coef : q0d;          // a NaN centre propagates
+            UniformPtr y = x + kSetHeader;
+            x = y + kNd * count;
+            double F[4] = {0.0, 0.0, 0.0, 0.0};
+            // two nodes a step, as in k_gamma_fwd_sets
+            struct Node {
+                double s, is, w[4];
+            };
+            auto read = [](UniformPtr z) {
+                Node c;
+                c.s = z[0];
+                c.is = z[1];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) c.w[b] = z[2 + b];
+                return c;
+            };
+            Node n0 = read(y), n1 = read(y + kNd);
+            int t = 0;
+            bool done;
+            do {
+                const Node c0 = n0, c1 = n1;
+                y += 2 * kNd;
+                n0 = read(y);
+                n1 = read(y + kNd);
+                __builtin_amdgcn_sched_barrier(0);         // issued here, not beside the table's
+                const double P0 = __builtin_fma(c0.is, I3, __builtin_fma(c0.s, I1 + c0.s, I2));
+                const double P1 = __builtin_fma(c1.is, I3, __builtin_fma(c1.s, I1 + c1.s, I2));
+                const double Q0 = __builtin_fma(c0.s, __builtin_fma(c0.s, q1, rr), X0);
+                const double Q1 = __builtin_fma(c1.s, __builtin_fma(c1.s, q1, rr), X0);
+                const NodeArgH v0 = node_arg_h(P0, Q0), v1 = node_arg_h(P1, Q1);
+                const double f0 = v0.y0 * exp_neg_tab_k<true>(v0.arg, tab);
+                const double f1 = v1.y0 * exp_neg_tab_k<true>(v1.arg, tab);
+#pragma unroll
+                for (int b = 0; b < 4; ++b)
+                    F[b] = __builtin_fma(c1.w[b], f1, __builtin_fma(c0.w[b], f0, F[b]));
+                t += 2;
+                done = (t >= count) | wave_all_beyond_h(v1.arg);
+            } while (!done);
+            nodes += t;
+#pragma unroll
+            for (int b = 0; b < 4; ++b) V[b] = __builtin_fma(F[b], cf, V[b]);
+        } while (!last);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) val[4 * j + b][threadIdx.x] = V[b];
+    }
+    count_work(work, live, nodes);
+    if (!live) return;
+    double* row = Bt + (int64_t)perm[slot] * ldb + 4 * g0;
+    if (kPair && ngr == kGroups) {
+#pragma unroll
+        for (int j = 0; j < kBlockRecs; j += 2)
+            *reinterpret_cast<double2*>(row + j) = make_double2(val[j][threadIdx.x],
+                                                                val[j + 1][threadIdx.x]);
+    } else {
+        for (int j = 0; j < 4 * ngr; ++j) row[j] = val[j][threadIdx.x];
+    }
+}
+
 // acc[c][slot] = (first ? 0 : acc[c][slot]) + sum over slabs of partial[slab][c][slot].
 __global__ void k_acc_fold(int64_t n, int64_t slabs, const double* __restrict__ partial,
                            double* __restrict__ acc, int first) {
@@ -2275,6 +2406,13 @@ __global__ void k_compose(int64_t n, const int32_t* __restrict__ perm,
     if (t < n) out[t] = rep[perm[t]];
 }
 
+// Whether the passes of a call can share node lists: groups of four functions that no aux chunk
+// cuts, and lists long enough to earn their choice (use_node_sets).
+static bool exch_may_share(int64_t M, int64_t N, int64_t n, int64_t Pc) {
+    return N % M == 0 && (N / M) % kMaxSetScales == 0 && Pc % kMaxSetScales == 0 &&
+           use_node_sets(n, N / M, false);
+}
+
 int exch_tc_layout(Arena& ar, int64_t M, int64_t N, int64_t n, int64_t Pc, bool grads,
                    ExchTcWs* w) {
     *w = ExchTcWs{};
@@ -2296,6 +2434,11 @@ int exch_tc_layout(Arena& ar, int64_t M, int64_t N, int64_t n, int64_t Pc, bool 
     w->n_groups_dev = ar.take<int64_t>(1);
     w->scan_bytes = pair_groups_scan_bytes(n);
     w->scan_tmp = ar.take<char>(w->scan_bytes + 1);
+    if (exch_may_share(M, N, n, Pc)) {
+        const NodeSets ns = node_sets(N, N / M, kSetExchange);
+        w->sets = ar.take<double>(ns.stride * ns.groups + kSetSlack);
+        w->box = ar.take<double>(node_set_box_doubles());
+    }
     GSDFT_TRY(pair_order_layout(ar, n, &w->pair_order));
     if (grads) {
         // bwd_split(W, m).slabs x n (the moments' slot stride is n) over every chunk width
@@ -2311,6 +2454,9 @@ int exch_tc_layout(Arena& ar, int64_t M, int64_t N, int64_t n, int64_t Pc, bool 
     }
     return GSDFT_OK;
 }
+
+// The shared lists hold the 1/r kernel's nodes only.
+static bool exch_shares(const ExchTcWs& w) { return w.sets && w.table.n == kNodes; }
 
 int exch_tc_prologue(int64_t M, const double* quat, const double* log_scale,
                      const double* centers, int64_t N, const double* log_alpha,
@@ -2330,9 +2476,15 @@ int exch_tc_prologue(int64_t M, const double* quat, const double* log_scale,
     k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, pi, pj, w.A6, centers, w.Nrm, w.q, w.rec);
     GSDFT_HIP(hipGetLastError());
     const int64_t G = (N % M == 0) ? N / M : 1;
-    k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
-                                                      nullptr, kAuxPlain, w.table, w.aux);
-    GSDFT_HIP(hipGetLastError());
+    if (exch_shares(w)) {
+        GSDFT_TRY(launch_pair_box(n, nullptr, w.rec, kRec, w.box, s));
+        GSDFT_TRY(launch_node_sets(N, G, kSetExchange, w.beta, w.kn, aux_centers, nullptr, nullptr,
+                                   w.box, w.sets, s));
+    } else {
+        k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
+                                                          nullptr, kAuxPlain, w.table, w.aux);
+        GSDFT_HIP(hipGetLastError());
+    }
     // one record per group (its first entry's), then the groups' slot order: the group count
     // stays on the device, the first n_groups_dev slots are the groups and the rest idle
     GSDFT_TRY(launch_pair_groups(M, n, pi, pj, w.q, w.pair_order, w.head, w.scan_tmp,
@@ -2353,7 +2505,7 @@ int exch_tc_prologue(int64_t M, const double* quat, const double* log_scale,
 int exch_tc_block(int64_t M, int64_t N, int64_t q0, int64_t W, const double* aux_centers,
                   int64_t n, int64_t ldb, double* Bt, const ExchTcWs& w, hipStream_t s) {
     if (n <= 0 || W <= 0) return GSDFT_OK;
-    (void)M; (void)N; (void)aux_centers;
+    (void)aux_centers;
     const int64_t gy = (W + kBlockRecs - 1) / kBlockRecs;
     if (gy > 65535) return fail(GSDFT_ERR_ARG, "exchange: aux chunk too wide");
     dim3 grid((unsigned)((n + 255) / 256), (unsigned)gy);
@@ -2361,7 +2513,18 @@ int exch_tc_block(int64_t M, int64_t N, int64_t q0, int64_t W, const double* aux
     profile_begin(kProfExchBlock, s);
     unsigned long long* work = profile_work_counter(kProfExchBlock);
     const double* aux = w.aux + kAuxRec * q0;
-    if (w.table.n == kLrNodes) {
+    if (exch_shares(w)) {
+        const int64_t stride = node_sets(N, N / M, kSetExchange).stride;
+        const double* sets = w.sets + stride * (q0 / kMaxSetScales);
+        if (pair)
+            k_exch_block_sets<true><<<grid, 256, 0, s>>>(n, w.rec_sorted, w.pair_order.perm,
+                                                         W / kMaxSetScales, stride, sets, ldb, Bt,
+                                                         work, w.n_groups_dev);
+        else
+            k_exch_block_sets<false><<<grid, 256, 0, s>>>(n, w.rec_sorted, w.pair_order.perm,
+                                                          W / kMaxSetScales, stride, sets, ldb, Bt,
+                                                          work, w.n_groups_dev);
+    } else if (w.table.n == kLrNodes) {
         if (pair)
             k_exch_block_pairs<true, kLrNodes><<<grid, 256, 0, s>>>(n, w.rec_sorted,
                                                                     w.pair_order.perm, W, aux, ldb,
@@ -2389,10 +2552,20 @@ int exch_tc_reverse(int64_t N, int64_t q0, int64_t W, int64_t n, int64_t n_est,
                     const double* Tbar, int64_t ldt, bool group_rows, bool first,
                     const ExchTcWs& w, hipStream_t s) {
     if (n <= 0 || W <= 0) return GSDFT_OK;
-    const Split sp = bwd_split(W, std::max<int64_t>(1, std::min(n, n_est)));
+    Split sp = bwd_split(W, std::max<int64_t>(1, std::min(n, n_est)));
+    if (exch_shares(w)) {                 // whole groups per slab: never more slabs than bwd_split's
+        sp.per_slab = (sp.per_slab + kMaxSetScales - 1) / kMaxSetScales;
+        sp.slabs = (W / kMaxSetScales + sp.per_slab - 1) / sp.per_slab;
+    }
     dim3 grid((unsigned)((n + 255) / 256), (unsigned)sp.slabs);
     profile_begin(kProfExchBwd, s);
-    if (w.table.n == kLrNodes)
+    if (exch_shares(w)) {
+        const int64_t stride = node_sets(N, kMaxSetScales, kSetExchange).stride;
+        k_gamma_bwd<true, false, true, kNodes, true><<<grid, 256, 0, s>>>(
+            n, w.rec_sorted, W / kMaxSetScales, w.sets + stride * (q0 / kMaxSetScales),
+            sp.per_slab, w.part, profile_work_counter(kProfExchBwd), Tbar, ldt, nullptr,
+            w.pair_order.perm, w.grp_first, w.n_groups_dev, group_rows ? 1 : 0, 0, -1, stride);
+    } else if (w.table.n == kLrNodes)
         k_gamma_bwd<true, false, false, kLrNodes><<<grid, 256, 0, s>>>(
             n, w.rec_sorted, W, w.aux + kAuxRec * q0, sp.per_slab, w.part,
             profile_work_counter(kProfExchBwd), Tbar, ldt, nullptr, w.pair_order.perm,
@@ -2407,7 +2580,6 @@ int exch_tc_reverse(int64_t N, int64_t q0, int64_t W, int64_t n, int64_t n_est,
     GSDFT_HIP(hipGetLastError());
     k_acc_fold<<<blocks_for(n * kAcc, 256), 256, 0, s>>>(n, sp.slabs, w.part, w.acc, first ? 1 : 0);
     GSDFT_HIP(hipGetLastError());
-    (void)N;
     return GSDFT_OK;
 }
 
@@ -3022,7 +3194,7 @@ int gamma_run(int64_t M, const double* quat, const double* log_scale, const doub
                              weight, w, s));
     const int64_t G = (N % M == 0) ? N / M : 1;          // scales per centre of a product aux
     const int64_t groups = fwd_groups(N, n);
-    const NodeSets ns = node_sets(N, G, false);
+    const NodeSets ns = node_sets(N, G, kSetForward);
     const bool sets = use_node_sets(n, G, false) &&
                       ns.stride * ns.groups + kSetSlack + groups * N <= kRec * n;
     if (sets) {
@@ -3041,7 +3213,7 @@ int gamma_run(int64_t M, const double* quat, const double* log_scale, const doub
     double* const set_area = w.rec;
     double* const partial = sets ? w.rec + ns.stride * ns.groups + kSetSlack : w.partial;
     if (sets)
-        GSDFT_TRY(launch_node_sets(N, G, false, w.beta, w.kn, aux_centers, nullptr, nullptr, w.q,
+        GSDFT_TRY(launch_node_sets(N, G, kSetForward, w.beta, w.kn, aux_centers, nullptr, nullptr, w.q,
                                    set_area, s));
     const int64_t per_block = sets ? kFwdRecs / std::min<int64_t>(G, kMaxSetScales) : kFwdRecs;
     const int64_t nrb = ((sets ? ns.groups : N) + per_block - 1) / per_block;
@@ -3153,12 +3325,12 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
                              weight, w, s));
     if (n > 0) {
         const int64_t G = (N % M == 0) ? N / M : 1;      // scales per centre of a product aux
-        const NodeSets ns = node_sets(N, G, true);
+        const NodeSets ns = node_sets(N, G, kSetFold);
         const bool sets = use_node_sets(n, G, true) &&
                           ns.stride * ns.groups + kSetSlack <= kAuxRec * N + kAuxRec;
         if (sets) {
             GSDFT_TRY(launch_pair_box(n, nullptr, w.rec, kRec, w.q, s));
-            GSDFT_TRY(launch_node_sets(N, G, true, w.beta, w.kn, aux_centers, dgamma, dgamma_scale,
+            GSDFT_TRY(launch_node_sets(N, G, kSetFold, w.beta, w.kn, aux_centers, dgamma, dgamma_scale,
                                        w.q, w.aux, s));
         } else {
             k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers,

@@ -158,12 +158,12 @@ int launch_pair_groups(int64_t M, int64_t n, const int32_t* pi, const int32_t* p
 
 // nodeset.hip: the reach and widths of n pair records (the first 12 doubles as for
 // launch_pair_order; n_live as there) into scratch[0..7], scratch holding node_set_box_doubles();
-// and one node list per group of aux functions (layout: common.h), its weights plain (`fold`
-// false; dgamma, dscale and kn unread) or carrying dgamma_P dscale kn_P summed over the group.
+// and one node list per group of aux functions in the given form (layout: common.h; dgamma and
+// dscale are read for kSetFold only, whose weights carry dgamma_P dscale kn_P).
 size_t node_set_box_doubles();
 int launch_pair_box(int64_t n, const int64_t* n_live, const double* rec, int rec_stride,
                     double* scratch, hipStream_t s);
-int launch_node_sets(int64_t N, int64_t G, bool fold, const double* beta, const double* kn,
+int launch_node_sets(int64_t N, int64_t G, SetForm form, const double* beta, const double* kn,
                      const double* R, const double* dgamma, const double* dscale,
                      const double* box, double* out, hipStream_t s);
 
@@ -185,6 +185,7 @@ struct ExchTcWs {
     size_t scan_bytes;
     PairOrderWs pair_order;
     NodeTable table;        // the kernel's node rule (set after exch_tc_layout)
+    double *sets, *box;     // shared node lists and the pairs' reach (null: plain aux records)
 };
 // The node rule of the 1/r kernel and of the long-range erf(omega r)/r kernel (omega > 0).
 NodeTable coulomb_table();

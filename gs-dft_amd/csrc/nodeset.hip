@@ -118,14 +118,13 @@ template <int NB>
 __global__ __launch_bounds__(kSetThreads) void k_node_sets(
     int64_t N, int64_t G, int64_t per_centre, int64_t stride, const double* __restrict__ beta,
     const double* __restrict__ kn, const double* __restrict__ R,
-    const double* __restrict__ dgamma, const double* __restrict__ dscale, int fold,
+    const double* __restrict__ dgamma, const double* __restrict__ dscale, SetForm form,
     const double* __restrict__ box, NodeTable tb, double* __restrict__ out) {
     constexpr int kCols = kNodes * NB;
     constexpr int kMaxRank = NB == 4 ? 72 : kCols;      // pivot rows in LDS
     constexpr int RG = kSetThreads / kCols;           // row classes
     constexpr int RT = kSetRows / RG;                 // rows per thread
     static_assert(RG * RT == kSetRows && RG * kCols == kSetThreads && kCols * kSetRows <= 8192, "");
-    constexpr int kW = set_node_doubles(NB) - 2;
     constexpr int CH = RT % 4 == 0 ? 4 : 3;           // row classes per step of the K sums
     static_assert(RT % CH == 0, "");
     constexpr int kLd = kCols + 1;                    // odd: a column of U is free of conflicts
@@ -163,6 +162,35 @@ __global__ __launch_bounds__(kSetThreads) void k_node_sets(
         wp = tb.w[ct] / ((b + t2) * sqrt(b + t2));
     }
     const double norm = kExpMinusHalf / kExpQuarticK;
+    const int nd = set_node_doubles(NB, form);
+    // node `at` of the list at y: s, and the weights w[b] of the functions
+    auto put = [&](double* y, int at, double sn, const double w[NB]) {
+        y += nd * at;
+        const double wn = norm / sqrt(sn);
+        y[0] = sn;
+        if (form == kSetFold) {
+            double x = 0.0;
+            for (int b = 0; b < nb; ++b) {
+                const int64_t p = aux_of_slot(slot0 + b, N, G);
+                x += dgamma[p] * (dscale ? *dscale : 1.0) * kn[p] * w[b];
+            }
+            y[1] = wn * x;
+            y[2] = sn * sn;
+            y[3] = 1.0 / sn;
+            return;
+        }
+        y[1] = 1.0 / sn;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const double k = form == kSetExchange && b < nb ? kn[aux_of_slot(slot0 + b, N, G)]
+                                                            : 1.0;
+            y[2 + b] = b < nb ? wn * w[b] * k : 0.0;
+        }
+        if (form == kSetExchange) {
+            y[6] = sn * sn;
+            y[7] = 0.0;
+        }
+    };
     int rank = 0;
     if (shared) {
         // reach: from R to the far corner of the pairs' centres, plus some widths of the widest
@@ -264,23 +292,17 @@ __global__ __launch_bounds__(kSetThreads) void k_node_sets(
     if (!shared) {                                                     // workgroup-uniform
         // one sub-record per function, in slot order
         if (rg == 0 && real_col) {
-            double* x = o + cb * (kSetHeader + kNodes * (fold ? 4 : kW + 2));
+            double* x = o + cb * (kSetHeader + kNodes * nd);
             const int64_t p = aux_of_slot(slot0 + cb, N, G);
             if (ct == 0) {
                 x[0] = R[3 * p]; x[1] = R[3 * p + 1]; x[2] = R[3 * p + 2];
                 x[3] = __builtin_bit_cast(double, (uint64_t)kNodes |
                                                       ((uint64_t)(cb == nb - 1) << 32));
             }
-            const double w = wp / sqrt(s) * norm;
-            if (fold) {
-                double* y = x + kSetHeader + 4 * ct;
-                const double u = dgamma[p] * (dscale ? *dscale : 1.0) * kn[p];
-                y[0] = s; y[1] = w * u; y[2] = s * s; y[3] = 1.0 / s;
-            } else {
-                double* y = x + kSetHeader + (kW + 2) * ct;
-                y[0] = s; y[1] = 1.0 / s;
-                for (int b = 0; b < kW; ++b) y[2 + b] = b == cb ? w : 0.0;
-            }
+            double w[NB];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) w[b] = b == cb ? wp : 0.0;
+            put(x + kSetHeader, ct, s, w);
         }
         return;
     }
@@ -313,27 +335,14 @@ __global__ __launch_bounds__(kSetThreads) void k_node_sets(
             const double x = cs[piv[m]];
             pos += (x < sm || (x == sm && m < tid)) ? 1 : 0;
         }
-        const double w = cw[piv[tid]] / sqrt(sm) * norm;
-        if (fold) {
-            double x = 0.0;
-            for (int b = 0; b < nb; ++b) {
-                const int64_t p = aux_of_slot(slot0 + b, N, G);
-                x += dgamma[p] * (dscale ? *dscale : 1.0) * kn[p] * wsum[tid][b];
-            }
-            double* y = o + kSetHeader + 4 * pos;
-            y[0] = sm; y[1] = w * x; y[2] = sm * sm; y[3] = 1.0 / sm;
-            if (pos == rank - 1 && (rank & 1)) {                       // an odd list's last node
-                y[4] = sm; y[5] = 0.0; y[6] = sm * sm; y[7] = 1.0 / sm;   // again, weight 0
-            }
-        } else {
-            double* y = o + kSetHeader + (kW + 2) * pos;
-            y[0] = sm; y[1] = 1.0 / sm;
-            for (int b = 0; b < kW; ++b) y[2 + b] = b < nb ? w * wsum[tid][b] : 0.0;
-            if (pos == rank - 1 && (rank & 1)) {
-                y += kW + 2;
-                y[0] = sm; y[1] = 1.0 / sm;
-                for (int b = 0; b < kW; ++b) y[2 + b] = 0.0;
-            }
+        double w[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) w[b] = cw[piv[tid]] * wsum[tid][b];
+        put(o + kSetHeader, pos, sm, w);
+        if (pos == rank - 1 && (rank & 1)) {      // an odd list's last node again, weight 0
+#pragma unroll
+            for (int b = 0; b < NB; ++b) w[b] = 0.0;
+            put(o + kSetHeader, rank, sm, w);
         }
     }
 }
@@ -350,19 +359,18 @@ int launch_pair_box(int64_t n, const int64_t* n_live, const double* rec, int rec
     return GSDFT_OK;
 }
 
-int launch_node_sets(int64_t N, int64_t G, bool fold, const double* beta, const double* kn,
+int launch_node_sets(int64_t N, int64_t G, SetForm form, const double* beta, const double* kn,
                      const double* R, const double* dgamma, const double* dscale,
                      const double* box, double* out, hipStream_t s) {
-    const NodeSets ns = node_sets(N, G, fold);
+    const NodeSets ns = node_sets(N, G, form);
     const unsigned g = (unsigned)ns.groups;
     const NodeTable tb = coulomb_table();
-    const int f = fold ? 1 : 0;
     if (ns.nb == 2)
         k_node_sets<2><<<g, kSetThreads, 0, s>>>(N, G, ns.per_centre, ns.stride, beta, kn, R,
-                                                 dgamma, dscale, f, box, tb, out);
+                                                 dgamma, dscale, form, box, tb, out);
     else
         k_node_sets<4><<<g, kSetThreads, 0, s>>>(N, G, ns.per_centre, ns.stride, beta, kn, R,
-                                                 dgamma, dscale, f, box, tb, out);
+                                                 dgamma, dscale, form, box, tb, out);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
 }

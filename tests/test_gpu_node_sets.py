@@ -66,3 +66,33 @@ def test_gamma_and_reverse_match_oracle(g, wl, orc, cuda, name):
         err = rel_max(a.cpu().numpy(), b)
         print(f"[sets] {name}: d{what} {err:.2e}", flush=True)
         assert err < 1e-9
+
+
+@pytest.mark.parametrize("scales", [(0.5, 1.0, 2.0, 4.0), (0.5, 0.7, 1.0, 1.4, 2.0, 2.8, 4.0, 5.6)])
+def test_exchange_on_shared_lists_matches_plain_records(g, wl, cuda, scales):
+    """RI-K takes the shared lists when the scales come in fours and no aux chunk cuts a group; an
+    aux chunk of 66 functions does, so the same call then runs on the plain records (checked against
+    the oracle elsewhere). lam = 1e-2 keeps the metric's condition near 1e4, where two correct
+    evaluations agree to the parity bars, 1e-10 for E_K and 1e-9 for gradients. Chunks of 64 and of
+    100 functions leave ragged last blocks and slabs."""
+    s = wl.make_small(190, 5, n_atoms=6, seed=4, spread=3.0)
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    basis = g.Splat(quat=t(s.quat), log_scale=t(s.log_scale), centers=t(s.centers))
+    C = t(s.C)
+    aux = g.init_product_aux(basis, scales=scales)
+    pi, pj, v = g.neighbor_pairs(basis, eps=1e-9, unique=False)
+    assert pi.shape[0] >= N_MIN
+    L = g.aux_cholesky(aux, 1e-2)
+
+    def run(chunk):
+        E = g.df_exchange_energy_screened(basis, C, aux, pi, pj, valid=v, cholV=L, aux_chunk=chunk)
+        return [E.detach()] + list(torch.autograd.grad(E, [basis.quat, basis.log_scale,
+                                                           basis.centers, C]))
+
+    plain = [x.cpu().numpy() for x in run(66)]
+    for chunk in (0, 64, 100):
+        got = [x.cpu().numpy() for x in run(chunk)]
+        errs = [rel_max(a, b) for a, b in zip(got, plain)]
+        print(f"[sets] exchange {len(scales)} scales, chunk {chunk}: n={pi.shape[0]} "
+              + " ".join(f"{e:.1e}" for e in errs), flush=True)
+        assert errs[0] < 1e-10 and max(errs[1:]) < 1e-9
