@@ -1685,11 +1685,12 @@ __device__ __forceinline__ double wave_sum_x(double v) {
 // ket_part[x][b - A0] for the whole slab (zeros where a wave had no ket). Lanes with a > b (only
 // near the diagonal) contribute nothing and do not hold the wave in the node loop.
 // 768 kets per workgroup: the per-wave ket sums then take 24 KB of LDS, so the kernel runs the
-// five waves per SIMD its registers allow (1024 kets, 32 KB: four, 1.9% slower).
+// five waves per SIMD its registers allow (1024 kets, 32 KB: four, 1.9% slower); shorter slabs
+// (eri_slab) where the list leaves too few workgroups.
 constexpr int kEriSymSlab = 768;
 
 __global__ __launch_bounds__(256) void k_eri_fwd_sym(int64_t n, const double* __restrict__ rec,
-                                                     int64_t A0, int64_t H,
+                                                     int64_t A0, int64_t H, int slab,
                                                      double* __restrict__ bra_part,
                                                      double* __restrict__ ket_part,
                                                      unsigned long long* __restrict__ work) {
@@ -1707,8 +1708,8 @@ __global__ __launch_bounds__(256) void k_eri_fwd_sym(int64_t n, const double* __
     const double Px = live ? ra[6] : kFarAway, Py = live ? ra[7] : kFarAway,
                  Pz = live ? ra[8] : kFarAway;
     const double ca = live ? ra[9] * ra[10] : 0.0;
-    const int64_t kb0 = A0 + (int64_t)blockIdx.y * kEriSymSlab;
-    const int64_t kb1 = min(n, kb0 + kEriSymSlab);
+    const int64_t kb0 = A0 + (int64_t)blockIdx.y * slab;
+    const int64_t kb1 = min(n, kb0 + slab);
     const int64_t amin = A0 + (int64_t)blockIdx.x * 256 + wv * 64;
     const double c256 = vgpr_const(kNegC256);
     double acc = 0.0;
@@ -1773,8 +1774,10 @@ __global__ void k_eri_sym_reduce(int64_t n, int64_t A0, int64_t H, int64_t group
     const int64_t b = A0 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (b >= n) return;
     double s = 0.0;
+#pragma unroll 8
     for (int64_t x = 0; x < groups; ++x) s += ket_part[x * (n - A0) + (b - A0)];
     if (b < A0 + H)
+#pragma unroll 8
         for (int64_t y = 0; y < slabs; ++y) s += bra_part[y * acc_stride + (b - A0)];
     Jacc[b] += s;
 }
@@ -1794,12 +1797,10 @@ constexpr int kEriAcc = 10;
 // and the ket's moments c_a (F, gT, -gd) (T is symmetric in a and b, d changes sign) are summed over
 // the wave (wave_sum10) and written per wave to ket_part[(4 x + wave) * 10 + c][b - A0] for every
 // ket of the workgroup's slab (zeros where the wave had no ket).
-// kets per workgroup of the reverse: the forward's, so that both passes sum the bra partials of
-// a band over the same slabs and their E_J agree bit for bit
-constexpr int kEriSymSlabB = kEriSymSlab;
-
+// The kets per workgroup (`slab`) are the forward's, so that both passes sum the bra partials of a
+// band over the same slabs and their E_J agree bit for bit.
 __global__ __launch_bounds__(256) void k_eri_bwd_sym(int64_t n, const double* __restrict__ rec,
-                                                     int64_t A0, int64_t H,
+                                                     int64_t A0, int64_t H, int slab,
                                                      double* __restrict__ bra_part,
                                                      double* __restrict__ ket_part,
                                                      unsigned long long* __restrict__ work) {
@@ -1815,8 +1816,8 @@ __global__ __launch_bounds__(256) void k_eri_bwd_sym(int64_t n, const double* __
     const double Px = live ? ra[6] : kFarAway, Py = live ? ra[7] : kFarAway,
                  Pz = live ? ra[8] : kFarAway;
     const double ca = live ? ra[9] * ra[10] : 0.0;
-    const int64_t kb0 = A0 + (int64_t)blockIdx.y * kEriSymSlabB;
-    const int64_t kb1 = min(n, kb0 + kEriSymSlabB);
+    const int64_t kb0 = A0 + (int64_t)blockIdx.y * slab;
+    const int64_t kb1 = min(n, kb0 + slab);
     const int64_t amin = A0 + (int64_t)blockIdx.x * 256 + wv * 64;
     const int64_t nk = n - A0;
     double* __restrict__ kp = ket_part + ((int64_t)blockIdx.x * 4 + wv) * kEriAcc * nk;
@@ -1915,21 +1916,21 @@ __global__ __launch_bounds__(256) void k_eri_bwd_sym(int64_t n, const double* __
 }
 
 // The band's share of every pair's ten reverse moments, in a fixed order: first
-// macc[c][b] += sum_x ket_part[x * 10 + c][b - A0] (x in order) for every b >= A0 (one thread per b),
+// macc[c][b] += sum_x ket_part[x * 10 + c][b - A0] (x in order) for every b >= A0 (one thread per
+// (b, c): with one per b the 29 k pairs of a small molecule kept 450 waves busy, 1.3 ms against 0.18),
 // then macc[c][b] += sum_y bra_part[y * 10 + c][b - A0] (y in order) for b in the band (one thread per
 // (c, b)).
 __global__ void k_eri_sym_reduce10_ket(int64_t n, int64_t A0, int64_t waves,
                                        const double* __restrict__ ket_part,
                                        double* __restrict__ macc) {
     const int64_t b = A0 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int c = blockIdx.y;
     if (b >= n) return;
     const int64_t nk = n - A0;
-#pragma unroll
-    for (int c = 0; c < kEriAcc; ++c) {
-        double s = 0.0;
-        for (int64_t x = 0; x < waves; ++x) s += ket_part[(x * kEriAcc + c) * nk + (b - A0)];
-        macc[(int64_t)c * n + b] += s;
-    }
+    double s = 0.0;
+#pragma unroll 8
+    for (int64_t x = 0; x < waves; ++x) s += ket_part[(x * kEriAcc + c) * nk + (b - A0)];
+    macc[(int64_t)c * n + b] += s;
 }
 
 __global__ void k_eri_sym_reduce10_bra(int64_t n, int64_t A0, int64_t H, int64_t slabs,
@@ -1940,6 +1941,7 @@ __global__ void k_eri_sym_reduce10_bra(int64_t n, int64_t A0, int64_t H, int64_t
     if (t >= kEriAcc * hb) return;
     const int64_t c = t / hb, i = t % hb;
     double s = 0.0;
+#pragma unroll 8
     for (int64_t y = 0; y < slabs; ++y) s += bra_part[(y * kEriAcc + c) * H + i];
     macc[c * n + A0 + i] += s;
 }
@@ -3613,20 +3615,41 @@ struct EriWs {
     PairOrderWs order;
 };
 
-// Bra band height of the symmetric forward: a multiple of 256, at most 16384, with the band's
-// ket partials ((band / 256) x n doubles) within 1 GiB.
+// Kets per workgroup of the symmetric passes. 256 bras against 768 kets are a millisecond of one
+// workgroup's work, and a CU holds three (reverse) or five: while the triangle of pair-pairs has
+// fewer than kEriBlocks of them (thirty rounds of the chip), the slab is halved, down to 192 kets
+// (shorter slabs only where not even kEriFew workgroups are left, as each writes its bras' partial
+// sums), so that an uneven last round costs little: energy and gradients of 28 k pairs 15.4 -> 8.6
+// ms, 50 k 35.1 -> 28.4, 167 k 429 -> 411.
+constexpr double kEriBlocks = 24576.0, kEriFew = 2048.0;
+int eri_slab(int64_t n) {
+    int slab = kEriSymSlab;
+    auto blocks = [&] { return 0.5 * (double)n * (double)n / (256.0 * slab); };
+    while (slab > 192 && blocks() < kEriBlocks) slab /= 2;
+    while (slab > 48 && blocks() < kEriFew) slab /= 2;
+    return slab;
+}
+
+// Bra groups of 256 per band, before the memory caps below: 128 (one band for a small list) while
+// the reverse's ket partials allow it, else 64. Both passes use the same, so that they agree bit for
+// bit wherever the caps do not differ.
+int64_t eri_groups(int64_t n) {
+    const int64_t fit = ((int64_t)1 << 30) / (kEriAcc * std::max<int64_t>(n, 1)) / 4;
+    return std::min<int64_t>((n + 255) / 256, fit >= 128 ? 128 : 64);
+}
+
+// Bra band height of the symmetric forward: eri_groups, with the band's ket partials
+// ((band / 256) x n doubles) within 1 GiB.
 int64_t eri_band(int64_t n) {
     const int64_t groups_cap = std::max<int64_t>(1, ((int64_t)1 << 27) / std::max<int64_t>(n, 1));
-    int64_t groups = std::min<int64_t>({(n + 255) / 256, 64, groups_cap});
-    return std::max<int64_t>(groups, 1) * 256;
+    return std::max<int64_t>(std::min(eri_groups(n), groups_cap), 1) * 256;
 }
 
 // The same for the reverse, whose ket partials are (band / 64) x 10 x n doubles, within 8 GiB
 // (fewer, fuller band launches: the reverse is the longer pass).
 int64_t eri_band10(int64_t n) {
     const int64_t waves_cap = ((int64_t)1 << 30) / (kEriAcc * std::max<int64_t>(n, 1));
-    const int64_t groups = std::min<int64_t>({(n + 255) / 256, 64, waves_cap / 4});
-    return std::max<int64_t>(groups, 1) * 256;
+    return std::max<int64_t>(std::min(eri_groups(n), waves_cap / 4), 1) * 256;
 }
 
 int layout_eri(Arena& ar, int64_t M, int64_t n, bool grads, EriWs* w) {
@@ -3641,7 +3664,7 @@ int layout_eri(Arena& ar, int64_t M, int64_t n, bool grads, EriWs* w) {
     w->band = 0;
     if (grads) {
         w->band = eri_band10(n);
-        const int64_t slabs = (n + kEriSymSlabB - 1) / kEriSymSlabB;
+        const int64_t slabs = (n + eri_slab(n) - 1) / eri_slab(n);
         w->jacc = ar.take<double>(kEriAcc * n + 1);
         w->bra_part = ar.take<double>(slabs * kEriAcc * w->band + 1);
         w->ket_part = ar.take<double>((w->band / 64) * kEriAcc * n + 1);
@@ -3649,7 +3672,7 @@ int layout_eri(Arena& ar, int64_t M, int64_t n, bool grads, EriWs* w) {
         w->contrib = ar.take<double>(20 * n + 1);
     } else {
         w->band = eri_band(n);
-        const int64_t slabs = (n + kEriSymSlab - 1) / kEriSymSlab;
+        const int64_t slabs = (n + eri_slab(n) - 1) / eri_slab(n);
         w->jacc = ar.take<double>(n + 1);
         w->bra_part = ar.take<double>(slabs * w->band + 1);
         w->ket_part = ar.take<double>((w->band / 256) * n + 1);
@@ -3754,18 +3777,19 @@ int exact_run(int64_t M, const double* quat, const double* log_scale, const doub
     k_eri_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, w.order.perm, pi, pj, w.A6, centers, w.Nrm,
                                                  w.q, weight, w.rec);
     GSDFT_HIP(hipGetLastError());
+    const int slab = eri_slab(n);
     if (!grads) {
         // bands of bra slots, each against the kets from its own start on
-        if ((n + kEriSymSlab - 1) / kEriSymSlab > 65535)
+        if ((n + slab - 1) / slab > 65535)
             return fail(GSDFT_ERR_ARG, "%s: n exceeds the supported %lld pairs", name,
-                        (long long)65535 * kEriSymSlab);
+                        (long long)65535 * slab);
         k_fill<<<blocks_for(n, 256), 256, 0, s>>>(n, 0.0, w.jacc);
         profile_begin(kProfEriFwd, s);
         for (int64_t A0 = 0; A0 < n; A0 += w.band) {
             const int64_t hb = std::min(w.band, n - A0);
             dim3 g((unsigned)((hb + 255) / 256),
-                   (unsigned)((n - A0 + kEriSymSlab - 1) / kEriSymSlab));
-            k_eri_fwd_sym<<<g, 256, 0, s>>>(n, w.rec, A0, w.band, w.bra_part, w.ket_part,
+                   (unsigned)((n - A0 + slab - 1) / slab));
+            k_eri_fwd_sym<<<g, 256, 0, s>>>(n, w.rec, A0, w.band, slab, w.bra_part, w.ket_part,
                                             profile_work_counter(kProfEriFwd));
             k_eri_sym_reduce<<<blocks_for(n - A0, 256), 256, 0, s>>>(
                 n, A0, w.band, g.x, g.y, w.band, w.bra_part, w.ket_part, w.jacc);
@@ -3774,18 +3798,18 @@ int exact_run(int64_t M, const double* quat, const double* log_scale, const doub
         GSDFT_HIP(hipGetLastError());
         k_eri_finish<<<blocks_for(n, 256), 256, 0, s>>>(n, 1, w.order.perm, w.rec, w.jacc, J);
     } else {
-        if ((n + kEriSymSlabB - 1) / kEriSymSlabB > 65535)
+        if ((n + slab - 1) / slab > 65535)
             return fail(GSDFT_ERR_ARG, "%s: n exceeds the supported %lld pairs", name,
-                        (long long)65535 * kEriSymSlabB);
+                        (long long)65535 * slab);
         k_fill<<<blocks_for(kEriAcc * n, 256), 256, 0, s>>>(kEriAcc * n, 0.0, w.jacc);
         profile_begin(kProfEriBwd, s);
         for (int64_t A0 = 0; A0 < n; A0 += w.band) {
             const int64_t hb = std::min(w.band, n - A0);
             dim3 g((unsigned)((hb + 255) / 256),
-                   (unsigned)((n - A0 + kEriSymSlabB - 1) / kEriSymSlabB));
-            k_eri_bwd_sym<<<g, 256, 0, s>>>(n, w.rec, A0, w.band, w.bra_part, w.ket_part,
+                   (unsigned)((n - A0 + slab - 1) / slab));
+            k_eri_bwd_sym<<<g, 256, 0, s>>>(n, w.rec, A0, w.band, slab, w.bra_part, w.ket_part,
                                             profile_work_counter(kProfEriBwd));
-            k_eri_sym_reduce10_ket<<<blocks_for(n - A0, 256), 256, 0, s>>>(
+            k_eri_sym_reduce10_ket<<<dim3(blocks_for(n - A0, 256), kEriAcc), 256, 0, s>>>(
                 n, A0, 4 * (int64_t)g.x, w.ket_part, w.jacc);
             k_eri_sym_reduce10_bra<<<blocks_for(kEriAcc * hb, 256), 256, 0, s>>>(
                 n, A0, w.band, g.y, w.bra_part, w.jacc);
