@@ -418,18 +418,13 @@ __global__ void k_pair_rec(int64_t n, const int32_t* __restrict__ pi,
     r[15] = 0.0;
 }
 
-// Node constants of one aux exponent b for the first tb.n nodes of the table:
-// s_t = t^2 b / (b + t^2), wp_t = w_t (b + t^2)^(-3/2).
-__device__ __forceinline__ void node_consts(double b, const NodeTable& tb, double s[kNodes],
-                                            double wp[kNodes]) {
-#pragma unroll
-    for (int t = 0; t < kNodes; ++t) {
-        if (t >= tb.n) break;
-        const double t2 = tb.t[t] * tb.t[t];
-        const double a = b + t2;
-        s[t] = t2 * b / a;
-        wp[t] = tb.w[t] / (a * sqrt(a));
-    }
+// Node constants of one aux exponent b at the node (t, w) of the table: s_t = t^2 b / (b + t^2),
+// wp_t = w_t (b + t^2)^(-3/2).
+__device__ __forceinline__ void node_const(double b, double t, double w, double* s, double* wp) {
+    const double t2 = t * t;
+    const double a = b + t2;
+    *s = t2 * b / a;
+    *wp = w / (a * sqrt(a));
 }
 
 // ------------------------------------------------------------------ node screen
@@ -874,42 +869,48 @@ __device__ __forceinline__ double wave_sum3(const double v[3], int* comp) {
 
 enum AuxFold { kAuxPlain = 0, kAuxFoldU = 1, kAuxForward = 2 };
 
+// One thread per (aux function, node): with one per function the divisions, roots and logarithms of
+// its twenty nodes took 21 us of a small system's pass, whatever its size (504 functions: 5 us).
 __global__ void k_aux_bwd_prep(int64_t N, int64_t G, const double* __restrict__ beta,
                                const double* __restrict__ kn, const double* __restrict__ R,
                                const double* __restrict__ dgamma,
                                const double* __restrict__ dscale, int fold, NodeTable tb,
                                double* __restrict__ out) {
-    const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t p = i / kNodes;
+    const int t = (int)(i % kNodes);
     if (p >= N) return;
     const double b = beta[p];
-    double s[kNodes], wp[kNodes];
-    node_consts(b, tb, s, wp);
     const int64_t slot = aux_slot(p, N, G);
     double* o = out + kAuxRec * slot;
-    o[0] = R[3 * p]; o[1] = R[3 * p + 1]; o[2] = R[3 * p + 2];
     const double u = (dgamma ? dgamma[p] : 1.0) * (dscale ? *dscale : 1.0) * kn[p];
-    o[3] = u;
-    bool first = true;
-    if (slot > 0) {
-        const int64_t q = aux_of_slot(slot - 1, N, G);
-        first = !(__builtin_bit_cast(uint64_t, R[3 * q]) == __builtin_bit_cast(uint64_t, R[3 * p]) &&
-                  __builtin_bit_cast(uint64_t, R[3 * q + 1]) ==
-                      __builtin_bit_cast(uint64_t, R[3 * p + 1]) &&
-                  __builtin_bit_cast(uint64_t, R[3 * q + 2]) ==
-                      __builtin_bit_cast(uint64_t, R[3 * p + 2]));
-    }
-    o[4] = b; o[5] = first ? 1.0 : 0.0; o[6] = 0.0; o[7] = 0.0;
-    for (int t = 0; t < kNodes; ++t) {
-        if (t < tb.n && fold == kAuxForward) {
-            put_fwd_node_consts(o, t, s[t], wp[t]);
-        } else if (t < tb.n) {
-            put_node_consts(o, t, s[t], wp[t], fold == kAuxFoldU ? u : 1.0);
-        } else {            // slots past the table: never read by a kernel of tb.n nodes
-            o[rec_s(t)] = 0.0;
-            o[rec_wh(t)] = 0.0;
-            o[rec_s2(t)] = 0.0;
-            o[rec_is(t)] = 0.0;
+    if (t == 0) {
+        o[0] = R[3 * p]; o[1] = R[3 * p + 1]; o[2] = R[3 * p + 2];
+        o[3] = u;
+        bool first = true;
+        if (slot > 0) {
+            const int64_t q = aux_of_slot(slot - 1, N, G);
+            first = !(__builtin_bit_cast(uint64_t, R[3 * q]) ==
+                          __builtin_bit_cast(uint64_t, R[3 * p]) &&
+                      __builtin_bit_cast(uint64_t, R[3 * q + 1]) ==
+                          __builtin_bit_cast(uint64_t, R[3 * p + 1]) &&
+                      __builtin_bit_cast(uint64_t, R[3 * q + 2]) ==
+                          __builtin_bit_cast(uint64_t, R[3 * p + 2]));
         }
+        o[4] = b; o[5] = first ? 1.0 : 0.0; o[6] = 0.0; o[7] = 0.0;
+    }
+    if (t < tb.n) {
+        double s, wp;
+        node_const(b, tb.t[t], tb.w[t], &s, &wp);
+        if (fold == kAuxForward)
+            put_fwd_node_consts(o, t, s, wp);
+        else
+            put_node_consts(o, t, s, wp, fold == kAuxFoldU ? u : 1.0);
+    } else {                // slots past the table: never read by a kernel of tb.n nodes
+        o[rec_s(t)] = 0.0;
+        o[rec_wh(t)] = 0.0;
+        o[rec_s2(t)] = 0.0;
+        o[rec_is(t)] = 0.0;
     }
 }
 
@@ -1366,7 +1367,7 @@ __device__ void pair_reverse(int64_t n, int64_t a, int64_t i, int64_t j,
 // Per pair: sum the slab moments, map them to dE/dAh, dE/dPa, dE/dKN_a, then through
 // gs_dft/coulomb/stream.py:203-215 to the two splats. Writes J and the two splats' parts
 // (pair_reverse).
-// Slot `slot` (of n) holds pair a = perm[slot] (its record and slab moments are stored by slot,
+// Slot `slot` (of n) holds pair a = perm[slot] (a = slot for a null perm; its record and slab moments are stored by slot,
 // stride n); J and contrib are indexed by pair, stride nc. pref is the integral's prefactor
 // (2 pi^3/sqrt(pi) for (P|a), 2 pi for the nuclear attraction); a null weight treats every entry
 // as live.
@@ -1382,7 +1383,7 @@ __global__ void k_pair_finalize(int64_t n, int64_t nc, int64_t slabs, double pre
                                 const int64_t* __restrict__ n_live = nullptr) {
     const int64_t slot = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (slot >= (n_live ? *n_live : n)) return;       // n_live: a device count of real slots
-    const int64_t a = perm[slot];
+    const int64_t a = perm ? perm[slot] : slot;
     if (weight && weight[a] == 0.0) {
         J[a] = 0.0;
         zero_splat_parts(contrib, nc, a);
@@ -1459,8 +1460,8 @@ __global__ __launch_bounds__(256) void k_splat_grad(
 }
 
 // dE/dC_mo = occ_o [sum_{a: i_a=m} J_a w_a C_{j_a o} + sum_{a: j_a=m} J_a w_a C_{i_a o}]
-// (gs_dft/coulomb/ri.py:456 reverse). The orbitals are cut into chunks of 256 CH, one workgroup
-// per (chunk, splat), thread t owning orbitals o = base + t + 256 c (c < CH) and streaming the
+// (gs_dft/coulomb/ri.py:456 reverse). The orbitals are cut into chunks of 256, one workgroup
+// per (chunk, splat), thread t owning orbital o = base + t and streaming the
 // partners' chunk rows coalesced. The splat's pairs (its CSR row, then its column) are taken 256
 // at a time: each thread resolves one pair's partner and scale J_a w_a into LDS, so the streaming
 // loop carries no dependent index loads. The logical blocks run chunk-major and XCD-contiguously,
@@ -1468,8 +1469,12 @@ __global__ __launch_bounds__(256) void k_splat_grad(
 // of their partners) for one chunk and find part of those rows in that XCD's L2: 32.0 ms at the
 // 700-atom globule against 36.0 ms with whole rows per workgroup (512-orbital chunks: 32.9 ms).
 // Each output element is summed by one thread over the pairs in CSR order.
-template <int CH>
-__global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunks,
+//
+// Few orbitals leave most of a workgroup's threads without one: L = 256 >> log2g threads (at least
+// k) then take a partner's row and 1 << log2g partners are summed side by side, each thread its
+// share of the partners in order, the shares in order at the end (CO2, k = 11: 27.6 us for 250
+// partner rows one after the other).
+__global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunks, int log2g,
                                             const int32_t* __restrict__ row_ptr,
                                             const int32_t* __restrict__ row_perm,
                                             const int32_t* __restrict__ col_ptr,
@@ -1485,12 +1490,14 @@ __global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunk
     __shared__ double scale[256];
     const int64_t lb = xcd_block(M * nchunks);
     if (lb < 0) return;                          // workgroup-uniform
-    const int64_t m = lb % M, base = (lb / M) * (256 * CH);
+    const int64_t m = lb % M, base = (lb / M) * 256;
     const int64_t r0 = row_ptr[m], r1 = row_ptr[m + 1], c0 = col_ptr[m], c1 = col_ptr[m + 1];
     const int64_t nr = r1 - r0, total = nr + (c1 - c0);
-    double acc[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c) acc[c] = 0.0;
+    const int L = 256 >> log2g, groups = 1 << log2g;
+    const int g = threadIdx.x / L;
+    const int64_t o = base + (threadIdx.x & (L - 1));
+    const int64_t oc = o < k ? o : k - 1;        // threads past k read its last column, store nothing
+    double acc = 0.0;
     for (int64_t b0 = 0; b0 < total; b0 += 256) {
         const int64_t e = b0 + threadIdx.x;
         if (e < total) {
@@ -1500,22 +1507,18 @@ __global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunk
         }
         __syncthreads();
         const int cnt = (int)min((int64_t)256, total - b0);
-        for (int q = 0; q < cnt; ++q) {
-            const double sc = scale[q];
-            const double* __restrict__ row = C + (int64_t)partner[q] * k;
-#pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const int64_t o = base + threadIdx.x + 256 * c;
-                if (o < k) acc[c] = __builtin_fma(sc, row[o], acc[c]);
-            }
-        }
+#pragma unroll 4
+        for (int q = g; q < cnt; q += groups)
+            acc = __builtin_fma(scale[q], C[(int64_t)partner[q] * k + oc], acc);
         __syncthreads();
     }
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int64_t o = base + threadIdx.x + 256 * c;
-        if (o < k) dC[m * k + o] = occ[o] * acc[c];
+    if (groups > 1) {
+        scale[threadIdx.x] = acc;
+        __syncthreads();
+        if (g != 0) return;
+        for (int h = 1; h < groups; ++h) acc += scale[h * L + threadIdx.x];
     }
+    if (o < k) dC[m * k + o] = occ[o] * acc;
 }
 
 // ------------------------------------------------------------------ nuclear attraction
@@ -2371,19 +2374,21 @@ int launch_dC(int64_t M, int64_t k, const int32_t* row_ptr, const int32_t* row_p
               const int32_t* col_ptr, const int32_t* col_perm, const int32_t* pi,
               const int32_t* pj, const double* J, const double* weight, const double* C,
               const double* occ, double* dC, hipStream_t s) {
-    constexpr int kCH = 1;                                 // orbitals per thread and chunk
-    const int64_t nchunks = (k + 256 * kCH - 1) / (256 * kCH);
+    const int64_t nchunks = (k + 255) / 256;
+    int log2g = 0;
+    while (log2g < 4 && (256 >> (log2g + 1)) >= k) ++log2g;
     if (M * nchunks > (int64_t)(UINT32_MAX / 256))
         return fail(GSDFT_ERR_ARG, "dC: M = %lld x %lld orbital chunks too many for one launch",
                     (long long)M, (long long)nchunks);
-    k_dC<kCH><<<xcd_grid(M * nchunks), 256, 0, s>>>(M, k, nchunks, row_ptr, row_perm, col_ptr,
-                                                    col_perm, pi, pj, J, weight, C, occ, dC);
+    k_dC<<<xcd_grid(M * nchunks), 256, 0, s>>>(M, k, nchunks, log2g, row_ptr, row_perm, col_ptr,
+                                               col_perm, pi, pj, J, weight, C, occ, dC);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
 }
 
 // Shared prologue of forward and reverse: chart, aux quantities (skipped for a null log_alpha),
-// pair density (zero for a null C), pair records.
+// pair density (zero for a null C), pair records in list order (w.rec; w.rec_sorted where the list
+// keeps its order).
 int gamma_prologue(int64_t M, const double* quat, const double* log_scale, const double* centers,
                    int64_t k, const double* C, const double* occ, int64_t N,
                    const double* log_alpha, int64_t n, const int32_t* pi, const int32_t* pj,
@@ -2400,10 +2405,26 @@ int gamma_prologue(int64_t M, const double* quat, const double* log_scale, const
             k_fill<<<blocks_for(n, 256), 256, 0, s>>>(n, 0.0, w.q);
             GSDFT_HIP(hipGetLastError());
         }
-        k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, pi, pj, w.A6, centers, w.Nrm, w.q, w.rec);
+        k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, pi, pj, w.A6, centers, w.Nrm, w.q,
+                                                      pair_list_order(n) ? w.rec_sorted : w.rec);
         GSDFT_HIP(hipGetLastError());
     }
     return GSDFT_OK;
+}
+
+// The records in slot order (w.rec_sorted) and, unless the list keeps its order, w.pair_order.perm.
+int sort_records(int64_t n, GammaWs& w, hipStream_t s) {
+    if (pair_list_order(n)) return GSDFT_OK;
+    GSDFT_TRY(launch_pair_order(n, w.rec, kRec, w.pair_order, s));
+    k_rec_gather<<<blocks_for(n * kRec, 256), 256, 0, s>>>(n, w.pair_order.perm, w.rec,
+                                                            w.rec_sorted);
+    GSDFT_HIP(hipGetLastError());
+    return GSDFT_OK;
+}
+
+// Slot -> pair, null where they are the same.
+const int32_t* slot_perm(int64_t n, const GammaWs& w) {
+    return pair_list_order(n) ? nullptr : w.pair_order.perm;
 }
 
 
@@ -2503,7 +2524,7 @@ int exch_tc_prologue(int64_t M, const double* quat, const double* log_scale,
         GSDFT_TRY(launch_node_sets(N, G, kSetExchange, w.beta, w.kn, aux_centers, nullptr, nullptr,
                                    w.box, w.sets, s));
     } else {
-        k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
+        k_aux_bwd_prep<<<blocks_for(N * kNodes, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
                                                           nullptr, kAuxPlain, w.table, w.aux);
         GSDFT_HIP(hipGetLastError());
     }
@@ -3220,17 +3241,15 @@ int gamma_run(int64_t M, const double* quat, const double* log_scale, const doub
     const bool sets = use_node_sets(n, G, false) &&
                       ns.stride * ns.groups + kSetSlack + groups * N <= kRec * n;
     if (sets) {
-        GSDFT_TRY(launch_pair_box(n, nullptr, w.rec, kRec, w.q, s));
+        GSDFT_TRY(launch_pair_box(n, nullptr, pair_list_order(n) ? w.rec_sorted : w.rec, kRec,
+                                  w.q, s));
     } else {
-        k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
+        k_aux_bwd_prep<<<blocks_for(N * kNodes, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
                                                           nullptr, kAuxForward, coulomb_table(),
                                                           w.aux);
         GSDFT_HIP(hipGetLastError());
     }
-    GSDFT_TRY(launch_pair_order(n, w.rec, kRec, w.pair_order, s));
-    k_rec_gather<<<blocks_for(n * kRec, 256), 256, 0, s>>>(n, w.pair_order.perm, w.rec,
-                                                            w.rec_sorted);
-    GSDFT_HIP(hipGetLastError());
+    GSDFT_TRY(sort_records(n, w, s));
     // the node lists take the dead pair records' slice as the block sums do, before them
     double* const set_area = w.rec;
     double* const partial = sets ? w.rec + ns.stride * ns.groups + kSetSlack : w.partial;
@@ -3351,18 +3370,17 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
         const bool sets = use_node_sets(n, G, true) &&
                           ns.stride * ns.groups + kSetSlack <= kAuxRec * N + kAuxRec;
         if (sets) {
-            GSDFT_TRY(launch_pair_box(n, nullptr, w.rec, kRec, w.q, s));
+            GSDFT_TRY(launch_pair_box(n, nullptr, pair_list_order(n) ? w.rec_sorted : w.rec, kRec,
+                                  w.q, s));
             GSDFT_TRY(launch_node_sets(N, G, kSetFold, w.beta, w.kn, aux_centers, dgamma, dgamma_scale,
                                        w.q, w.aux, s));
         } else {
-            k_aux_bwd_prep<<<blocks_for(N, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers,
+            k_aux_bwd_prep<<<blocks_for(N * kNodes, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers,
                                                               dgamma, dgamma_scale, kAuxFoldU,
                                                               coulomb_table(), w.aux);
             GSDFT_HIP(hipGetLastError());
         }
-        GSDFT_TRY(launch_pair_order(n, w.rec, kRec, w.pair_order, s));
-        k_rec_gather<<<blocks_for(n * kRec, 256), 256, 0, s>>>(n, w.pair_order.perm, w.rec,
-                                                                w.rec_sorted);
+        GSDFT_TRY(sort_records(n, w, s));
         // the slabs of groups that hold bwd_split_records' records: never more slabs than those
         Split sp = bwd_split_records(N, n);
         if (sets) {
@@ -3391,7 +3409,7 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
         }
         profile_end(kProfGammaBwd, s);
         k_pair_finalize<<<blocks_for(n, 256), 256, 0, s>>>(n, n, 1, kPref3c,
-                                                           w.pair_order.perm, pi, pj, weight,
+                                                           slot_perm(n, w), pi, pj, weight,
                                                            w.A6, centers, w.Nrm, w.rec_sorted,
                                                            w.acc, J, w.contrib);
         GSDFT_HIP(hipGetLastError());
@@ -3466,9 +3484,7 @@ int external_pass(int64_t M, const double* quat, const double* log_scale, const 
     k_atom_rec<<<blocks_for(n_atoms, 256), 256, 0, s>>>(n_atoms, atom_coords, atom_charges,
                                                         w.g.aux);
     GSDFT_HIP(hipGetLastError());
-    GSDFT_TRY(launch_pair_order(n, w.g.rec, kRec, w.g.pair_order, s));
-    k_rec_gather<<<blocks_for(n * kRec, 256), 256, 0, s>>>(n, w.g.pair_order.perm, w.g.rec,
-                                                            w.g.rec_sorted);
+    GSDFT_TRY(sort_records(n, w.g, s));
     const Split sp = bwd_split(n_atoms, n);
     dim3 grid((unsigned)((n + 255) / 256), (unsigned)sp.slabs);
     profile_begin(kProfNucPairs, s);
@@ -3484,7 +3500,7 @@ int external_pass(int64_t M, const double* quat, const double* log_scale, const 
     profile_end(kProfNucPairs, s);
     GSDFT_HIP(hipGetLastError());
     k_pair_finalize<<<blocks_for(n, 256), 256, 0, s>>>(n, n, sp.slabs, kPrefNuc,
-                                                       w.g.pair_order.perm, pi, pj, weight,
+                                                       slot_perm(n, w.g), pi, pj, weight,
                                                        w.g.A6, centers, w.g.Nrm, w.g.rec_sorted,
                                                        w.g.acc, V, w.g.contrib);
     GSDFT_HIP(hipGetLastError());

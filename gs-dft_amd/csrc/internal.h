@@ -141,6 +141,8 @@ struct PairOrderWs {
     size_t sort_bytes;
 };
 int pair_order_layout(Arena& ar, int64_t n, PairOrderWs* w);
+// Whether launch_pair_order leaves a list of n pairs in its own order (perm[slot] = slot).
+bool pair_list_order(int64_t n);
 // With n_live (a device count), only the first *n_live records are real: the rest take the slots
 // after them.
 int launch_pair_order(int64_t n, const double* rec, int rec_stride, const PairOrderWs& w,
