@@ -2245,10 +2245,17 @@ struct Split {
     int64_t per_slab;
 };
 
+// Slabs of aux records for kBwdBlocks workgroups (four rounds of the chip) or, as long as a slab
+// keeps kSlabRecords records, up to four times as many: a workgroup of a long list walks hundreds
+// of records, so a few rounds end unevenly (C20H42, 590 k pairs: step 95.2 ms with 4096 workgroups,
+// 93.1 with 8192, 91.8 with 16384; water octamer 11.48, 11.19, 11.30), while on short slabs each
+// one's 25 moments a pair cost more than that (37 k pairs x 1200 records 1.74, 1.79, 1.84).
+constexpr int64_t kBwdBlocks = 4096, kBwdBlocksMax = 16384, kSlabRecords = 128;
+
 Split bwd_split(int64_t N, int64_t n) {
     const int64_t groups = n > 0 ? (n + 255) / 256 : 1;
-    const int64_t target = 256 * 4 * 4;
-    int64_t slabs = (target + groups - 1) / groups;
+    int64_t slabs = std::max((kBwdBlocks + groups - 1) / groups,
+                             std::min((kBwdBlocksMax + groups - 1) / groups, N / kSlabRecords));
     slabs = slabs < 1 ? 1 : slabs;
     const int64_t max_slabs = (N + 15) / 16;
     if (slabs > max_slabs) slabs = max_slabs < 1 ? 1 : max_slabs;
@@ -2485,11 +2492,13 @@ int exch_tc_layout(Arena& ar, int64_t M, int64_t N, int64_t n, int64_t Pc, bool 
     GSDFT_TRY(pair_order_layout(ar, n, &w->pair_order));
     if (grads) {
         // bwd_split(W, m).slabs x n (the moments' slot stride is n) over every chunk width
-        // W <= Pc and slab estimate m >= n / 2: at most (4096 / ceil(m / 256) + 1) n <=
-        // 2 x 4096 x 256 + n + 512, and at most the slab cap x n
+        // W <= Pc and slab estimate m >= n / 2: at most (B / ceil(m / 256) + 1) n <= 2 x B x 256 +
+        // n + 512 for B workgroups, and at most the slab cap x n
         int64_t cap = std::min<int64_t>((Pc + 15) / 16, 65535);
         if (cap < 1) cap = 1;
-        const int64_t bound = std::min<int64_t>(cap * n, 2 * 4096 * 256 + n + 512);
+        const int64_t bound =
+            std::max(std::min<int64_t>(cap * n, 2 * kBwdBlocks * 256 + n + 512),
+                     std::min<int64_t>(Pc / kSlabRecords * n, 2 * kBwdBlocksMax * 256 + n + 512));
         w->part = ar.take<double>(kAcc * bound + 1);
         w->acc = ar.take<double>(kAcc * n + 1);
         w->J = ar.take<double>(n + 1);
