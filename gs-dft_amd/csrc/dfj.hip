@@ -931,31 +931,19 @@ __global__ void k_aux_bwd_prep(int64_t N, int64_t G, const double* __restrict__ 
 // of ut[e * ldu + p] (the exchange's dE/d(P|a) per entry, rows in key order), added in order; with
 // ugroup the group's entries share one cotangent row, ut[g * ldu + p], and u = x[3] * (that row
 // times the entry count uptr[g + 1] - uptr[g]).
-// With kAtomF the records are nuclei (point charges) and the pass also forms every nucleus' force
-// from the same node sums: per (nucleus p, pair a) the vector 2 KN_a q_a (f0 d + f1 Ah d + f2 Ah^2 d),
-// f0 = -I3 sum g s, f1 = -(I1 sum g s^2 + sum g s^3), f2 = sum g s^2 (dF/dR of
-// gs_dft/ks/forces.py:53-77 through pairs.py:348-370), summed over the wave (wave_sum3), then over
-// the four waves in LDS per chunk of 64 nuclei, into atom_part[pair block][p][3] (times -Z_p 2 pi
-// later).
-constexpr int kAtomChunk = 64;
-
-// The nuclear-force form (kAtomF) is held to four waves per SIMD (128 registers, a 20-byte spill
-// outside the node loop): 1.6% faster than the three its 134 registers allowed. The other forms
-// keep their allocation (for kLaneU four waves cost a 32-byte spill and 2.6%); kSet with
-// its two nodes a step fits four waves (12 bytes spilled outside the node loop; equal to three).
-template <bool kLaneU, bool kAtomF = false, bool kFold = false, int kN = kNodes, bool kSet = false>
-__global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kAtomF || kSet ? 4 : 1) void k_gamma_bwd(
+// The kernel keeps its allocation (for kLaneU four waves per SIMD cost a 32-byte spill and 2.6%);
+// kSet with its two nodes a step fits four (12 bytes spilled outside the node loop; equal to three).
+template <bool kLaneU, bool kFold = false, int kN = kNodes, bool kSet = false>
+__global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kSet ? 4 : 1) void k_gamma_bwd(
     int64_t n, const double* __restrict__ rec, int64_t N, const double* __restrict__ aux,
     int64_t per_slab, double* __restrict__ partial, unsigned long long* __restrict__ work,
-    const double* __restrict__ ut, int64_t ldu, double* __restrict__ atom_part,
-    const int32_t* __restrict__ uperm, const int32_t* __restrict__ uptr,
+    const double* __restrict__ ut, int64_t ldu, const int32_t* __restrict__ uperm, const int32_t* __restrict__ uptr,
     const int64_t* __restrict__ n_live, int ugroup = 0, int64_t slab0 = 0, int acc_first = -1,
     int64_t set_stride = 0) {
-    static_assert(!kSet || (kFold && !kAtomF), "");
+    static_assert(!kSet || kFold, "");
     // whole workgroups past the real slots leave at once (workgroup-uniform, before any barrier)
     if (n_live && (int64_t)blockIdx.x * blockDim.x >= *n_live) return;
     __shared__ double tab[256];
-    __shared__ double af[kAtomF ? 4 : 1][kAtomF ? kAtomChunk : 1][3];
     // Each lane's Ah (6) and centre (3), read again at every new aux centre: held in LDS (one
     // slot per lane, structure of arrays) rather than in registers across the loop.
     __shared__ double geo[9][256];
@@ -975,8 +963,6 @@ __global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kAtomF || kSet ? 4 : 1) v
     double Sa[6] = {0, 0, 0, 0, 0, 0}, Sb[6] = {0, 0, 0, 0, 0, 0};
     double C0 = 0, C1 = 0, C2 = 0;
     double d[3] = {0, 0, 0}, q0 = 0, q1 = 0, X0 = 0, rr = 0;
-    double ad[3] = {0, 0, 0}, a2d[3] = {0, 0, 0};      // Ah d, Ah^2 d (kAtomF)
-    const double cq2 = kAtomF && live ? 2.0 * r[13] * r[14] : 0.0;
     int64_t ut0 = 0;                     // kLaneU: the lane's cotangent rows [ut0, ut0 + utn)
     int utn = 0;
     double uscale = 1.0;                 // kLaneU with ugroup: the group's entry count
@@ -996,7 +982,6 @@ __global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kAtomF || kSet ? 4 : 1) v
         }
     }
     const int64_t slab = slab0 + blockIdx.y;       // aux slab of this workgroup
-    int64_t chunk0 = slab * per_slab;
     double F = 0, dP0 = 0, dP1 = 0, dP2 = 0, gs1 = 0, gs2 = 0, gs3 = 0;      // node sums
     auto flush = [&]() {
         if constexpr (kFold) {           // the node sums span the centre's records, u folded in
@@ -1046,12 +1031,6 @@ __global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kAtomF || kSet ? 4 : 1) v
         const double q2 = __builtin_fma(ax, ax, __builtin_fma(ay, ay, az * az));
         X0 = I3 * q0;
         rr = __builtin_fma(I1, q1, -q2);
-        if constexpr (kAtomF) {
-            ad[0] = ax; ad[1] = ay; ad[2] = az;
-            a2d[0] = __builtin_fma(xx, ax, __builtin_fma(xy, ay, xz * az));
-            a2d[1] = __builtin_fma(xy, ax, __builtin_fma(yy, ay, yz * az));
-            a2d[2] = __builtin_fma(xz, ax, __builtin_fma(yz, ay, zz * az));
-        }
     };
     // one node's terms added to the node sums; returns z - 1/2
     auto add_node = [&](double st, double wh, double s2, double is) {
@@ -1224,25 +1203,6 @@ __global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kAtomF || kSet ? 4 : 1) v
         C0 = __builtin_fma(u, -gs1, C0);
         C1 = __builtin_fma(u, -gs2, C1);
         C2 = __builtin_fma(u, -gs3, C2);
-        if constexpr (kAtomF) {
-            const double f0 = -I3 * gs1, f1 = -__builtin_fma(I1, gs2, gs3), f2 = gs2;
-            double fv[3];
-#pragma unroll
-            for (int c = 0; c < 3; ++c)
-                fv[c] = cq2 * __builtin_fma(f0, d[c], __builtin_fma(f1, ad[c], f2 * a2d[c]));
-            int comp;
-            const double tot = wave_sum3(fv, &comp);
-            if (comp >= 0) af[threadIdx.x >> 6][p - chunk0][comp] = tot;
-            if (p - chunk0 == kAtomChunk - 1 || p == p1 - 1) {     // workgroup-uniform
-                __syncthreads();
-                const int i = threadIdx.x / 3, c = threadIdx.x % 3;
-                if (threadIdx.x < 3 * kAtomChunk && chunk0 + i <= p)
-                    atom_part[((int64_t)blockIdx.x * N + chunk0 + i) * 3 + c] =
-                        ((af[0][i][c] + af[1][i][c]) + af[2][i][c]) + af[3][i][c];
-                __syncthreads();
-                chunk0 = p + 1;
-            }
-        }
     }
     flush();
     count_work(work, live, nodes);
@@ -1531,23 +1491,184 @@ __global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunk
 // (2/sqrt(pi)) pi^1.5 = 2 pi.
 constexpr double kPrefNuc = 2.0 * kPi;
 
+// The nuclei as k_nuclear_pairs reads them, in the aux records' place: the nodes' s = t^2, 1/s, s^2
+// and weight w_t s^(-1/2) / K, then R (3) and -Z of each nucleus.
+constexpr int kNucNodes = 4 * kNodes;
+constexpr int kAtomRec = 4;
+constexpr int kAtomChunk = 64;          // nuclei between two sums of the forces over the workgroup
 __global__ void k_atom_rec(int64_t n_atoms, const double* __restrict__ coords,
                            const double* __restrict__ charges, double* __restrict__ out) {
     const int64_t A = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (A >= n_atoms) return;
-    double* o = out + kAuxRec * A;
-    o[0] = coords[3 * A]; o[1] = coords[3 * A + 1]; o[2] = coords[3 * A + 2];
-    o[3] = -charges[A];
-    bool first = true;
-    if (A > 0)
-        first = !(__builtin_bit_cast(uint64_t, coords[3 * A - 3]) ==
-                      __builtin_bit_cast(uint64_t, coords[3 * A]) &&
-                  __builtin_bit_cast(uint64_t, coords[3 * A - 2]) ==
-                      __builtin_bit_cast(uint64_t, coords[3 * A + 1]) &&
-                  __builtin_bit_cast(uint64_t, coords[3 * A - 1]) ==
-                      __builtin_bit_cast(uint64_t, coords[3 * A + 2]));
-    o[4] = 0.0; o[5] = first ? 1.0 : 0.0; o[6] = 0.0; o[7] = 0.0;
-    for (int t = 0; t < kNodes; ++t) put_node_consts(o, t, quad_t(t) * quad_t(t), quad_w(t));
+    if (A < n_atoms) {
+        double* o = out + kNucNodes + kAtomRec * A;
+        o[0] = coords[3 * A]; o[1] = coords[3 * A + 1]; o[2] = coords[3 * A + 2];
+        o[3] = -charges[A];
+    }
+    if (A < kNodes) {
+        const double t = quad_t((int)A), s = t * t;
+        double* o = out + 4 * A;
+        o[0] = s;
+        o[1] = 1.0 / s;
+        o[2] = s * s;
+        o[3] = quad_w((int)A) / t / kExpPolyK;
+    }
+}
+
+// The pair pass of the nuclear attraction: k_gamma_bwd's sums (jt, T1..T3, the d-moments) over a
+// slab of nuclei with u = -Z, and with kForce every nucleus' force. A nucleus is a point, so its
+// nodes are s_t = t^2 for all of them and the pair's determinants Pr_t = I3/s + I2 + s I1 + s^2 (the
+// scaled Pn of node_val_h) do not depend on it: a lane forms 1/Pr_t and wh Pr_t^(-3/2) once for its
+// pair, to full precision, and keeps them in registers through the slab. A node is then z = Qn/Pr,
+// G = wh Pr^(-3/2) e^-z and seven sums,
+//   gm, g1..g3 = sum G (1/s, 1, s, s^2),   h0..h2 = sum G z (1/s, 1, s),
+// without the determinant, the root and its corrections; F = sum G Pr = I3 gm + I2 g1 + I1 g2 + g3,
+// all terms positive, and dPk = h_k - 1/2 (gm, g1, g2) close them once per nucleus.
+// Bound by its VALU instructions, ~24 a node against ~34 and a quarter-rate root where each nucleus
+// formed its own. The table's eighty registers leave two waves per SIMD, which its independent sums
+// fill: held to three (a forty-register table, 1/Pr formed from Pr^(-1/2)) the kernel spills and is
+// 1 to 8% slower. 300 atoms, 10.3 M pairs: 44.5 -> 37.6 ms (the step 70.9 -> 64.0); 60 atoms, 560 k
+// pairs: the step 3.7 -> 3.0 ms.
+template <bool kForce>
+__global__ __launch_bounds__(256, 2) void k_nuclear_pairs(
+    int64_t n, const double* __restrict__ rec, int64_t n_atoms, const double* __restrict__ atoms,
+    int64_t per_slab, double* __restrict__ partial, unsigned long long* __restrict__ work,
+    double* __restrict__ atom_part) {
+    __shared__ double tab[256];
+    __shared__ double af[kForce ? 4 : 1][kForce ? kAtomChunk : 1][3];
+    __shared__ double geo[9][256];         // each lane's Ah and centre, read again at every nucleus
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) tab[i] = exp2_frac_lead(i);
+    const int l = threadIdx.x;
+    const int64_t a = blockIdx.x * (int64_t)blockDim.x + l;
+    const bool live = a < n;
+    const double* r = rec + kRec * (live ? a : 0);
+    const double I1 = r[0], I2 = r[1], I3 = r[2];
+#pragma unroll
+    for (int c = 0; c < 6; ++c) geo[c][l] = r[3 + c];
+    geo[6][l] = live ? r[9] : kFarAway;
+    geo[7][l] = live ? r[10] : kFarAway;
+    geo[8][l] = live ? r[11] : kFarAway;
+    const double cq2 = kForce && live ? 2.0 * r[13] * r[14] : 0.0;
+    __syncthreads();
+    UniformPtr nodes = uniform_ptr(atoms);
+    double ip[kNodes], c3[kNodes];         // 1/Pr_t and wh_t Pr_t^(-3/2)
+#pragma unroll
+    for (int t = 0; t < kNodes; ++t) {
+        const double s = nodes[4 * t], is = nodes[4 * t + 1];
+        const double P = __builtin_fma(is, I3, __builtin_fma(s, I1 + s, I2));
+        // y0 (1 + e/2 + 3 e^2/8), e = 1 - P y0^2 below 1.1e-7
+        const double y0 = __builtin_amdgcn_rsq(P);
+        const double e = __builtin_fma(-P * y0, y0, 1.0);
+        const double y = __builtin_fma(y0 * e, __builtin_fma(e, 0.375, 0.5), y0);
+        ip[t] = y * y;
+        c3[t] = nodes[4 * t + 3] * (y * ip[t]);
+    }
+    double jt = 0, T1 = 0, T2 = 0, T3 = 0;
+    double Vc[3] = {0, 0, 0}, Va[3] = {0, 0, 0}, Vb[3] = {0, 0, 0};
+    double Sa[6] = {0, 0, 0, 0, 0, 0}, Sb[6] = {0, 0, 0, 0, 0, 0};
+    const int64_t p0 = blockIdx.y * per_slab;
+    const int64_t p1 = min(n_atoms, p0 + per_slab);
+    int64_t chunk0 = p0;
+    uint32_t count = 0;
+    for (int64_t p = p0; p < p1; ++p) {
+        UniformPtr x = uniform_ptr(atoms + kNucNodes + kAtomRec * p);
+        const double u = x[3];
+        const double dx = x[0] - geo[6][l], dy = x[1] - geo[7][l], dz = x[2] - geo[8][l];
+        const double xx = geo[0][l], yy = geo[1][l], zz = geo[2][l], xy = geo[3][l],
+                     xz = geo[4][l], yz = geo[5][l];
+        const double ax = __builtin_fma(xx, dx, __builtin_fma(xy, dy, xz * dz));
+        const double ay = __builtin_fma(xy, dx, __builtin_fma(yy, dy, yz * dz));
+        const double az = __builtin_fma(xz, dx, __builtin_fma(yz, dy, zz * dz));
+        const double q0 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+        const double q1 = __builtin_fma(dx, ax, __builtin_fma(dy, ay, dz * az));
+        const double q2 = __builtin_fma(ax, ax, __builtin_fma(ay, ay, az * az));
+        const double X0 = I3 * q0;
+        const double rr = __builtin_fma(I1, q1, -q2);
+        double gm = 0, g1 = 0, g2 = 0, g3 = 0, h0 = 0, h1 = 0, h2 = 0;
+        double n_s = nodes[0], n_is = nodes[1], n_s2 = nodes[2];
+        auto node = [&](auto tc) {
+            constexpr int t = decltype(tc)::value;
+            const double s = n_s, is = n_is, s2 = n_s2;
+            if constexpr (t + 1 < kNodes) {
+                n_s = nodes[4 * t + 4];
+                n_is = nodes[4 * t + 5];
+                n_s2 = nodes[4 * t + 6];
+            }
+            const double z = __builtin_fma(s, __builtin_fma(s, q1, rr), X0) * ip[t];
+            const double G = c3[t] * exp_neg_tab_k(z, tab);
+            const double Gz = G * z;
+            gm = __builtin_fma(G, is, gm);
+            g1 += G;
+            g2 = __builtin_fma(G, s, g2);
+            g3 = __builtin_fma(G, s2, g3);
+            h0 = __builtin_fma(Gz, is, h0);
+            h1 += Gz;
+            h2 = __builtin_fma(Gz, s, h2);
+            if constexpr (t + 1 < kNodes)
+                asm volatile("" ::"s"(n_s), "s"(n_is), "s"(n_s2));
+            return screen_after(t) && __builtin_amdgcn_ballot_w64(!(z > kSkipZ)) == 0;
+        };
+        count += node_loop<0>(node);
+        const double F = __builtin_fma(I3, gm, __builtin_fma(I2, g1, __builtin_fma(I1, g2, g3)));
+        const double dP0 = __builtin_fma(gm, -0.5, h0), dP1 = __builtin_fma(g1, -0.5, h1),
+                     dP2 = __builtin_fma(g2, -0.5, h2);
+        jt = __builtin_fma(u, (q0 == q0) ? F : q0, jt);          // a NaN centre propagates
+        T3 = __builtin_fma(u, __builtin_fma(q0, -g1, dP0), T3);
+        T2 = __builtin_fma(u, dP1, T2);
+        T1 = __builtin_fma(u, __builtin_fma(q1, -g2, dP2), T1);
+        const double C0 = -u * g1, C1 = -u * g2, C2 = -u * g3;
+        const double e1x = C1 * dx, e1y = C1 * dy, e1z = C1 * dz;
+        const double e2x = C2 * dx, e2y = C2 * dy, e2z = C2 * dz;
+        Vc[0] = __builtin_fma(C0, dx, Vc[0]);
+        Vc[1] = __builtin_fma(C0, dy, Vc[1]);
+        Vc[2] = __builtin_fma(C0, dz, Vc[2]);
+        Va[0] += e1x; Va[1] += e1y; Va[2] += e1z;
+        Vb[0] += e2x; Vb[1] += e2y; Vb[2] += e2z;
+        Sa[0] = __builtin_fma(e1x, dx, Sa[0]);
+        Sa[1] = __builtin_fma(e1y, dy, Sa[1]);
+        Sa[2] = __builtin_fma(e1z, dz, Sa[2]);
+        Sa[3] = __builtin_fma(e1x, dy, Sa[3]);
+        Sa[4] = __builtin_fma(e1x, dz, Sa[4]);
+        Sa[5] = __builtin_fma(e1y, dz, Sa[5]);
+        Sb[0] = __builtin_fma(e2x, dx, Sb[0]);
+        Sb[1] = __builtin_fma(e2y, dy, Sb[1]);
+        Sb[2] = __builtin_fma(e2z, dz, Sb[2]);
+        Sb[3] = __builtin_fma(e2x, dy, Sb[3]);
+        Sb[4] = __builtin_fma(e2x, dz, Sb[4]);
+        Sb[5] = __builtin_fma(e2y, dz, Sb[5]);
+        if constexpr (kForce) {
+            // per (nucleus, pair) the vector 2 KN_a q_a (f0 d + f1 Ah d + f2 Ah^2 d), f0 = -I3 sum g s,
+            // f1 = -(I1 sum g s^2 + sum g s^3), f2 = sum g s^2 (dF/dR of gs_dft/ks/forces.py:53-77
+            // through pairs.py:348-370), summed over the wave, then over the four waves in LDS per
+            // chunk of nuclei, into atom_part[pair block][nucleus][3] (times -Z 2 pi later)
+            const double f0 = -I3 * g1, f1 = -__builtin_fma(I1, g2, g3), f2 = g2;
+            const double bx = __builtin_fma(xx, ax, __builtin_fma(xy, ay, xz * az));
+            const double by = __builtin_fma(xy, ax, __builtin_fma(yy, ay, yz * az));
+            const double bz = __builtin_fma(xz, ax, __builtin_fma(yz, ay, zz * az));
+            const double fv[3] = {cq2 * __builtin_fma(f0, dx, __builtin_fma(f1, ax, f2 * bx)),
+                                  cq2 * __builtin_fma(f0, dy, __builtin_fma(f1, ay, f2 * by)),
+                                  cq2 * __builtin_fma(f0, dz, __builtin_fma(f1, az, f2 * bz))};
+            int comp;
+            const double tot = wave_sum3(fv, &comp);
+            if (comp >= 0) af[l >> 6][p - chunk0][comp] = tot;
+            if (p - chunk0 == kAtomChunk - 1 || p == p1 - 1) {     // workgroup-uniform
+                __syncthreads();
+                const int i = l / 3, c = l % 3;
+                if (l < 3 * kAtomChunk && chunk0 + i <= p)
+                    atom_part[((int64_t)blockIdx.x * n_atoms + chunk0 + i) * 3 + c] =
+                        ((af[0][i][c] + af[1][i][c]) + af[2][i][c]) + af[3][i][c];
+                __syncthreads();
+                chunk0 = p + 1;
+            }
+        }
+    }
+    count_work(work, live, count);
+    if (!live) return;
+    double* o = partial + (int64_t)blockIdx.y * kAcc * n + a;
+    const double v[kAcc] = {jt, T1, T2, T3, Vc[0], Vc[1], Vc[2], Va[0], Va[1], Va[2],
+                            Vb[0], Vb[1], Vb[2], Sa[0], Sa[1], Sa[2], Sa[3], Sa[4], Sa[5],
+                            Sb[0], Sb[1], Sb[2], Sb[3], Sb[4], Sb[5]};
+#pragma unroll
+    for (int c = 0; c < kAcc; ++c) o[(int64_t)c * n] = v[c];
 }
 
 // ------------------------------------------------------------------ exact pair-pair Coulomb
@@ -2613,21 +2734,21 @@ int exch_tc_reverse(int64_t N, int64_t q0, int64_t W, int64_t n, int64_t n_est,
     profile_begin(kProfExchBwd, s);
     if (exch_shares(w)) {
         const int64_t stride = node_sets(N, kMaxSetScales, kSetExchange).stride;
-        k_gamma_bwd<true, false, true, kNodes, true><<<grid, 256, 0, s>>>(
+        k_gamma_bwd<true, true, kNodes, true><<<grid, 256, 0, s>>>(
             n, w.rec_sorted, W / kMaxSetScales, w.sets + stride * (q0 / kMaxSetScales),
-            sp.per_slab, w.part, profile_work_counter(kProfExchBwd), Tbar, ldt, nullptr,
+            sp.per_slab, w.part, profile_work_counter(kProfExchBwd), Tbar, ldt,
             w.pair_order.perm, w.grp_first, w.n_groups_dev, group_rows ? 1 : 0, 0, -1, stride);
     } else if (w.table.n == kLrNodes)
-        k_gamma_bwd<true, false, false, kLrNodes><<<grid, 256, 0, s>>>(
+        k_gamma_bwd<true, false, kLrNodes><<<grid, 256, 0, s>>>(
             n, w.rec_sorted, W, w.aux + kAuxRec * q0, sp.per_slab, w.part,
-            profile_work_counter(kProfExchBwd), Tbar, ldt, nullptr, w.pair_order.perm,
+            profile_work_counter(kProfExchBwd), Tbar, ldt, w.pair_order.perm,
             w.grp_first, w.n_groups_dev, group_rows ? 1 : 0);
     else
         k_gamma_bwd<true><<<grid, 256, 0, s>>>(n, w.rec_sorted, W, w.aux + kAuxRec * q0,
                                                sp.per_slab, w.part,
                                                profile_work_counter(kProfExchBwd), Tbar, ldt,
-                                               nullptr, w.pair_order.perm, w.grp_first,
-                                               w.n_groups_dev, group_rows ? 1 : 0);
+                                               w.pair_order.perm, w.grp_first, w.n_groups_dev,
+                                               group_rows ? 1 : 0);
     profile_end(kProfExchBwd, s);
     GSDFT_HIP(hipGetLastError());
     k_acc_fold<<<blocks_for(n * kAcc, 256), 256, 0, s>>>(n, sp.slabs, w.part, w.acc, first ? 1 : 0);
@@ -3403,13 +3524,13 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
             dim3 grid((unsigned)((n + 255) / 256), (unsigned)r);
             unsigned long long* work = profile_work_counter(kProfGammaBwd);
             if (sets)
-                k_gamma_bwd<false, false, true, kNodes, true><<<grid, 256, 0, s>>>(
+                k_gamma_bwd<false, true, kNodes, true><<<grid, 256, 0, s>>>(
                     n, w.rec_sorted, ns.groups, w.aux, sp.per_slab, w.acc, work, nullptr, 0,
-                    nullptr, nullptr, nullptr, nullptr, 0, sl, sl == 0 ? 1 : 0, ns.stride);
+                    nullptr, nullptr, nullptr, 0, sl, sl == 0 ? 1 : 0, ns.stride);
             else
-                k_gamma_bwd<false, false, true><<<grid, 256, 0, s>>>(
+                k_gamma_bwd<false, true><<<grid, 256, 0, s>>>(
                     n, w.rec_sorted, N, w.aux, sp.per_slab, w.acc, work, nullptr, 0, nullptr,
-                    nullptr, nullptr, nullptr, 0, sl, sl == 0 ? 1 : 0);
+                    nullptr, nullptr, 0, sl, sl == 0 ? 1 : 0);
             GSDFT_HIP(hipGetLastError());
             if (r > 1) {
                 k_slab_fold<<<blocks_for(n * kAcc, 256), 256, 0, s>>>(n, r, w.acc);
@@ -3481,8 +3602,7 @@ __global__ void k_atom_force_finish(int64_t n_atoms, int64_t groups,
     datoms[i] = -charges[i / 3] * kPrefNuc * s;
 }
 
-// V (n) = the nuclear attraction of every listed pair (J of the reverse kernel with the nuclei as
-// point-charge records) and, for a non-null C, the slot moments behind its gradient.
+// V (n) = the nuclear attraction of every listed pair (jt of k_nuclear_pairs) and, for a non-null C, the slot moments behind its gradient.
 int external_pass(int64_t M, const double* quat, const double* log_scale, const double* centers,
                   int64_t k, const double* C, const double* occ, int64_t n, const int32_t* pi,
                   const int32_t* pj, const double* weight, int64_t n_atoms,
@@ -3498,14 +3618,14 @@ int external_pass(int64_t M, const double* quat, const double* log_scale, const 
     dim3 grid((unsigned)((n + 255) / 256), (unsigned)sp.slabs);
     profile_begin(kProfNucPairs, s);
     if (atom_forces)
-        k_gamma_bwd<false, true><<<grid, 256, 0, s>>>(n, w.g.rec_sorted, n_atoms, w.g.aux,
-                                                      sp.per_slab, w.g.acc,
-                                                      profile_work_counter(kProfNucPairs),
-                                                      nullptr, 0, w.atom_partial, nullptr, nullptr, nullptr);
+        k_nuclear_pairs<true><<<grid, 256, 0, s>>>(n, w.g.rec_sorted, n_atoms, w.g.aux,
+                                                   sp.per_slab, w.g.acc,
+                                                   profile_work_counter(kProfNucPairs),
+                                                   w.atom_partial);
     else
-        k_gamma_bwd<false><<<grid, 256, 0, s>>>(n, w.g.rec_sorted, n_atoms, w.g.aux, sp.per_slab,
-                                                w.g.acc, profile_work_counter(kProfNucPairs),
-                                                nullptr, 0, nullptr, nullptr, nullptr, nullptr);
+        k_nuclear_pairs<false><<<grid, 256, 0, s>>>(n, w.g.rec_sorted, n_atoms, w.g.aux,
+                                                    sp.per_slab, w.g.acc,
+                                                    profile_work_counter(kProfNucPairs), nullptr);
     profile_end(kProfNucPairs, s);
     GSDFT_HIP(hipGetLastError());
     k_pair_finalize<<<blocks_for(n, 256), 256, 0, s>>>(n, n, sp.slabs, kPrefNuc,
