@@ -371,7 +371,8 @@ struct DmaOperand {
     }
 };
 
-template <bool kAK, bool kBK>
+// MS: 16-row m sub-tiles per wave, so a workgroup's tile has 32 MS rows of C (kTile for 4).
+template <bool kAK, bool kBK, int MS>
 __device__ __forceinline__ void gemm_tile_dma_gen(int64_t m0, int64_t n0, int64_t Mr, int64_t Nc,
                                                   int64_t K, const double* __restrict__ A,
                                                   int64_t lda, const double* __restrict__ B,
@@ -391,22 +392,22 @@ __device__ __forceinline__ void gemm_tile_dma_gen(int64_t m0, int64_t n0, int64_
         *lb = *la + kOpMax;
     };
 
-    v4d acc[4][4];
+    v4d acc[4][MS];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
+        for (int j = 0; j < MS; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
 
     // the sub-steps [0, ksub) of one staged K step; operands of sub-step kk + 4 read during the
     // sixteen MFMAs of sub-step kk
     auto compute = [&](const double* __restrict__ la, const double* __restrict__ lb, int ksub) {
-        double bn[2][4], am[2][4];
+        double bn[2][4], am[2][MS];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             bn[0][i] = lb[DmaOperand<kBK>::at(wn * 64 + i * 16 + l16, l4)];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            am[0][j] = la[DmaOperand<kAK>::at(wm * 64 + j * 16 + l16, l4)];
+        for (int j = 0; j < MS; ++j)
+            am[0][j] = la[DmaOperand<kAK>::at(wm * 16 * MS + j * 16 + l16, l4)];
 #pragma unroll
         for (int kk = 0; kk < kStepK; kk += 4) {
             if (kk >= ksub) break;
@@ -416,13 +417,13 @@ __device__ __forceinline__ void gemm_tile_dma_gen(int64_t m0, int64_t n0, int64_
                 for (int i = 0; i < 4; ++i)
                     bn[nxt][i] = lb[DmaOperand<kBK>::at(wn * 64 + i * 16 + l16, kk + 4 + l4)];
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    am[nxt][j] = la[DmaOperand<kAK>::at(wm * 64 + j * 16 + l16, kk + 4 + l4)];
+                for (int j = 0; j < MS; ++j)
+                    am[nxt][j] = la[DmaOperand<kAK>::at(wm * 16 * MS + j * 16 + l16, kk + 4 + l4)];
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = mfma(bn[cur][i], am[cur][j], acc[i][j]);
+                for (int j = 0; j < MS; ++j) acc[i][j] = mfma(bn[cur][i], am[cur][j], acc[i][j]);
         }
     };
 
@@ -457,7 +458,7 @@ __device__ __forceinline__ void gemm_tile_dma_gen(int64_t m0, int64_t n0, int64_
         __syncthreads();
         compute(la, lb, (int)(K - K0));
     }
-    const bool edge = m0 + kTile > Mr || n0 + kTile > Nc;       // workgroup-uniform
+    const bool edge = m0 + 32 * MS > Mr || n0 + kTile > Nc;       // workgroup-uniform
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -466,8 +467,8 @@ __device__ __forceinline__ void gemm_tile_dma_gen(int64_t m0, int64_t n0, int64_
             if (edge && n >= Nc) continue;
             double* col = C + n * ldc;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int64_t m = m0 + wm * 64 + 16 * j + l16;
+            for (int j = 0; j < MS; ++j) {
+                const int64_t m = m0 + wm * 16 * MS + 16 * j + l16;
                 if (!edge || m < Mr) epilogue(col + m, acc[i][j][r], alpha, beta);
             }
         }
@@ -485,7 +486,7 @@ struct Batch {
     double alpha, beta;
 };
 
-template <int kMode, bool kAK = true, bool kBK = true>
+template <int kMode, bool kAK = true, bool kBK = true, int MS = 4>
 __global__ __launch_bounds__(kThreads, 2) void k_gemm_tn_sub(int64_t Mr, int64_t Nc, int64_t K,
                                                              const double* __restrict__ A,
                                                              int64_t lda,
@@ -503,7 +504,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_tn_sub(int64_t Mr, int64_t
         gemm_tile_dma(tm * kTile, tn * kTile, K, A, lda, B, ldb, C, ldc, lds);
     } else if constexpr (kMode == kDmaGen) {
         __shared__ __align__(16) double lds[2 * 2 * kOpMax];
-        gemm_tile_dma_gen<kAK, kBK>(tm * kTile, tn * kTile, Mr, Nc, K, A, lda, B, ldb, C, ldc,
+        gemm_tile_dma_gen<kAK, kBK, MS>(tm * 32 * MS, tn * kTile, Mr, Nc, K, A, lda, B, ldb, C, ldc,
                                     lds, bt.alpha, bt.beta);
     } else {
         __shared__ double As[2][kTile][kLdsK];
@@ -513,16 +514,36 @@ __global__ __launch_bounds__(kThreads, 2) void k_gemm_tn_sub(int64_t Mr, int64_t
     }
 }
 
-template <int kMode, bool kAK = true, bool kBK = true>
+template <int kMode, bool kAK = true, bool kBK = true, int MS = 4>
 int launch_tiles(int64_t Mr, int64_t Nc, int64_t K, const double* A, int64_t lda,
                  const double* B, int64_t ldb, double* C, int64_t ldc, TileSet ts, int64_t blocks,
                  hipStream_t s, Batch bt = Batch{0, 0, 0, -1.0, 1.0}, int64_t batch = 1) {
     if (blocks <= 0 || batch <= 0) return GSDFT_OK;
     if (blocks > INT32_MAX || batch > 65535) return fail(GSDFT_ERR_ARG, "gemm: too many tiles");
-    k_gemm_tn_sub<kMode, kAK, kBK><<<dim3((unsigned)blocks, (unsigned)batch), kThreads, 0, s>>>(
+    k_gemm_tn_sub<kMode, kAK, kBK, MS><<<dim3((unsigned)blocks, (unsigned)batch), kThreads, 0, s>>>(
         Mr, Nc, K, A, lda, B, ldb, C, ldc, ts, bt);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
+}
+
+// Rows of a DMA tile in units of 32: the orbital count is often the row count of a product (81 at
+// C20H42), and a 128-row tile then multiplies rows that are not there. Up to 256 rows the tile is
+// the one that pads least, the larger of equals; beyond that what 128 rows pad is below a third and
+// wider tiles read less. Grid step of C20H42 (81 orbitals: 96 rows in place of 128) 10.58 -> 9.60 ms,
+// of 700 splats with 30 orbitals 1.30 -> 0.94 ms, of 2600 with 150 (two tiles of 96) 15.2 -> 12.1;
+// RI-K of C20H42: the k-row products 20.8 -> 18.1 ms.
+inline int dma_row_tiles(int64_t Mr) {
+    if (Mr > 2 * kTile) return 4;
+    int best = 4;
+    int64_t pad = (Mr + 127) / 128 * 128;
+    for (int ms = 3; ms >= 1; --ms) {
+        const int64_t p = (Mr + 32 * ms - 1) / (32 * ms) * (32 * ms);
+        if (p < pad) {
+            best = ms;
+            pad = p;
+        }
+    }
+    return best;
 }
 
 // Every tile of an Mr x Nc product: the interior ones on the fast path for the layouts (DMA when
@@ -537,10 +558,21 @@ int launch_all_tiles(int64_t Mr, int64_t Nc, int64_t K, const double* A, int64_t
     const bool dma = lda % 2 == 0 && ldb % 2 == 0 && bt.sa % 2 == 0 && bt.sb % 2 == 0 &&
                      reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                      reinterpret_cast<uintptr_t>(B) % 16 == 0;
-    if (dma)                                   // every tile, the edge ones included
-        return launch_tiles<kDmaGen, kAK, kBK>(Mr, Nc, K, A, lda, B, ldb, C, ldc,
-                                               TileSet{0, 0, tiles_m, 0}, tiles_m * tiles_n, s,
-                                               bt, batch);
+    if (dma) {                                 // every tile, the edge ones included
+        auto rows = [&](auto ms) {
+            constexpr int MS = decltype(ms)::value;
+            const int64_t tm = (Mr + 32 * MS - 1) / (32 * MS);
+            return launch_tiles<kDmaGen, kAK, kBK, MS>(Mr, Nc, K, A, lda, B, ldb, C, ldc,
+                                                       TileSet{0, 0, tm, 0}, tm * tiles_n, s, bt,
+                                                       batch);
+        };
+        switch (dma_row_tiles(Mr)) {
+            case 1: return rows(std::integral_constant<int, 1>{});
+            case 2: return rows(std::integral_constant<int, 2>{});
+            case 3: return rows(std::integral_constant<int, 3>{});
+            default: return rows(std::integral_constant<int, 4>{});
+        }
+    }
     if (K % kStepK == 0)
         GSDFT_TRY((launch_tiles<kPlain, kAK, kBK>(Mr, Nc, K, A, lda, B, ldb, C, ldc,
                                                  TileSet{0, 0, fm, 0}, fm * fn, s, bt, batch)));
