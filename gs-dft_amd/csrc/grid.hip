@@ -92,27 +92,56 @@ __global__ void k_grid_scale_occ(int64_t Gc, int64_t k, int64_t ldk,
     out[e] = psi[e] * occ[i % k];
 }
 
-// grad_rd = 2 sum_m phi_rm dg_d,rm, one wave per row (grid.py:104-107).
+// grad_rd = 2 sum_m phi_rm dg_d,rm (grid.py:104-107), one wave per kGradRows rows: dg is formed
+// again from g (bit for bit as k_grid_basis forms it), so the forward neither writes nor reads the
+// three dg blocks, and a splat's chart is read once for the wave's rows. Bound by reading phi and g:
+// 131 MB a chunk of 4096 x 2000 in 24.8 us, against 57.8 us with the dg blocks (which k_grid_basis
+// also took 16 us longer to write).
+constexpr int kGradRows = 4;
 __global__ __launch_bounds__(256) void k_grid_grad_phi(int64_t Gc, int64_t M,
                                                        const double* __restrict__ phi,
-                                                       const double* __restrict__ dg,
+                                                       const double* __restrict__ g,
+                                                       const double* __restrict__ pts,
+                                                       const double* __restrict__ A6,
+                                                       const double* __restrict__ mu,
                                                        double* __restrict__ grad) {
-    const int64_t r = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6;
+    const int64_t r0 = ((blockIdx.x * (int64_t)blockDim.x + threadIdx.x) >> 6) * kGradRows;
     const int lane = threadIdx.x & 63;
-    if (r >= Gc) return;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+    if (r0 >= Gc) return;
+    double s[kGradRows][3], x[kGradRows][3];
+    int64_t row[kGradRows];                  // past the end: the last row again, not stored
+#pragma unroll
+    for (int q = 0; q < kGradRows; ++q) {
+        row[q] = min(r0 + q, Gc - 1);
+        for (int c = 0; c < 3; ++c) {
+            s[q][c] = 0.0;
+            x[q][c] = pts[3 * row[q] + c];
+        }
+    }
     for (int64_t m = lane; m < M; m += 64) {
-        const double f = phi[r * M + m];
-        s0 = __builtin_fma(f, dg[r * M + m], s0);
-        s1 = __builtin_fma(f, dg[(Gc + r) * M + m], s1);
-        s2 = __builtin_fma(f, dg[(2 * Gc + r) * M + m], s2);
+        const double* a = A6 + 6 * m;
+        const double a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3], a4 = a[4], a5 = a[5];
+        const double m0 = mu[3 * m], m1 = mu[3 * m + 1], m2 = mu[3 * m + 2];
+        double f[kGradRows], gv[kGradRows];
+#pragma unroll
+        for (int q = 0; q < kGradRows; ++q) {
+            f[q] = phi[row[q] * M + m];
+            gv[q] = g[row[q] * M + m];
+        }
+#pragma unroll
+        for (int q = 0; q < kGradRows; ++q) {
+            const double dx = x[q][0] - m0, dy = x[q][1] - m1, dz = x[q][2] - m2;
+            s[q][0] = __builtin_fma(f[q], -2.0 * (a0 * dx + a3 * dy + a4 * dz) * gv[q], s[q][0]);
+            s[q][1] = __builtin_fma(f[q], -2.0 * (a3 * dx + a1 * dy + a5 * dz) * gv[q], s[q][1]);
+            s[q][2] = __builtin_fma(f[q], -2.0 * (a4 * dx + a5 * dy + a2 * dz) * gv[q], s[q][2]);
+        }
     }
-    s0 = wave_sum(s0); s1 = wave_sum(s1); s2 = wave_sum(s2);
-    if (lane == 0) {
-        grad[3 * r] = 2.0 * s0;
-        grad[3 * r + 1] = 2.0 * s1;
-        grad[3 * r + 2] = 2.0 * s2;
-    }
+#pragma unroll
+    for (int q = 0; q < kGradRows; ++q)
+        for (int c = 0; c < 3; ++c) {
+            const double t = wave_sum(s[q][c]);
+            if (lane == 0 && r0 + q < Gc) grad[3 * (r0 + q) + c] = 2.0 * t;
+        }
 }
 
 // grad_rd = 2 sum_o occ_o psi_ro dpsi_d,ro and tau_r = 1/2 sum_o occ_o |dpsi_ro|^2 (grid.py:128-134).
@@ -223,20 +252,27 @@ __global__ __launch_bounds__(256) void k_grid_basis_bwd(
     for (int c = 0; c < 10; ++c) o[(int64_t)c * M] += acc[c];
 }
 
-// Per splat: sum the slab partials in fixed order, then the chart reverse.
-__global__ void k_grid_splat_grad(int64_t M, int64_t slabs, const double* __restrict__ partial,
-                                  const double* __restrict__ quat,
-                                  const double* __restrict__ log_scale,
-                                  double* __restrict__ dquat, double* __restrict__ dlog_scale,
-                                  double* __restrict__ dcenters) {
-    const int64_t m = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (m >= M) return;
-    double acc[10];
-    for (int c = 0; c < 10; ++c) {
+// Per splat: sum the slab partials in fixed order, one thread per (splat, component), then the chart
+// reverse. Bound by its chains of loads (64 slabs): 7 us for 2000 splats,
+// 159 us with one thread per splat.
+constexpr int kSumSplats = 16;
+__global__ __launch_bounds__(10 * kSumSplats) void k_grid_splat_grad(
+    int64_t M, int64_t slabs, const double* __restrict__ partial, const double* __restrict__ quat,
+    const double* __restrict__ log_scale, double* __restrict__ dquat,
+    double* __restrict__ dlog_scale, double* __restrict__ dcenters) {
+    __shared__ double sum[10][kSumSplats];
+    const int i = threadIdx.x % kSumSplats, c = threadIdx.x / kSumSplats;
+    const int64_t m = blockIdx.x * (int64_t)kSumSplats + i;
+    if (m < M) {
         double s = 0.0;
+#pragma unroll 8
         for (int64_t k = 0; k < slabs; ++k) s += partial[(k * 10 + c) * M + m];
-        acc[c] = s;
+        sum[c][i] = s;
     }
+    __syncthreads();
+    if (c != 0 || m >= M) return;
+    double acc[10];
+    for (int q = 0; q < 10; ++q) acc[q] = sum[q][i];
     chart_reverse(m, acc, quat, log_scale, dquat, dlog_scale, dcenters);
 }
 
@@ -356,7 +392,8 @@ extern "C" int gsdft_grid_density(int64_t M, const double* quat, const double* l
     GSDFT_TRY(launch_chart(M, quat, log_scale, w.A6, w.Nrm, s));
     for (int64_t r0 = 0; r0 < G; r0 += chunk) {
         const int64_t Gc = G - r0 < chunk ? G - r0 : chunk;
-        double* dg = mode >= 1 ? w.gb + Gc * M : nullptr;
+        // rho's orbitals and, with k_grid_grad_phi, its gradient ask for g alone
+        double* dg = mode == 2 ? w.gb + Gc * M : nullptr;
         k_grid_basis<<<dim3(nblk(M, 256), (unsigned)Gc), 256, 0, s>>>(M, Gc, points + 3 * r0, w.A6,
                                                                       centers, w.Nrm, w.gb, dg);
         GSDFT_HIP(hipGetLastError());
@@ -370,7 +407,8 @@ extern "C" int gsdft_grid_density(int64_t M, const double* quat, const double* l
             k_grid_scale_occ<<<nblk(Gc * k, 256), 256, 0, s>>>(Gc, k, ldk, w.pb, occ, pocc);
             GSDFT_HIP(hipGetLastError());
             GSDFT_TRY(gemm_cm('T', 'N', M, Gc, k, 1.0, Cuse, ldk, pocc, ldk, 0.0, w.phi, M, s));
-            k_grid_grad_phi<<<nblk(Gc * 64, 256), 256, 0, s>>>(Gc, M, w.phi, dg, grad + 3 * r0);
+            k_grid_grad_phi<<<nblk((Gc + kGradRows - 1) / kGradRows * 64, 256), 256, 0, s>>>(
+                Gc, M, w.phi, w.gb, points + 3 * r0, w.A6, centers, grad + 3 * r0);
         } else if (mode == 2) {
             k_grid_grad_tau<<<nblk(Gc * 64, 256), 256, 0, s>>>(Gc, k, ldk, w.pb, occ,
                                                                grad + 3 * r0, tau + r0);
@@ -430,7 +468,7 @@ extern "C" int gsdft_grid_density_vjp(int64_t M, const double* quat, const doubl
             w.partial);
         GSDFT_HIP(hipGetLastError());
     }
-    k_grid_splat_grad<<<nblk(M, 256), 256, 0, s>>>(M, slabs, w.partial, quat, log_scale, dquat,
+    k_grid_splat_grad<<<nblk(M, kSumSplats), 10 * kSumSplats, 0, s>>>(M, slabs, w.partial, quat, log_scale, dquat,
                                                    dlog_scale, dcenters);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
