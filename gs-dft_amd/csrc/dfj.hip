@@ -1434,6 +1434,7 @@ __global__ __launch_bounds__(256) void k_splat_grad(
 // k) then take a partner's row and 1 << log2g partners are summed side by side, each thread its
 // share of the partners in order, the shares in order at the end (CO2, k = 11: 27.6 us for 250
 // partner rows one after the other).
+// With `only_if`, a device flag, the launch leaves dC alone unless it is set.
 __global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunks, int log2g,
                                             const int32_t* __restrict__ row_ptr,
                                             const int32_t* __restrict__ row_perm,
@@ -1445,7 +1446,9 @@ __global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunk
                                             const double* __restrict__ weight,
                                             const double* __restrict__ C,
                                             const double* __restrict__ occ,
-                                            double* __restrict__ dC) {
+                                            double* __restrict__ dC,
+                                            const int32_t* __restrict__ only_if) {
+    if (only_if && *only_if == 0) return;        // grid-uniform
     __shared__ int32_t partner[256];
     __shared__ double scale[256];
     const int64_t lb = xcd_block(M * nchunks);
@@ -1481,13 +1484,82 @@ __global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunk
     if (o < k) dC[m * k + o] = occ[o] * acc;
 }
 
+// The same sum as one dense product, dC^T = occ (C^T W) with W (M x M) the list's J w: k_dC reads a row
+// of C for each pair and side, 16 n k bytes at ~7.3 TB/s, where the product takes 2 M^2 k operations.
+// k_pair_matrix writes row m of W, k_dense_c copies C with rows of ldk (a 16-byte multiple) and
+// zeros in place of infinities and NaN, whose products with W's zeros would reach every row: it
+// reports them in *bad, and k_dC then does the work after all.
+// One workgroup per splat; its entries in k_dC's order, 256 at a time: of the threads whose partners
+// share a slot of `claim` the lowest adds, then the next, so a pair listed more than once is summed
+// in list order. Bound by writing W.
+constexpr int kClaims = 2048;
+__global__ __launch_bounds__(256) void k_pair_matrix(int64_t M, int64_t ldw,
+                                                     const int32_t* __restrict__ row_ptr,
+                                                     const int32_t* __restrict__ row_perm,
+                                                     const int32_t* __restrict__ col_ptr,
+                                                     const int32_t* __restrict__ col_perm,
+                                                     const int32_t* __restrict__ pi,
+                                                     const int32_t* __restrict__ pj,
+                                                     const double* __restrict__ J,
+                                                     const double* __restrict__ weight, double* W) {
+    __shared__ int claim[kClaims];
+    const int64_t m = blockIdx.x;
+    const int tid = threadIdx.x;
+    double* row = W + m * ldw;
+    for (int64_t j = tid; j < ldw; j += 256) row[j] = 0.0;
+    for (int h = tid; h < kClaims; h += 256) claim[h] = 256;
+    __syncthreads();
+    const int64_t r0 = row_ptr[m], r1 = row_ptr[m + 1], c0 = col_ptr[m], c1 = col_ptr[m + 1];
+    const int64_t nr = r1 - r0, total = nr + (c1 - c0);
+    for (int64_t b0 = 0; b0 < total; b0 += 256) {
+        const int64_t e = b0 + tid;
+        bool pending = e < total;
+        int32_t j = 0;
+        double v = 0.0;
+        if (pending) {
+            const int64_t a = e < nr ? row_perm[r0 + e] : col_perm[c0 + e - nr];
+            j = e < nr ? pj[a] : pi[a];
+            v = J[a] * weight[a];
+        }
+        int* slot = claim + j % kClaims;
+        do {                                     // each round serves every claimed slot once
+            if (pending) atomicMin(slot, tid);
+            __syncthreads();
+            const bool mine = pending && *slot == tid;
+            __syncthreads();
+            if (mine) {
+                row[j] += v;
+                *slot = 256;
+                pending = false;
+            }
+        } while (__syncthreads_or(pending ? 1 : 0));
+    }
+}
+
+__global__ void k_dense_c(int64_t M, int64_t k, int64_t ldk, const double* __restrict__ C,
+                          double* __restrict__ Cp, int32_t* __restrict__ bad) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i >= M * ldk) return;
+    const int64_t m = i / ldk, o = i % ldk;
+    const double v = o < k ? C[m * k + o] : 0.0;
+    const bool finite = __builtin_fabs(v) <= 0x1.fffffffffffffp+1023;
+    Cp[i] = finite ? v : 0.0;
+    if (!finite) atomicOr(bad, 1);
+}
+
+__global__ void k_scale_rows(int64_t M, int64_t k, const double* __restrict__ occ,
+                             double* __restrict__ dC) {
+    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (i < M * k) dC[i] = occ[i % k] * dC[i];
+}
+
 // ------------------------------------------------------------------ nuclear attraction
 // gs_dft/screening/pairs.py:348-370: V_a = -N_i N_j K sum_A Z_A (2/sqrt(pi)) sum_t w_t pi^1.5
 // det(B_t)^(-1/2) exp(-(t^2 |d|^2 - t^4 d.adj(B_t) d / det B_t)), B_t = Ah + t^2 I, d = Pa - R_A.
 // With s = t^2: det B_t = Pn(s) and the exponent is s d.Ah (Ah + s I)^-1 d = s Qn(s)/Pn(s), the
 // three-centre node of an aux function whose exponent b grows without bound (s_t = t^2 b/(b + t^2)
-// -> t^2, w_t (b + t^2)^(-3/2) -> w_t once the aux norm is divided out). So the nuclei enter the
-// reverse kernel as aux records with s_t = t^2, wp_t = w_t and u = -Z_A, and the prefactor is
+// -> t^2, w_t (b + t^2)^(-3/2) -> w_t once the aux norm is divided out). So a nucleus is an aux
+// function of the reverse kernel with s_t = t^2, wp_t = w_t and u = -Z_A, and the prefactor is
 // (2/sqrt(pi)) pi^1.5 = 2 pi.
 constexpr double kPrefNuc = 2.0 * kPi;
 
@@ -2501,7 +2573,7 @@ int launch_pair_density(int64_t n, const int32_t* pi, const int32_t* pj, const d
 int launch_dC(int64_t M, int64_t k, const int32_t* row_ptr, const int32_t* row_perm,
               const int32_t* col_ptr, const int32_t* col_perm, const int32_t* pi,
               const int32_t* pj, const double* J, const double* weight, const double* C,
-              const double* occ, double* dC, hipStream_t s) {
+              const double* occ, double* dC, hipStream_t s, const int32_t* only_if = nullptr) {
     const int64_t nchunks = (k + 255) / 256;
     int log2g = 0;
     while (log2g < 4 && (256 >> (log2g + 1)) >= k) ++log2g;
@@ -2509,9 +2581,50 @@ int launch_dC(int64_t M, int64_t k, const int32_t* row_ptr, const int32_t* row_p
         return fail(GSDFT_ERR_ARG, "dC: M = %lld x %lld orbital chunks too many for one launch",
                     (long long)M, (long long)nchunks);
     k_dC<<<xcd_grid(M * nchunks), 256, 0, s>>>(M, k, nchunks, log2g, row_ptr, row_perm, col_ptr,
-                                               col_perm, pi, pj, J, weight, C, occ, dC);
+                                               col_perm, pi, pj, J, weight, C, occ, dC, only_if);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
+}
+
+// dC as a dense product (k_pair_matrix) where that is the shorter way and `room` doubles at `area`
+// hold W, the copy of C and the flag; else k_dC.
+// With r = n / M^2, k_dC takes 16 r M^2 k bytes at 7.3 TB/s (globules) to 18 TB/s (a chain, whose
+// partners stay in L2), the product 3.4e-14 M^2 k s and W 6e-12 M^2 s: against the faster k_dC the
+// product is ahead from r = 0.038 + 6.7 / k on. Nuclear attraction of 12000 splats, k = 600, r =
+// 0.072: dC 13.7 -> 3.9 ms (the step 63.9 -> 53.5); of 5000, k = 330: the step 12.4 -> 10.8; below the
+// line, a chain of 11001 splats with k = 500 would go 18.4 -> 19.8 and 2203 splats with k = 97 stay
+// at 3.05.
+constexpr int64_t kDenseMinM = 2048;
+inline bool dense_dC_pays(int64_t M, int64_t k, int64_t n) {
+    return M >= kDenseMinM && (double)n * k > (double)M * M * (0.04 * k + 8.0);
+}
+
+int launch_dC_list(int64_t M, int64_t k, int64_t n, const int32_t* row_ptr,
+                   const int32_t* row_perm, const int32_t* col_ptr, const int32_t* col_perm,
+                   const int32_t* pi, const int32_t* pj, const double* J, const double* weight,
+                   const double* C, const double* occ, double* dC, double* area, int64_t room,
+                   hipStream_t s) {
+    const int64_t ldw = M + (M & 1), ldk = k + (k & 1);
+    const int64_t fixed = M * ldw + M * ldk + 2;
+    if (!dense_dC_pays(M, k, n) || fixed > room || reinterpret_cast<uintptr_t>(area) % 16 != 0 ||
+        M * ldk > (int64_t)UINT32_MAX - 256)
+        return launch_dC(M, k, row_ptr, row_perm, col_ptr, col_perm, pi, pj, J, weight, C, occ, dC,
+                         s);
+    double* W = area;
+    double* Cp = W + M * ldw;
+    double* flag = Cp + M * ldk;
+    int32_t* bad = reinterpret_cast<int32_t*>(flag);
+    k_fill<<<1, 64, 0, s>>>(1, 0.0, flag);
+    k_dense_c<<<blocks_for(M * ldk, 256), 256, 0, s>>>(M, k, ldk, C, Cp, bad);
+    k_pair_matrix<<<(unsigned)M, 256, 0, s>>>(M, ldw, row_ptr, row_perm, col_ptr, col_perm, pi, pj,
+                                              J, weight, W);
+    GSDFT_HIP(hipGetLastError());
+    GSDFT_TRY(gemm_cm_split('N', 'N', k, M, M, 1.0, Cp, ldk, W, ldw, 0.0, dC, k, flag + 2,
+                            room - fixed, s));
+    k_scale_rows<<<blocks_for(M * k, 256), 256, 0, s>>>(M, k, occ, dC);
+    GSDFT_HIP(hipGetLastError());
+    return launch_dC(M, k, row_ptr, row_perm, col_ptr, col_perm, pi, pj, J, weight, C, occ, dC, s,
+                     bad);
 }
 
 // Shared prologue of forward and reverse: chart, aux quantities (skipped for a null log_alpha),
@@ -3602,7 +3715,8 @@ __global__ void k_atom_force_finish(int64_t n_atoms, int64_t groups,
     datoms[i] = -charges[i / 3] * kPrefNuc * s;
 }
 
-// V (n) = the nuclear attraction of every listed pair (jt of k_nuclear_pairs) and, for a non-null C, the slot moments behind its gradient.
+// V (n) = the nuclear attraction of every listed pair (jt of k_nuclear_pairs) and, for a non-null C,
+// the slot moments behind its gradient.
 int external_pass(int64_t M, const double* quat, const double* log_scale, const double* centers,
                   int64_t k, const double* C, const double* occ, int64_t n, const int32_t* pi,
                   const int32_t* pj, const double* weight, int64_t n_atoms,
@@ -3721,8 +3835,10 @@ extern "C" int gsdft_external_energy(
                                                              log_scale, dquat, dlog_scale,
                                                              dcenters);
         GSDFT_HIP(hipGetLastError());
-        GSDFT_TRY(launch_dC(M, k, row_ptr, row_perm, col_ptr, col_perm, pi, pj, V, weight, C, occ,
-                            dC, s));
+        // the moments are dead once folded into V and the splats' contributions
+        const int64_t room = std::max(bwd_split(n_atoms, n).slabs * kAcc * n, kRec * n);
+        GSDFT_TRY(launch_dC_list(M, k, n, row_ptr, row_perm, col_ptr, col_perm, pi, pj, V, weight,
+                                 C, occ, dC, w.g.acc, room, s));
     }
     if (datoms) {
         // the pair pass left each pair block's force on every nucleus: sum them in fixed order
