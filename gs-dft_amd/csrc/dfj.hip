@@ -1491,7 +1491,8 @@ __global__ __launch_bounds__(256) void k_dC(int64_t M, int64_t k, int64_t nchunk
 // reports them in *bad, and k_dC then does the work after all.
 // One workgroup per splat; its entries in k_dC's order, 256 at a time: of the threads whose partners
 // share a slot of `claim` the lowest adds, then the next, so a pair listed more than once is summed
-// in list order. Bound by writing W.
+// in list order; a value of zero (padding inside a list: thousands of (0, 0) entries would take a
+// round each) adds nothing to a sum that starts at +0 and is left out. Bound by writing W.
 constexpr int kClaims = 2048;
 __global__ __launch_bounds__(256) void k_pair_matrix(int64_t M, int64_t ldw,
                                                      const int32_t* __restrict__ row_ptr,
@@ -1520,6 +1521,7 @@ __global__ __launch_bounds__(256) void k_pair_matrix(int64_t M, int64_t ldw,
             const int64_t a = e < nr ? row_perm[r0 + e] : col_perm[c0 + e - nr];
             j = e < nr ? pj[a] : pi[a];
             v = J[a] * weight[a];
+            pending = v != 0.0;
         }
         int* slot = claim + j % kClaims;
         do {                                     // each round serves every claimed slot once

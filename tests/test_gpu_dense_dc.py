@@ -60,3 +60,28 @@ def test_dense_dc_keeps_a_bad_coefficient_to_its_partners(g, wl, cuda, bad):
     fine = torch.isfinite(ref)
     assert bool((torch.isfinite(got) == fine).all()) and bool((~fine).any()) and bool(fine.any())
     assert bool(((got - ref).abs()[fine] <= 4200 * 2.0 ** -53 * mag[fine]).all())
+
+
+def test_dense_dc_padding_inside_the_list(g, wl, cuda):
+    """Weightless (0, 0) entries between the real ones change nothing but the order of sums: 2 M
+    terms a row on each side, and V's nodes a few dozen roundings apart."""
+    M, k = 2048, 96
+    s = wl.make_small(M, k, n_atoms=30, seed=5, spread=2.0)
+    cu = lambda a: torch.tensor(np.asarray(a), device="cuda", dtype=torch.float64)
+    b = g.Splat(quat=cu(s.quat), log_scale=cu(s.log_scale), centers=cu(s.centers))
+    pi, pj, w = g.neighbor_pairs(b, eps=1e-7, unique=True)
+    w = w.to(torch.float64)
+    h = len(pi) // 2
+    got = []
+    for pad in (0, 100001):
+        z = lambda t: torch.cat([t[:h], torch.zeros(pad, dtype=t.dtype, device=t.device), t[h:]])
+        C = cu(s.C).requires_grad_(True)
+        g.screened_external_energy(b, C, s.occ, z(pi), z(pj), s.atoms, s.charges,
+                                   valid=z(w)).backward()
+        got.append(C.grad)
+    x = (g.screened_nuclear_pairs(b, pi, pj, s.atoms, s.charges) * w).abs()
+    mag = torch.zeros_like(got[0])
+    for p, q in ((pi.long(), pj.long()), (pj.long(), pi.long())):
+        mag.index_add_(0, p, x[:, None] * cu(s.C)[q].abs())
+    mag *= cu(s.occ)
+    assert bool(((got[0] - got[1]).abs() <= (4 * M + 64) * 2.0 ** -53 * mag).all())
