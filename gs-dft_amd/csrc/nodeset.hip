@@ -9,17 +9,19 @@
 // over exp(-s u), u = |R - r|^2, with a positive weight (it is the integral of the product Gaussian
 // against exp(-s |R - r|^2)), so any node list that reproduces
 //     K_b(u) = sum_t w_t (b + t^2)^(-3/2) exp(-s_t u)
-// to a relative error e at every u in reach reproduces every (P|a), and its derivatives, to e.
+// to a relative error e at every u in reach reproduces every (P|a) to e.
 // k_node_sets picks such a list for each centre: of the centre's 20 nb nodes, the columns that
 // Gaussian elimination with complete pivoting takes from the matrix exp(-s_j u_i) w_j / min_b
 // K_b(u_i), until what is left is below kSetTol; the others' weights are spread over those taken
 // (an interpolative decomposition: the coefficients stay of order one). 40 to 60 nodes replace the
-// 80 of four scales, 27 to 36 the 40 of two; against 80-bit arithmetic the lists reproduce K_b(u)
-// to 2e-16 (root mean square over u; at most 2e-14 anywhere) for exponents from 0.05 to 64 and
-// |R - r| up to 55 Bohr. Every product Gaussian is, in turn, an average of isotropic Gaussians of
-// exponent l >= its largest eigenvalue, so the matrix is formed for those (s -> s l / (l + s),
-// weights (l / (l + s))^(3/2), u the squared distance to their centres), which takes a node or two
-// fewer where b > l.
+// 80 of four scales, 27 to 40 the 40 of two. Against 80-bit arithmetic the lists reproduce (P|a) of
+// random pairs (exponents from 0.03 to 64, eigenvalues from 0.02 to 60, systems of 0.01 to 40 Bohr) to
+// 2e-16 in the median and 7e-15 at most. A derivative has no bound of its own: 1e-15 of its terms'
+// magnitudes in the median, 3e-13 at most within 3 Bohr and 2e-12 at 20, where it is small beside
+// (P|a) itself.
+// Every product Gaussian is, in turn, an average of isotropic Gaussians of exponent l >= its largest
+// eigenvalue, so the matrix is formed for those (s -> s l / (l + s), weights (l / (l + s))^(3/2), u the
+// squared distance to their centres), which takes a node or two fewer where b > l.
 #include "common.h"
 #include "internal.h"
 
@@ -31,6 +33,13 @@ constexpr int kSetRows = 96;          // points in u
 constexpr int kSetThreads = 320;
 constexpr double kSetTol = 4e-15;
 constexpr double kSetFirst = 2.0;     // u grid: u_i = c (e^(a i) - 1), c = kSetFirst / largest s
+// The u grid ends kSetTail^(1/2) widths past the far corner of the pairs' centres, where the widest
+// pair's Gaussian has fallen to e^-kSetTail; the lists extrapolate beyond. Over 1200 random clusters
+// within 3 Bohr, splats up to fifty times as long as thick, (P|a) erred by up to 1.1e-13 with 8 and
+// by 3e-15 to 6e-15 with 10 to 60, its derivatives by 7e-12 and by 2e-13 to 3e-13 of their terms, for
+// 27 nodes in the mean with 8, 28 with 10, 29.5 with 16 and 32 with 36. The water octamer's step
+// takes 11.20 ms with 16, 11.00 with 8; C20H42's 90.3 and 89.1.
+constexpr double kSetTail = 16.0;
 constexpr int kBoxBlocks = 256;
 
 template <int kCtrl>
@@ -193,14 +202,14 @@ __global__ __launch_bounds__(kSetThreads) void k_node_sets(
     };
     int rank = 0;
     if (shared) {
-        // reach: from R to the far corner of the pairs' centres, plus some widths of the widest
+        // reach: from R to the far corner of the pairs' centres, plus the tail of the widest
         const double lam = __builtin_fmin(__builtin_fmax(box[7], 1e-30), 1e30);
         double d2 = 0.0;
         for (int c = 0; c < 3; ++c) {
             const double d = __builtin_fmax(rc[c] + box[c], box[3 + c] - rc[c]);
             d2 += d * d;
         }
-        const double reach = sqrt(d2) + sqrt(8.0 * box[6]);
+        const double reach = sqrt(d2) + sqrt(kSetTail * box[6]);
         const double c0 = kSetFirst * (lam + bmax) / (bmax * lam);
         double um = __builtin_fmax(__builtin_fmin(reach * reach, 1e12), 4.0 * c0);
         // the smallest s of the group; past s u = 600 every term has vanished

@@ -96,3 +96,71 @@ def test_exchange_on_shared_lists_matches_plain_records(g, wl, cuda, scales):
         print(f"[sets] exchange {len(scales)} scales, chunk {chunk}: n={pi.shape[0]} "
               + " ".join(f"{e:.1e}" for e in errs), flush=True)
         assert errs[0] < 1e-10 and max(errs[1:]) < 1e-9
+
+
+def _aligned_gamma(mu, ls, ac, la, W):
+    """gamma of splats whose precisions are all diagonal, (scales, centres), in the arithmetic of the
+    arguments: with eigenvalues l = e^ls the pair's are L = l_i + l_j, and a node of exponent s takes
+    prod_k (L_k + s)^(-1/2) exp(-s L_k d_k^2 / (L_k + s)). W holds the weights of the pairs (i, j)."""
+    from oracle import oracle as orc
+    t, wt = (a.astype(np.longdouble) for a in orc.quad_table())
+    l = np.exp(ls)
+    pi = 4 * np.arctan(np.longdouble(1))
+    N = np.prod((2 * l / pi) ** np.longdouble(0.25), axis=1)
+    L = l[:, None] + l[None]
+    P = ((l * mu)[:, None] + (l * mu)[None]) / L
+    D = mu[:, None] - mu[None]
+    q = N[:, None] * N[None] * np.exp(-(l[:, None] * l[None] / L * D * D).sum(2)) * W
+    out = np.zeros(la.shape, L.dtype)
+    for c in range(la.shape[1]):
+        d2 = (ac[c] - P) ** 2
+        for g in range(la.shape[0]):
+            b = np.exp(np.longdouble(la[g, c]))
+            s = (t * t * b / (b + t * t))[:, None, None, None]
+            f = np.prod(1 / np.sqrt(L + s), axis=3) * np.exp(-(s * L * d2 / (L + s)).sum(3))
+            w = wt / ((b + t * t) * np.sqrt(b + t * t))
+            out[g, c] = ((w[:, None, None] * f).sum(0) * q).sum() * (2 * b / pi) ** np.longdouble(0.75)
+    return out * 2 * pi ** 3 / np.sqrt(pi)
+
+
+@pytest.mark.parametrize("scales", [4, 2])
+def test_compact_cluster_of_wide_splats(g, cuda, scales):
+    """Splats ten times as long as they are thick, side by side within 0.2 Bohr, so that the widest
+    pair's Gaussian reaches far past the box of the pairs' centres, and diffuse aux on them. The
+    reference is 80-bit arithmetic, its derivatives by complex steps; all terms of gamma are positive.
+
+    A node's value errs by at most 8e-15 of its prefactor (the hardware root's estimate, squared, and
+    the exponential), so gamma errs by 1e-14, and a derivative, whose terms cancel to a few parts in
+    ten here, by 1e-13 of the largest."""
+    M, n = 8, N_MIN + 8
+    rng = np.random.default_rng(3)
+    mu = rng.normal(0.0, 0.1, (M, 3))
+    ls = -np.log(2.0 * np.array([4.0, 0.3, 0.3]) ** 2) + rng.uniform(-0.05, 0.05, (M, 3))
+    la = np.log(0.1 * np.geomspace(0.5, 4.0, scales))[:, None] + rng.uniform(-0.1, 0.1, M)[None]
+    ac = mu.copy()
+    a = np.arange(n) % (M * M)
+    i, j = (a // M).astype(np.int32), (a % M).astype(np.int32)
+    w = rng.uniform(0.5, 2.0, n)
+    W = np.zeros((M, M), np.longdouble)
+    np.add.at(W, (i, j), w.astype(np.longdouble))
+    ref = _aligned_gamma(mu.astype(np.longdouble), ls.astype(np.longdouble), ac, la, W)
+    h = np.longdouble(1e-30)
+    dref = np.zeros((2, M, 3), np.longdouble)
+    for v, m, k in np.ndindex(2, M, 3):
+        x = [mu.astype(np.clongdouble), ls.astype(np.clongdouble)]
+        x[v][m, k] += 1j * h
+        dref[v, m, k] = _aligned_gamma(*x, ac, la, W).imag.sum() / h
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    quat = np.zeros((M, 4))
+    quat[:, 0] = 1.0
+    basis = g.Splat(quat=t(quat), log_scale=t(ls), centers=t(mu))
+    aux = g.IsotropicSplat(log_alpha=la.ravel(), centers=np.tile(ac, (scales, 1)))
+    gam = g.df_coulomb_gamma_screened(basis, np.ones((M, 1)), np.ones(1), aux, torch.tensor(i),
+                                      torch.tensor(j), valid=torch.tensor(w))
+    got = gam.detach().cpu().numpy().reshape(la.shape)
+    dl, dc = torch.autograd.grad(gam.sum(), [basis.log_scale, basis.centers])
+    errs = [float(np.abs(got / ref - 1).max())] + [
+        float(np.abs(x.cpu().numpy() - y).max() / np.abs(y).max()) for x, y in zip((dc, dl), dref)]
+    print(f"[sets] compact, {scales} scales: gamma {errs[0]:.1e} dcenters {errs[1]:.1e} "
+          f"dlog_scale {errs[2]:.1e}", flush=True)
+    assert errs[0] < 1e-14 and max(errs[1:]) < 1e-13
