@@ -514,10 +514,13 @@ constexpr double kExpMinusHalf = 0x1.368b2fc6f960ap-1;     // e^(-1/2), correctl
 // Layout of the node lists that k_node_sets (nodeset.hip) writes and the three-centre passes read.
 // The aux functions are taken in groups of at most kMaxSetScales consecutive slots of one centre.
 // A group holds sub-records (one, unless its functions do not share a centre): a header R (3),
-// bits (node count, even | last << 32), then per node, in ascending s: s, 1/s and the weight of
-// each function (kSetForward); s, weight, s^2, 1/s with the functions' cotangents folded into the
-// one weight (kSetFold); or s, 1/s, the four functions' weights times KN_P, s^2 and a pad
-// (kSetExchange). Weights carry s^(-1/2) e^(-1/2) / 24 (exp_quartic).
+// bits (node count, even | last << 32 | only << 33), then per node, in ascending s: s, 1/s and the
+// weight of each function (kSetForward); s, weight, s^2, 1/s with the functions' cotangents folded
+// into the one weight (kSetFold); or s, 1/s, the four functions' weights times KN_P, s^2 and a pad
+// (kSetExchange). Weights carry s^(-1/2) e^(-1/2) / 24 (exp_quartic). A sub-record of a single
+// function b has only = b + 1 (else 0), and the other functions' sums leave it alone, as its centre
+// or exponent may be NaN; in kSetForward its nodes are a plain record's four values s, -ln w', S, 1/s
+// (exp_neg_tab_k_w), one after the other.
 constexpr int kMaxSetScales = 4;
 constexpr int kSetHeader = 4;
 

@@ -695,6 +695,41 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_sets(int64_t n, int64_t pairs
     const int64_t a_end = min(n, a_begin + pairs);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint64_t lane_nodes = 0;                 // profiling: node evaluations over live lanes
+    // a single function's twenty nodes, k_gamma_fwd_pairs' two a step, into sum `at`
+    auto one = [&](UniformPtr y, double I1, double I2, double I3, double q1, double rr, double X0,
+                   double cf, int at) {
+        const double c256 = vgpr_const(kNegC256);
+        struct Node {
+            double s, lw, S, is;
+        };
+        auto read = [](UniformPtr z) { return Node{z[0], z[1], z[2], z[3]}; };
+        Node n0 = read(y), n1 = read(y + 4);
+        double F = 0.0, arg = 0.0;
+        auto add = [&](const Node& c) {
+            const double Pr = __builtin_fma(c.is, I3, __builtin_fma(c.s, I1 + c.s, I2));
+            const double Qn = __builtin_fma(c.s, __builtin_fma(c.s, q1, rr), X0);
+            const double y0 = __builtin_amdgcn_rsq(Pr);
+            const double h = y0 * y0;
+            const double e1 = __builtin_fma(-Pr, h, 2.0);
+            arg = __builtin_fma(Qn, h, -0.5);
+            F = __builtin_fma(y0, exp_neg_tab_k_w(__builtin_fma(arg, e1, c.lw), c.S, c256, tab), F);
+        };
+        int t = 0;
+        bool done;
+        do {
+            const Node c0 = n0, c1 = n1;
+            y += 8;
+            n0 = read(y);
+            n1 = read(y + 4);
+            __builtin_amdgcn_sched_barrier(0);
+            add(c0);
+            add(c1);
+            t += 2;
+            done = (t >= kNodes) | wave_all_beyond_h(arg);
+        } while (!done);
+        acc[at][threadIdx.x] = __builtin_fma(F, cf, acc[at][threadIdx.x]);
+        return t;
+    };
     for (int64_t a0 = a_begin + 64 * wave; a0 < a_end; a0 += 256) {      // wave-uniform
         const int64_t a = a0 + lane;
         const bool live = a < a_end;
@@ -711,7 +746,8 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_sets(int64_t n, int64_t pairs
             do {                                     // wave-uniform; once unless centres differ
                 const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
                 const int count = (int)(uint32_t)head;
-                last = (head >> 32) != 0;
+                last = (head >> 32 & 1) != 0;
+                const int only = (int)(head >> 33);
                 const double dx = x[0] - Px, dy = x[1] - Py, dz = x[2] - Pz;
                 const double ax = __builtin_fma(xx, dx, __builtin_fma(xy, dy, xz * dz));
                 const double ay = __builtin_fma(xy, dx, __builtin_fma(yy, dy, yz * dz));
@@ -722,11 +758,15 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_sets(int64_t n, int64_t pairs
                 const double X0 = I3 * q0d;
                 const double rr = __builtin_fma(I1, q1, -q2);
                 const double cf = (q0d == q0d) ? coef : q0d;      // a NaN centre propagates
+                UniformPtr y = x + kSetHeader;
+                x = y + kNd * count;
+                if (only) {                          // wave-uniform: one function's plain nodes
+                    lane_nodes += lanes * (uint64_t)one(y, I1, I2, I3, q1, rr, X0, cf, only - 1 + NB * j);
+                    continue;
+                }
                 double F[NB];
 #pragma unroll
                 for (int b = 0; b < NB; ++b) F[b] = 0.0;
-                UniformPtr y = x + kSetHeader;
-                x = y + kNd * count;
                 // Two nodes a step (lists are padded to an even length): one's latencies are filled
                 // by the other's instructions, and the screen is tested once, on the second (the
                 // larger exponent). The next two nodes' constants are read meanwhile (the slots
@@ -1101,7 +1141,7 @@ __global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kSet ? 4 : 1) void k_gamm
             do {                                     // wave-uniform; once unless centres differ
                 const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
                 const int count = (int)(uint32_t)head;
-                last = (head >> 32) != 0;
+                last = (head >> 32 & 1) != 0;
                 centre(x[0], x[1], x[2]);
                 constexpr int kNd = kLaneU ? 8 : 4;
                 UniformPtr y = x + kSetHeader;
@@ -2338,7 +2378,8 @@ __global__ __launch_bounds__(256) void k_exch_block_sets(int64_t n, const double
         do {                                     // wave-uniform; once unless centres differ
             const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
             const int count = (int)(uint32_t)head;
-            last = (head >> 32) != 0;
+            last = (head >> 32 & 1) != 0;
+            const int only = (int)(head >> 33);
             const double dx = x[0] - Px, dy = x[1] - Py, dz = x[2] - Pz;
             const double ax = xx * dx + xy * dy + xz * dz;
             const double ay = xy * dx + yy * dy + yz * dz;
@@ -2388,7 +2429,8 @@ __global__ __launch_bounds__(256) void k_exch_block_sets(int64_t n, const double
             } while (!done);
             nodes += t;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) V[b] = __builtin_fma(F[b], cf, V[b]);
+            for (int b = 0; b < 4; ++b)
+                if (only == 0 || only == b + 1) V[b] = __builtin_fma(F[b], cf, V[b]);
         } while (!last);
 #pragma unroll
         for (int b = 0; b < 4; ++b) val[4 * j + b][threadIdx.x] = V[b];

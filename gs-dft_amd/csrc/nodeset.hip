@@ -306,12 +306,22 @@ __global__ __launch_bounds__(kSetThreads) void k_node_sets(
             if (ct == 0) {
                 x[0] = R[3 * p]; x[1] = R[3 * p + 1]; x[2] = R[3 * p + 2];
                 x[3] = __builtin_bit_cast(double, (uint64_t)kNodes |
-                                                      ((uint64_t)(cb == nb - 1) << 32));
+                                                      ((uint64_t)(cb == nb - 1) << 32) |
+                                                      ((uint64_t)(cb + 1) << 33));
             }
-            double w[NB];
+            if (form == kSetForward) {
+                double* y = x + kSetHeader + 4 * ct;
+                double S;
+                y[0] = s;
+                y[1] = fold_weight(wp / sqrt(s) * (kExpMinusHalf / kExpPolyK), &S);
+                y[2] = S;
+                y[3] = 1.0 / s;
+            } else {
+                double w[NB];
 #pragma unroll
-            for (int b = 0; b < NB; ++b) w[b] = b == cb ? wp : 0.0;
-            put(x + kSetHeader, ct, s, w);
+                for (int b = 0; b < NB; ++b) w[b] = b == cb ? wp : 0.0;
+                put(x + kSetHeader, ct, s, w);
+            }
         }
         return;
     }

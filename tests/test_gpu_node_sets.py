@@ -164,3 +164,28 @@ def test_compact_cluster_of_wide_splats(g, cuda, scales):
     print(f"[sets] compact, {scales} scales: gamma {errs[0]:.1e} dcenters {errs[1]:.1e} "
           f"dlog_scale {errs[2]:.1e}", flush=True)
     assert errs[0] < 1e-14 and max(errs[1:]) < 1e-13
+
+
+@pytest.mark.parametrize("scales", [3, 4])
+@pytest.mark.parametrize("bad", ["centre", "exponent", "overflow"])
+def test_bad_function_keeps_to_itself(g, wl, orc, cuda, scales, bad):
+    """One aux function with a NaN centre, a NaN exponent or one past the largest double: gamma of every
+    other function, those grouped with it included, agrees with the oracle (bar as above)."""
+    s, la, ac, i, j, w = _case(wl, "three" if scales == 3 else "four")
+    la, ac = la.copy(), ac.copy()
+    at = s.M + 4                                   # second scale of the fifth centre
+    if bad == "centre":
+        ac[at, 1] = np.nan
+    else:
+        la[at] = np.nan if bad == "exponent" else 800.0
+    basis = g.Splat(quat=s.quat, log_scale=s.log_scale, centers=s.centers)
+    got = g.df_coulomb_gamma_screened(basis, s.C, s.occ, g.IsotropicSplat(log_alpha=la, centers=ac),
+                                      torch.tensor(i), torch.tensor(j),
+                                      valid=torch.tensor(w)).cpu().numpy()
+    la[at], ac[at] = 0.0, 0.0
+    ref = orc.gamma(s.quat, s.log_scale, s.centers, s.C, s.occ, la, ac, i, j, w)
+    big = np.full((s.M, 1), np.sqrt(np.abs((s.C * s.occ) @ s.C.T).max()))
+    unit = orc.gamma(s.quat, s.log_scale, s.centers, big, np.ones(1), la, ac, i, j, w)
+    rest = np.arange(len(la)) != at
+    assert not np.isfinite(got[at])
+    assert np.all(np.abs(got - ref)[rest] <= 1e-12 * unit[rest])
