@@ -2373,7 +2373,6 @@ __global__ __launch_bounds__(256) void k_exch_block_sets(int64_t n, const double
     uint32_t nodes = 0;
     for (int j = 0; j < ngr; ++j) {
         UniformPtr x = uniform_ptr(sets + stride * (g0 + j));
-        double V[4] = {0.0, 0.0, 0.0, 0.0};
         bool last;
         do {                                     // wave-uniform; once unless centres differ
             const uint64_t head = __builtin_bit_cast(uint64_t, x[3]);
@@ -2392,48 +2391,55 @@ __global__ __launch_bounds__(256) void k_exch_block_sets(int64_t n, const double
             const double cf = (q0d == q0d) ? coef : q0d;          // a NaN centre propagates
             UniformPtr y = x + kSetHeader;
             x = y + kNd * count;
-            double F[4] = {0.0, 0.0, 0.0, 0.0};
-            // two nodes a step, as in k_gamma_fwd_sets
-            struct Node {
-                double s, is, w[4];
+            // two nodes a step, as in k_gamma_fwd_sets; the sums of KB functions from `b0` on
+            auto walk = [&](auto kb, int b0, double (&F)[decltype(kb)::value]) {
+                constexpr int KB = decltype(kb)::value;
+                struct Node {
+                    double s, is, w[KB];
+                };
+                auto read = [b0](UniformPtr z) {
+                    Node c;
+                    c.s = z[0];
+                    c.is = z[1];
+#pragma unroll
+                    for (int b = 0; b < KB; ++b) c.w[b] = z[2 + b0 + b];
+                    return c;
+                };
+                Node n0 = read(y), n1 = read(y + kNd);
+                int t = 0;
+                bool done;
+                do {
+                    const Node c0 = n0, c1 = n1;
+                    y += 2 * kNd;
+                    n0 = read(y);
+                    n1 = read(y + kNd);
+                    __builtin_amdgcn_sched_barrier(0);     // issued here, not beside the table's
+                    const double P0 = __builtin_fma(c0.is, I3, __builtin_fma(c0.s, I1 + c0.s, I2));
+                    const double P1 = __builtin_fma(c1.is, I3, __builtin_fma(c1.s, I1 + c1.s, I2));
+                    const double Q0 = __builtin_fma(c0.s, __builtin_fma(c0.s, q1, rr), X0);
+                    const double Q1 = __builtin_fma(c1.s, __builtin_fma(c1.s, q1, rr), X0);
+                    const NodeArgH v0 = node_arg_h(P0, Q0), v1 = node_arg_h(P1, Q1);
+                    const double f0 = v0.y0 * exp_neg_tab_k<true>(v0.arg, tab);
+                    const double f1 = v1.y0 * exp_neg_tab_k<true>(v1.arg, tab);
+#pragma unroll
+                    for (int b = 0; b < KB; ++b)
+                        F[b] = __builtin_fma(c1.w[b], f1, __builtin_fma(c0.w[b], f0, F[b]));
+                    t += 2;
+                    done = (t >= count) | wave_all_beyond_h(v1.arg);
+                } while (!done);
+                nodes += t;
             };
-            auto read = [](UniformPtr z) {
-                Node c;
-                c.s = z[0];
-                c.is = z[1];
+            if (only) {                              // wave-uniform
+                double F[1] = {0.0};
+                walk(std::integral_constant<int, 1>{}, only - 1, F);
+                val[4 * j + only - 1][threadIdx.x] = F[0] * cf;
+            } else {
+                double F[4] = {0.0, 0.0, 0.0, 0.0};
+                walk(std::integral_constant<int, 4>{}, 0, F);
 #pragma unroll
-                for (int b = 0; b < 4; ++b) c.w[b] = z[2 + b];
-                return c;
-            };
-            Node n0 = read(y), n1 = read(y + kNd);
-            int t = 0;
-            bool done;
-            do {
-                const Node c0 = n0, c1 = n1;
-                y += 2 * kNd;
-                n0 = read(y);
-                n1 = read(y + kNd);
-                __builtin_amdgcn_sched_barrier(0);         // issued here, not beside the table's
-                const double P0 = __builtin_fma(c0.is, I3, __builtin_fma(c0.s, I1 + c0.s, I2));
-                const double P1 = __builtin_fma(c1.is, I3, __builtin_fma(c1.s, I1 + c1.s, I2));
-                const double Q0 = __builtin_fma(c0.s, __builtin_fma(c0.s, q1, rr), X0);
-                const double Q1 = __builtin_fma(c1.s, __builtin_fma(c1.s, q1, rr), X0);
-                const NodeArgH v0 = node_arg_h(P0, Q0), v1 = node_arg_h(P1, Q1);
-                const double f0 = v0.y0 * exp_neg_tab_k<true>(v0.arg, tab);
-                const double f1 = v1.y0 * exp_neg_tab_k<true>(v1.arg, tab);
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    F[b] = __builtin_fma(c1.w[b], f1, __builtin_fma(c0.w[b], f0, F[b]));
-                t += 2;
-                done = (t >= count) | wave_all_beyond_h(v1.arg);
-            } while (!done);
-            nodes += t;
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-                if (only == 0 || only == b + 1) V[b] = __builtin_fma(F[b], cf, V[b]);
+                for (int b = 0; b < 4; ++b) val[4 * j + b][threadIdx.x] = F[b] * cf;
+            }
         } while (!last);
-#pragma unroll
-        for (int b = 0; b < 4; ++b) val[4 * j + b][threadIdx.x] = V[b];
     }
     count_work(work, live, nodes);
     if (!live) return;

@@ -189,3 +189,30 @@ def test_bad_function_keeps_to_itself(g, wl, orc, cuda, scales, bad):
     rest = np.arange(len(la)) != at
     assert not np.isfinite(got[at])
     assert np.all(np.abs(got - ref)[rest] <= 1e-12 * unit[rest])
+
+
+@pytest.mark.parametrize("which", ["all", "some"])
+def test_exchange_groups_without_a_common_centre(g, wl, cuda, which):
+    """RI-K where no group of four functions, or only every second one, shares a centre, against the
+    plain records (an aux chunk of 66); lam and the bars as above."""
+    s = wl.make_small(190, 5, n_atoms=6, seed=4, spread=3.0)
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    basis = g.Splat(quat=t(s.quat), log_scale=t(s.log_scale), centers=t(s.centers))
+    C = t(s.C)
+    aux = g.init_product_aux(basis, scales=(0.5, 1.0, 2.0, 4.0))
+    rng = np.random.default_rng(8)
+    ac = aux.centers.detach().cpu().numpy().reshape(4, s.M, 3).copy()
+    ac[:, ::1 if which == "all" else 2] += rng.normal(0.0, 0.3, ac[:, ::1 if which == "all" else 2].shape)
+    aux = g.IsotropicSplat(log_alpha=aux.log_alpha.detach(), centers=ac.reshape(-1, 3))
+    pi, pj, v = g.neighbor_pairs(basis, eps=1e-9, unique=False)
+    assert pi.shape[0] >= N_MIN
+    L = g.aux_cholesky(aux, 1e-2)
+    out = []
+    for chunk in (66, 0, 64):
+        E = g.df_exchange_energy_screened(basis, C, aux, pi, pj, valid=v, cholV=L, aux_chunk=chunk)
+        out.append([E.detach().cpu().numpy()] + [x.cpu().numpy() for x in torch.autograd.grad(
+            E, [basis.quat, basis.log_scale, basis.centers, C])])
+    for got in out[1:]:
+        errs = [rel_max(a, b) for a, b in zip(got, out[0])]
+        print(f"[sets] exchange, {which} apart: " + " ".join(f"{e:.1e}" for e in errs), flush=True)
+        assert errs[0] < 1e-10 and max(errs[1:]) < 1e-9
