@@ -391,13 +391,16 @@ __global__ __launch_bounds__(256) void k_pair_density_run(int64_t n,
     }
 }
 
-// Pair record: I1 I2 I3 | Ah (6) | Pa (3) | coef = KN q pref | KN | q | pad.
-__global__ void k_pair_rec(int64_t n, const int32_t* __restrict__ pi,
+// Pair record: I1 I2 I3 | Ah (6) | Pa (3) | coef = KN q pref | KN | q | pad. Record `slot` is that of
+// pair perm[slot] (of pair `slot` for a null perm).
+__global__ void k_pair_rec(int64_t n, const int32_t* __restrict__ perm,
+                           const int32_t* __restrict__ pi,
                            const int32_t* __restrict__ pj, const double* __restrict__ A6,
                            const double* __restrict__ mu, const double* __restrict__ Nrm,
                            const double* __restrict__ q, double* __restrict__ rec) {
-    const int64_t a = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (a >= n) return;
+    const int64_t slot = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (slot >= n) return;
+    const int64_t a = perm ? perm[slot] : slot;
     const int64_t i = pi[a], j = pj[a];
     const Sym3 Ai = load_sym(A6 + 6 * i), Aj = load_sym(A6 + 6 * j);
     const double mui[3] = {mu[3 * i], mu[3 * i + 1], mu[3 * i + 2]};
@@ -405,7 +408,7 @@ __global__ void k_pair_rec(int64_t n, const int32_t* __restrict__ pi,
     Sym3 Ah;
     double P[3], KN;
     pair_quantities(Ai, Aj, mui, muj, Nrm[i], Nrm[j], &Ah, P, &KN);
-    double* r = rec + kRec * a;
+    double* r = rec + kRec * slot;
     r[0] = Ah.xx + Ah.yy + Ah.zz;
     r[1] = Ah.xx * Ah.yy + Ah.xx * Ah.zz + Ah.yy * Ah.zz - Ah.xy * Ah.xy - Ah.xz * Ah.xz
          - Ah.yz * Ah.yz;
@@ -1367,7 +1370,7 @@ __device__ void pair_reverse(int64_t n, int64_t a, int64_t i, int64_t j,
 // Per pair: sum the slab moments, map them to dE/dAh, dE/dPa, dE/dKN_a, then through
 // gs_dft/coulomb/stream.py:203-215 to the two splats. Writes J and the two splats' parts
 // (pair_reverse).
-// Slot `slot` (of n) holds pair a = perm[slot] (a = slot for a null perm; its record and slab moments are stored by slot,
+// Slot `slot` (of n) holds pair a = perm[slot] (its record and slab moments are stored by slot,
 // stride n); J and contrib are indexed by pair, stride nc. pref is the integral's prefactor
 // (2 pi^3/sqrt(pi) for (P|a), 2 pi for the nuclear attraction); a null weight treats every entry
 // as live.
@@ -1383,7 +1386,7 @@ __global__ void k_pair_finalize(int64_t n, int64_t nc, int64_t slabs, double pre
                                 const int64_t* __restrict__ n_live = nullptr) {
     const int64_t slot = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (slot >= (n_live ? *n_live : n)) return;       // n_live: a device count of real slots
-    const int64_t a = perm ? perm[slot] : slot;
+    const int64_t a = perm[slot];
     if (weight && weight[a] == 0.0) {
         J[a] = 0.0;
         zero_splat_parts(contrib, nc, a);
@@ -2678,8 +2681,8 @@ int launch_dC_list(int64_t M, int64_t k, int64_t n, const int32_t* row_ptr,
 }
 
 // Shared prologue of forward and reverse: chart, aux quantities (skipped for a null log_alpha),
-// pair density (zero for a null C), pair records in list order (w.rec; w.rec_sorted where the list
-// keeps its order).
+// pair density (zero for a null C), pair records: of a short list in slot order (w.rec_sorted, with
+// w.pair_order.perm), else in list order (w.rec).
 int gamma_prologue(int64_t M, const double* quat, const double* log_scale, const double* centers,
                    int64_t k, const double* C, const double* occ, int64_t N,
                    const double* log_alpha, int64_t n, const int32_t* pi, const int32_t* pj,
@@ -2696,14 +2699,17 @@ int gamma_prologue(int64_t M, const double* quat, const double* log_scale, const
             k_fill<<<blocks_for(n, 256), 256, 0, s>>>(n, 0.0, w.q);
             GSDFT_HIP(hipGetLastError());
         }
-        k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, pi, pj, w.A6, centers, w.Nrm, w.q,
-                                                      pair_list_order(n) ? w.rec_sorted : w.rec);
+        const bool list = pair_list_order(n);
+        if (list) GSDFT_TRY(launch_list_order(M, n, pi, w.pair_order, s));
+        k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, list ? w.pair_order.perm : nullptr, pi, pj,
+                                                      w.A6, centers, w.Nrm, w.q,
+                                                      list ? w.rec_sorted : w.rec);
         GSDFT_HIP(hipGetLastError());
     }
     return GSDFT_OK;
 }
 
-// The records in slot order (w.rec_sorted) and, unless the list keeps its order, w.pair_order.perm.
+// The records in slot order (w.rec_sorted) and w.pair_order.perm, after gamma_prologue.
 int sort_records(int64_t n, GammaWs& w, hipStream_t s) {
     if (pair_list_order(n)) return GSDFT_OK;
     GSDFT_TRY(launch_pair_order(n, w.rec, kRec, w.pair_order, s));
@@ -2712,12 +2718,6 @@ int sort_records(int64_t n, GammaWs& w, hipStream_t s) {
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
 }
-
-// Slot -> pair, null where they are the same.
-const int32_t* slot_perm(int64_t n, const GammaWs& w) {
-    return pair_list_order(n) ? nullptr : w.pair_order.perm;
-}
-
 
 }  // namespace
 
@@ -2809,7 +2809,8 @@ int exch_tc_prologue(int64_t M, const double* quat, const double* log_scale,
         k_fill<<<blocks_for(n, 256), 256, 0, s>>>(n, 1.0, w.q);
         GSDFT_HIP(hipGetLastError());
     }
-    k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, pi, pj, w.A6, centers, w.Nrm, w.q, w.rec);
+    k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, nullptr, pi, pj, w.A6, centers, w.Nrm, w.q,
+                                                  w.rec);
     GSDFT_HIP(hipGetLastError());
     const int64_t G = (N % M == 0) ? N / M : 1;
     if (exch_shares(w)) {
@@ -3702,7 +3703,7 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
         }
         profile_end(kProfGammaBwd, s);
         k_pair_finalize<<<blocks_for(n, 256), 256, 0, s>>>(n, n, 1, kPref3c,
-                                                           slot_perm(n, w), pi, pj, weight,
+                                                           w.pair_order.perm, pi, pj, weight,
                                                            w.A6, centers, w.Nrm, w.rec_sorted,
                                                            w.acc, J, w.contrib);
         GSDFT_HIP(hipGetLastError());
@@ -3793,7 +3794,7 @@ int external_pass(int64_t M, const double* quat, const double* log_scale, const 
     profile_end(kProfNucPairs, s);
     GSDFT_HIP(hipGetLastError());
     k_pair_finalize<<<blocks_for(n, 256), 256, 0, s>>>(n, n, sp.slabs, kPrefNuc,
-                                                       slot_perm(n, w.g), pi, pj, weight,
+                                                       w.g.pair_order.perm, pi, pj, weight,
                                                        w.g.A6, centers, w.g.Nrm, w.g.rec_sorted,
                                                        w.g.acc, V, w.g.contrib);
     GSDFT_HIP(hipGetLastError());
@@ -4082,9 +4083,14 @@ int exact_run(int64_t M, const double* quat, const double* log_scale, const doub
     } else {
         GSDFT_TRY(launch_pair_density(n, pi, pj, weight, den.k, den.C, den.occ, w.q, s));
     }
-    k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, pi, pj, w.A6, centers, w.Nrm, w.q, w.rec3);
-    GSDFT_HIP(hipGetLastError());
-    GSDFT_TRY(launch_pair_order(n, w.rec3, kRec, w.order, s));
+    if (pair_list_order(n)) {
+        GSDFT_TRY(launch_list_order(M, n, pi, w.order, s));
+    } else {
+        k_pair_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, nullptr, pi, pj, w.A6, centers, w.Nrm, w.q,
+                                                      w.rec3);
+        GSDFT_HIP(hipGetLastError());
+        GSDFT_TRY(launch_pair_order(n, w.rec3, kRec, w.order, s));
+    }
     k_eri_rec<<<blocks_for(n, 256), 256, 0, s>>>(n, w.order.perm, pi, pj, w.A6, centers, w.Nrm,
                                                  w.q, weight, w.rec);
     GSDFT_HIP(hipGetLastError());

@@ -141,8 +141,10 @@ struct PairOrderWs {
     size_t sort_bytes;
 };
 int pair_order_layout(Arena& ar, int64_t n, PairOrderWs* w);
-// Whether launch_pair_order leaves a list of n pairs in its own order (perm[slot] = slot).
+// Whether a list of n pairs is short: launch_pair_order leaves it in its own order (perm[slot] = slot);
+// launch_list_order does where it runs over i in ascending order, and else brings it into that.
 bool pair_list_order(int64_t n);
+int launch_list_order(int64_t M, int64_t n, const int32_t* pi, const PairOrderWs& w, hipStream_t s);
 // With n_live (a device count), only the first *n_live records are real: the rest take the slots
 // after them.
 int launch_pair_order(int64_t n, const double* rec, int rec_stride, const PairOrderWs& w,

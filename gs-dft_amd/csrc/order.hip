@@ -1,13 +1,13 @@
 // Slot order of the pairs in the three-centre passes (one lane per pair slot).
 //
-// Pairs are sorted by a band of I3/I2 (a factor sqrt(2) in the pair precision's smallest
+// Pairs of long lists are sorted by a band of I3/I2 (a factor sqrt(2) in the pair precision's smallest
 // eigenvalue scale) and then by the Morton code of the product centre on a 0.5-Bohr grid (+-256
 // Bohr, clamped), so that the 64 pairs of a wave are close in space and in width and the node
 // screen fires for whole waves (on the 700-atom globule, a simulation of the screen puts the nodes
 // evaluated at 44.8% of all with these bands, 45.9% with bands of a factor 4, 48.6% in list order;
 // the per-lane floor is 40.6%). The order only decides which pairs share a wave: each pair's sums
 // run over the aux records in the same sequence whatever its slot. A stable radix sort of 36-bit
-// keys makes the order a pure function of the inputs.
+// keys makes the order a pure function of the inputs. Short lists run over ascending i (kListOrderMax).
 #include <hipcub/hipcub.hpp>
 
 #include "common.h"
@@ -54,16 +54,112 @@ __global__ void k_pair_keys(int64_t n, const int64_t* __restrict__ n_live,
     key[a] = ((uint64_t)band << 30) | code;
 }
 
-// Lists of up to kListOrderMax pairs keep their own order: it already runs over neighbouring splats
-// (a list from neighbor_pairs is sorted), and on a short list the sort's launches cost more than the
-// nodes its order saves, also where the splats are spread out (DF-J steps in us, sorted / list
-// order: 7.9 k pairs of a compact molecule 415 / 354, 17 k 846 / 756, 37 k 1814 / 1723; an alkane
-// chain of 50 Bohr 639 / 551, 1541 / 1421 and, at 55 k pairs, 3925 / 3745).
+// A list of up to kListOrderMax pairs that runs over i in ascending order (one from neighbor_pairs
+// does) keeps its own order: it already runs over neighbouring splats, and on a short list the
+// sort's launches cost more than the nodes its order saves, also where the splats are spread out
+// (DF-J steps in us, sorted / list order: 7.9 k pairs of a compact molecule 415 / 354, 17 k 846 /
+// 756, 37 k 1814 / 1723; an alkane chain of 50 Bohr 639 / 551, 1541 / 1421 and, at 55 k pairs, 3925 /
+// 3745).
 constexpr int64_t kListOrderMax = 65536;
 
 __global__ void k_list_order(int64_t n, int32_t* __restrict__ perm) {
     const int64_t a = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (a < n) perm[a] = (int32_t)a;
+}
+
+// A short list in another order is brought into ascending i, each i's entries in list order, by one
+// workgroup: a stable counting sort over `passes` digits of i, its sixteen waves a contiguous part
+// each, 64 entries at a time ranked among their equals by ballots. Up to one descent in kRunLength
+// entries leaves a wave with a few runs, and the list as it is. It is launched either way, as the
+// host does not read the list: 3 us where there is nothing to do (the 350 us step of 7.9 k pairs is
+// 10 us longer for its two), 0.12 ms for 54 k shuffled pairs. That chain's step, shuffled, takes 3.70
+// ms; 4.28 in the order of the list and 3.43 if that is ascending.
+constexpr int kRunLength = 32;
+constexpr int kDigitBits = 10;         // 64 KB of counts
+constexpr int kPlaceWaves = 16;
+constexpr int kPlaceAhead = 4;         // steps whose entries a wave loads together
+
+__global__ __launch_bounds__(64 * kPlaceWaves) void k_list_place(int n, int passes,
+                                                                 const int32_t* __restrict__ pi,
+                                                                 int32_t* other, int32_t* rank,
+                                                                 int32_t* perm) {
+    constexpr int kDigits = 1 << kDigitBits, kThreads = 64 * kPlaceWaves;
+    static_assert(kDigits == kThreads, "a thread per digit");
+    __shared__ int at[kPlaceWaves][kDigits];      // a wave's counts, then where its digits start
+    __shared__ int sum[kDigits], drops;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (tid == 0) drops = 0;
+    __syncthreads();
+    int d = 0;
+#pragma unroll 8
+    for (int a = tid; a < n; a += kThreads) d += pi[a] < pi[a > 0 ? a - 1 : 0] ? 1 : 0;
+    if (d) atomicAdd(&drops, d);
+    __syncthreads();
+    if ((int64_t)drops * kRunLength <= n) {                               // workgroup-uniform
+#pragma unroll 8
+        for (int a = tid; a < n; a += kThreads) perm[a] = a;
+        return;
+    }
+    const int part = (n + kPlaceWaves - 1) / kPlaceWaves;
+    const int a0 = min(n, wave * part), a1 = min(n, a0 + part);
+    const uint64_t below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+    for (int p = 0; p < passes; ++p) {
+        const bool last = (passes - 1 - p) % 2 == 0;
+        const int32_t* src = p == 0 ? nullptr : last ? other : perm;      // null: the list itself
+        int32_t* dst = last ? perm : other;
+        // body(position, entry, its digit) for kPlaceAhead entries of the lane (positions past the
+        // part: its last entry again)
+        auto walk = [&](auto body) {
+            for (int a = a0; a < a1; a += 64 * kPlaceAhead) {             // wave-uniform
+                int e[kPlaceAhead], g[kPlaceAhead];
+#pragma unroll
+                for (int u = 0; u < kPlaceAhead; ++u) {
+                    const int x = min(a + 64 * u + lane, a1 - 1);
+                    e[u] = src ? src[x] : x;
+                }
+#pragma unroll
+                for (int u = 0; u < kPlaceAhead; ++u)
+                    g[u] = (int)((uint32_t)pi[e[u]] >> (kDigitBits * p)) & (kDigits - 1);
+#pragma unroll
+                for (int u = 0; u < kPlaceAhead; ++u) body(a + 64 * u + lane, e[u], g[u]);
+            }
+        };
+        for (int x = lane; x < kDigits; x += 64) at[wave][x] = 0;
+        walk([&](int x, int, int g) {             // each entry's place among its wave's equals
+            const bool in = x < a1;
+            uint64_t same = __ballot(in);
+#pragma unroll
+            for (int b = 0; b < kDigitBits; ++b) {
+                const uint64_t set = __ballot(g >> b & 1);
+                same &= (g >> b & 1) ? set : ~set;
+            }
+            if (!in) return;
+            const int first = at[wave][g];
+            rank[x] = first + __popcll(same & below);
+            if ((same & below) == 0) at[wave][g] = first + __popcll(same);
+        });
+        __syncthreads();
+        int total = 0;
+        for (int w = 0; w < kPlaceWaves; ++w) {
+            const int c = at[w][tid];
+            at[w][tid] = total;
+            total += c;
+        }
+        sum[tid] = total;
+        __syncthreads();
+        for (int off = 1; off < kDigits; off <<= 1) {
+            const int v = tid >= off ? sum[tid - off] : 0;
+            __syncthreads();
+            sum[tid] += v;
+            __syncthreads();
+        }
+        for (int w = 0; w < kPlaceWaves; ++w) at[w][tid] += sum[tid] - total;
+        __syncthreads();
+        walk([&](int x, int e, int g) {
+            if (x < a1) dst[at[wave][g] + rank[x]] = e;
+        });
+        __syncthreads();
+    }
 }
 
 // Group key of list entry p: min(i, j) M + max(i, j) for a live entry (the two orders of a splat
@@ -120,6 +216,17 @@ inline int bit_length(uint64_t v) { return v == 0 ? 1 : 64 - __builtin_clzll(v);
 }  // namespace
 
 bool pair_list_order(int64_t n) { return n <= kListOrderMax; }
+
+int launch_list_order(int64_t M, int64_t n, const int32_t* pi, const PairOrderWs& w,
+                      hipStream_t s) {
+    if (n <= 0) return GSDFT_OK;
+    if (!pair_list_order(n)) return fail(GSDFT_ERR_ARG, "list order: %lld pairs", (long long)n);
+    const int passes = (bit_length((uint64_t)(M > 1 ? M - 1 : 1)) + kDigitBits - 1) / kDigitBits;
+    k_list_place<<<1, 64 * kPlaceWaves, 0, s>>>((int)n, passes, pi, w.idx_in,
+                                                reinterpret_cast<int32_t*>(w.key_in), w.perm);
+    GSDFT_HIP(hipGetLastError());
+    return GSDFT_OK;
+}
 
 size_t pair_groups_scan_bytes(int64_t n) {
     size_t b = 0;
