@@ -205,9 +205,11 @@ def main() -> int:
     bwd_tf = integrals * FLOPS_BWD / (bwd_ms * 1e-3)
     # What the kernels executed: the node screen leaves out nodes whose terms are below e^-36, and
     # from 32768 pairs on the exponent scales of a centre share one node list (its centre terms
-    # once, each forward node added to every scale's sum).
+    # once, each forward node added to every scale's sum; in the reverse with two scales and
+    # multiples of four only).
     scales = min(len(s.scales), 4) if n >= 32768 else 1
-    fwd_share, bwd_share = (scales if scales > 2 else 1), scales
+    fwd_share = scales if scales > 2 else 1
+    bwd_share = scales if len(s.scales) == 2 or len(s.scales) % 4 == 0 else 1
     fwd_fixed, bwd_fixed = FWD_PER_INTEGRAL / fwd_share, BWD_PER_INTEGRAL / bwd_share
     fwd_node = FWD_PER_NODE + 2 * (fwd_share - 1)
     fwd_exec_tf = (integrals * fwd_fixed + fwd_nodes * fwd_node) / (fwd_ms * 1e-3)

@@ -2542,13 +2542,16 @@ int64_t bwd_slabs_per_launch(int64_t N, int64_t n) {
     return r < sp.slabs ? r : sp.slabs;
 }
 
-// Whether a DF-J pass takes the shared node lists (nodeset.hip). Choosing them costs ~0.15 ms, or
-// 0.25 us a centre, which a centre's nodes saved earn back from ~32,000 pairs on (four scales, step
-// in ms, plain / shared: 17 k pairs 0.93 / 0.98, 37 k 2.02 / 1.87, 167 k 16.1 / 11.8, 590 k 117 /
-// 93; 7.9 k 0.48 / 0.64). One scale leaves 18 of 20 nodes, less than the loop over a list costs
-// (2203 functions, 560 k pairs: 78.9 / 79.2); two leave 32 of 40, of use to the reverse only,
+// Whether a DF-J pass takes the shared node lists (nodeset.hip), if they fit its workspace. Choosing
+// them costs ~0.15 ms, or 0.25 us a centre, which a centre's nodes saved earn back from ~32,000 pairs on
+// (four scales, step in ms, plain / shared: 17 k pairs 0.93 / 0.98, 37 k 2.02 / 1.87, 167 k 16.1 / 11.8,
+// 590 k 117 / 93; 7.9 k 0.48 / 0.64). One scale leaves 18 of 20 nodes, less than the loop over a list
+// costs (2203 functions, 560 k pairs: 78.9 / 79.2); two leave 32 of 40, of use to the reverse only,
 // whose node costs no more for a second function (gamma 9.69 / 9.77 ms; step of 17 k pairs 1.845 /
 // 1.785).
+// The reverse keeps its lists in the aux records' place, 88 doubles a function. Two scales and
+// multiples of four take 84; a ragged group is stored as four functions, 336 doubles, so that 3, 5,
+// 6 or 7 scales do not fit and the reverse walks plain records there.
 constexpr int64_t kSetMinPairs = 32768;
 constexpr int64_t kSetSlack = 16;       // the passes read two nodes past a list
 inline bool use_node_sets(int64_t n, int64_t G, bool reverse) {
@@ -3675,7 +3678,8 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
             GSDFT_HIP(hipGetLastError());
         }
         GSDFT_TRY(sort_records(n, w, s));
-        // the slabs of groups that hold bwd_split_records' records: never more slabs than those
+        // the slabs of groups that hold bwd_split_records' records; the launches below are cut to the
+        // slabs that the moments' storage holds, whatever their count
         Split sp = bwd_split_records(N, n);
         if (sets) {
             sp.per_slab = (sp.per_slab + ns.nb - 1) / ns.nb;

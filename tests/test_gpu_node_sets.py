@@ -2,7 +2,8 @@
 per centre): gamma and its reverse pass against the oracle's twenty nodes per function.
 
 The cases are the forms the lists can take: 2 to 6 scales per centre (groups of four, the last one
-ragged), exponents over six decades, aux far from every pair, and aux whose functions do not share
+ragged; gamma shares nodes from three scales on, the reverse with two and with multiples of four:
+test_route), exponents over six decades, aux far from every pair, and aux whose functions do not share
 a centre although their count is a multiple of the splats' (every function then keeps its own nodes).
 One list is a single pair short, so it takes the plain records.
 
@@ -216,3 +217,32 @@ def test_exchange_groups_without_a_common_centre(g, wl, cuda, which):
         errs = [rel_max(a, b) for a, b in zip(got, out[0])]
         print(f"[sets] exchange, {which} apart: " + " ".join(f"{e:.1e}" for e in errs), flush=True)
         assert errs[0] < 1e-10 and max(errs[1:]) < 1e-9
+
+
+@pytest.mark.parametrize("name,forward,reverse", [("two", False, True), ("three", True, False),
+                                                  ("four", True, True), ("five", True, False),
+                                                  ("six", True, False), ("short", False, False)])
+def test_route(g, wl, cuda, name, forward, reverse):
+    """Which scale counts share nodes, by the nodes each pass evaluates: plain records take all twenty of
+    a function here (the system is compact: the screen leaves out 2%), shared lists of two scales nine
+    tenths of them (18 a function), of more scales fewer."""
+    from gs_dft_amd import _lib
+    s, la, ac, i, j, w = _case(wl, name)
+    ids = (_lib.PROF_GAMMA_FWD, _lib.PROF_GAMMA_BWD)
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    basis = g.Splat(quat=t(s.quat), log_scale=t(s.log_scale), centers=t(s.centers))
+    _lib.profile_enable(True)
+    try:
+        for kid in ids:
+            _lib.profile_read_work(kid, reset=True)
+        gam = g.df_coulomb_gamma_screened(basis, t(s.C), s.occ,
+                                          g.IsotropicSplat(log_alpha=la, centers=ac),
+                                          torch.tensor(i), torch.tensor(j), valid=torch.tensor(w))
+        gam.sum().backward()
+        torch.cuda.synchronize()
+        part = [_lib.profile_read_work(kid, reset=True) / (20.0 * len(la) * len(i)) for kid in ids]
+    finally:
+        _lib.profile_enable(False)
+    print(f"[sets] {name}: of all nodes, forward {part[0]:.3f}, reverse {part[1]:.3f}", flush=True)
+    for x, shared in zip(part, (forward, reverse)):
+        assert x < 0.93 if shared else x > 0.96
