@@ -42,6 +42,13 @@ constexpr int kAuxRec = 88;   // doubles per aux record of the reverse pass
 constexpr int kAcc = 25;      // cotangent moments per pair
 
 inline unsigned blocks_for(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
+// Blocks of 256 threads for work that can pass the 2^32 - 1 work-items of one grid dimension, block
+// (x, y) taking the items from 256 (y gridDim.x + x) on.
+inline dim3 blocks_2d(int64_t items) {
+    const int64_t blocks = (items + 255) / 256, row = std::min<int64_t>(std::max<int64_t>(blocks, 1),
+                                                                        1 << 23);
+    return dim3((unsigned)row, (unsigned)((blocks + row - 1) / row));
+}
 // Blocks in the y or z dimension of a grid (the x dimension is bounded by its 2^32 - 1 work-items).
 constexpr int64_t kMaxGridY = 65535;
 
@@ -919,7 +926,7 @@ __global__ void k_aux_bwd_prep(int64_t N, int64_t G, const double* __restrict__ 
                                const double* __restrict__ dgamma,
                                const double* __restrict__ dscale, int fold, NodeTable tb,
                                double* __restrict__ out) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int64_t i = (blockIdx.y * (int64_t)gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;
     const int64_t p = i / kNodes;
     const int t = (int)(i % kNodes);
     if (p >= N) return;
@@ -2821,8 +2828,8 @@ int exch_tc_prologue(int64_t M, const double* quat, const double* log_scale,
         GSDFT_TRY(launch_node_sets(N, G, kSetExchange, w.beta, w.kn, aux_centers, nullptr, nullptr,
                                    w.box, w.sets, s));
     } else {
-        k_aux_bwd_prep<<<blocks_for(N * kNodes, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
-                                                          nullptr, kAuxPlain, w.table, w.aux);
+        k_aux_bwd_prep<<<blocks_2d(N * kNodes), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
+                                                             nullptr, kAuxPlain, w.table, w.aux);
         GSDFT_HIP(hipGetLastError());
     }
     // one record per group (its first entry's), then the groups' slot order: the group count
@@ -3541,9 +3548,9 @@ int gamma_run(int64_t M, const double* quat, const double* log_scale, const doub
         GSDFT_TRY(launch_pair_box(n, nullptr, pair_list_order(n) ? w.rec_sorted : w.rec, kRec,
                                   w.q, s));
     } else {
-        k_aux_bwd_prep<<<blocks_for(N * kNodes, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
-                                                          nullptr, kAuxForward, coulomb_table(),
-                                                          w.aux);
+        k_aux_bwd_prep<<<blocks_2d(N * kNodes), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
+                                                             nullptr, kAuxForward,
+                                                             coulomb_table(), w.aux);
         GSDFT_HIP(hipGetLastError());
     }
     GSDFT_TRY(sort_records(n, w, s));
@@ -3672,9 +3679,9 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
             GSDFT_TRY(launch_node_sets(N, G, kSetFold, w.beta, w.kn, aux_centers, dgamma, dgamma_scale,
                                        w.q, w.aux, s));
         } else {
-            k_aux_bwd_prep<<<blocks_for(N * kNodes, 256), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers,
-                                                              dgamma, dgamma_scale, kAuxFoldU,
-                                                              coulomb_table(), w.aux);
+            k_aux_bwd_prep<<<blocks_2d(N * kNodes), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers,
+                                                                 dgamma, dgamma_scale, kAuxFoldU,
+                                                                 coulomb_table(), w.aux);
             GSDFT_HIP(hipGetLastError());
         }
         GSDFT_TRY(sort_records(n, w, s));

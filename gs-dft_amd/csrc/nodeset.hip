@@ -22,6 +22,8 @@
 // Every product Gaussian is, in turn, an average of isotropic Gaussians of exponent l >= its largest
 // eigenvalue, so the matrix is formed for those (s -> s l / (l + s), weights (l / (l + s))^(3/2), u the
 // squared distance to their centres), which takes a node or two fewer where b > l.
+#include <algorithm>
+
 #include "common.h"
 #include "internal.h"
 
@@ -125,7 +127,8 @@ __device__ __forceinline__ double pivot_key(double v, uint32_t index) {
 // three workgroups to a CU overlap them.
 template <int NB>
 __global__ __launch_bounds__(kSetThreads) void k_node_sets(
-    int64_t N, int64_t G, int64_t per_centre, int64_t stride, const double* __restrict__ beta,
+    int64_t N, int64_t G, int64_t per_centre, int64_t groups, int64_t stride,
+    const double* __restrict__ beta,
     const double* __restrict__ kn, const double* __restrict__ R,
     const double* __restrict__ dgamma, const double* __restrict__ dscale, SetForm form,
     const double* __restrict__ box, NodeTable tb, double* __restrict__ out) {
@@ -144,7 +147,8 @@ __global__ __launch_bounds__(kSetThreads) void k_node_sets(
     __shared__ double wavekey[2][kSetThreads / 64];
     __shared__ int piv[kMaxRank];
     const int tid = threadIdx.x;
-    const int64_t group = blockIdx.x;
+    const int64_t group = blockIdx.y * (int64_t)gridDim.x + blockIdx.x;
+    if (group >= groups) return;                                       // workgroup-uniform
     int64_t slot0;
     const int nb = set_group(group, G, per_centre, &slot0);
     double* o = out + stride * group;
@@ -382,14 +386,16 @@ int launch_node_sets(int64_t N, int64_t G, SetForm form, const double* beta, con
                      const double* R, const double* dgamma, const double* dscale,
                      const double* box, double* out, hipStream_t s) {
     const NodeSets ns = node_sets(N, G, form);
-    const unsigned g = (unsigned)ns.groups;
+    // groups in two dimensions: one holds at most 2^32 - 1 work-items, 13.4 million groups
+    const int64_t row = std::min<int64_t>(std::max<int64_t>(ns.groups, 1), 1 << 20);
+    const dim3 g((unsigned)row, (unsigned)((ns.groups + row - 1) / row));
     const NodeTable tb = coulomb_table();
     if (ns.nb == 2)
-        k_node_sets<2><<<g, kSetThreads, 0, s>>>(N, G, ns.per_centre, ns.stride, beta, kn, R,
-                                                 dgamma, dscale, form, box, tb, out);
+        k_node_sets<2><<<g, kSetThreads, 0, s>>>(N, G, ns.per_centre, ns.groups, ns.stride, beta, kn,
+                                                 R, dgamma, dscale, form, box, tb, out);
     else
-        k_node_sets<4><<<g, kSetThreads, 0, s>>>(N, G, ns.per_centre, ns.stride, beta, kn, R,
-                                                 dgamma, dscale, form, box, tb, out);
+        k_node_sets<4><<<g, kSetThreads, 0, s>>>(N, G, ns.per_centre, ns.groups, ns.stride, beta, kn,
+                                                 R, dgamma, dscale, form, box, tb, out);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;
 }

@@ -246,3 +246,31 @@ def test_route(g, wl, cuda, name, forward, reverse):
     print(f"[sets] {name}: of all nodes, forward {part[0]:.3f}, reverse {part[1]:.3f}", flush=True)
     for x, shared in zip(part, (forward, reverse)):
         assert x < 0.93 if shared else x > 0.96
+
+
+def test_more_groups_than_one_grid_dimension_holds(g, cuda):
+    """13.43 million centres of two functions: their lists' workgroups pass 2^32 work-items, which
+    wraps a one-dimensional launch. J = sum_P v_P (P|a), all terms positive, against the plain records
+    (a list of 64 pairs)."""
+    from gs_dft_amd import ri
+    M, n = 13_430_000, N_MIN
+    assert M * 320 > 2 ** 32
+    gen = torch.Generator("cuda").manual_seed(5)
+    f8 = dict(device="cuda", dtype=torch.float64)
+    centers = torch.randn(M, 3, generator=gen, **f8) * 2.0
+    basis = g.Splat(quat=torch.randn(M, 4, generator=gen, **f8),
+                    log_scale=torch.randn(M, 3, generator=gen, **f8) * 0.3 - 1.0, centers=centers)
+    la = torch.rand(M, generator=gen, **f8)
+    aux = g.IsotropicSplat(log_alpha=torch.cat([la, la + 1.0]), centers=torch.cat([centers, centers]))
+    i = torch.arange(n, dtype=torch.int32, device="cuda") * 400
+    w = torch.ones(n, **f8)
+    v = torch.rand(2 * M, generator=gen, **f8) + 0.5
+    out = []
+    for m in (64, n):
+        x = ri._Inputs(basis, torch.ones(M, 1, **f8), torch.ones(1, **f8), aux, i[:m], i[:m] + 1,
+                       w[:m], None)
+        print(f"[sets] {2 * M} functions, {m} pairs", flush=True)
+        out.append(ri._gamma_vjp(x, v, None)[0].cpu().numpy())
+        del x
+        torch.cuda.empty_cache()
+    assert np.all(np.abs(out[1][:64] - out[0]) <= 1e-12 * np.abs(out[0]))
