@@ -93,3 +93,86 @@ def test_shuffled_list_of_few_and_many_splats(g, cuda, M, n):
            for o in (np.arange(n), mix)]
     print(f"[order] M={M} n={n}: {rel_max(out[1], out[0]):.1e}", flush=True)
     assert rel_max(out[1], out[0]) < 1e-12
+
+
+def _repeated(M, n, rng):
+    """Every ordered pair of M splats, over and over, shuffled; some entries dead."""
+    a = rng.permutation(np.arange(n) % (M * M))
+    w = rng.uniform(0.5, 2.0, n)
+    w[::7] = 0.0
+    w[-1] = 1.0
+    return (a // M).astype(np.int32), (a % M).astype(np.int32), w
+
+
+@pytest.mark.parametrize("n", [65536, 65537, 70001])
+def test_long_list_against_oracle(g, wl, orc, cuda, n):
+    """Both sides of the length from which lists are sorted, shared node lists in both passes."""
+    s = wl.make_small(30, 6, n_atoms=4, seed=11, spread=4.0)
+    rng = np.random.default_rng(n)
+    i, j, w = _repeated(s.M, n, rng)
+    la = (np.log(rng.uniform(0.1, 12.0, s.M))[None] + np.log(np.geomspace(0.5, 4.0, 4))[:, None])
+    ac = np.tile(s.centers + rng.normal(0.0, 0.2, (s.M, 3)), (4, 1))
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    basis = g.Splat(quat=t(s.quat), log_scale=t(s.log_scale), centers=t(s.centers))
+    C = t(s.C)
+    gam = g.df_coulomb_gamma_screened(basis, C, s.occ,
+                                      g.IsotropicSplat(log_alpha=la.ravel(), centers=ac),
+                                      torch.tensor(i), torch.tensor(j), valid=torch.tensor(w))
+    v = rng.normal(size=la.size)
+    got = torch.autograd.grad(gam, [basis.quat, basis.log_scale, basis.centers, C],
+                              torch.tensor(v, device="cuda"))
+    ref = orc.gamma(s.quat, s.log_scale, s.centers, s.C, s.occ, la.ravel(), ac, i, j, w)
+    back = orc.gamma_vjp(s.quat, s.log_scale, s.centers, s.C, s.occ, la.ravel(), ac, i, j, w, v)
+    errs = [rel_max(gam.detach().cpu().numpy(), ref)] + [rel_max(a.cpu().numpy(), b)
+                                                         for a, b in zip(got, back[-4:])]
+    print(f"[order] oracle n={n}: " + " ".join(f"{e:.1e}" for e in errs), flush=True)
+    assert errs[0] < 1e-12 and max(errs[1:]) < 1e-9
+
+
+@pytest.mark.parametrize("n", [65536, 70001])
+def test_nuclear_gradients_on_a_long_list(g, wl, tr, cuda, n):
+    s = wl.make_small(24, 5, n_atoms=4, seed=6)
+    rng = np.random.default_rng(n)
+    i, j, w = _repeated(s.M, n, rng)
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    basis = g.Splat(quat=t(s.quat), log_scale=t(s.log_scale), centers=t(s.centers))
+    C, R = t(s.C), t(np.asarray(s.atoms))
+    E = g.screened_external_energy(basis, C, s.occ, torch.tensor(i), torch.tensor(j), R, s.charges,
+                                   valid=torch.tensor(w))
+    got = torch.autograd.grad(E, [basis.quat, basis.log_scale, basis.centers, C, R])
+    # the oracle on the distinct pairs, their weights added
+    W = np.zeros(s.M * s.M)
+    np.add.at(W, i.astype(np.int64) * s.M + j, w)
+    p, q = (torch.as_tensor(a) for a in np.divmod(np.arange(s.M * s.M), s.M))
+    c = lambda a: torch.tensor(np.asarray(a), dtype=torch.float64)
+    ref = [c(a).requires_grad_() for a in (s.quat, s.log_scale, s.centers, s.C, s.atoms)]
+    Er = tr.screened_external_energy(*ref[:4], c(s.occ), p, q, c(W), ref[4], c(s.charges))
+    want = torch.autograd.grad(Er, ref)
+    errs = [abs(E.item() / Er.item() - 1)] + [rel_max(a.cpu().numpy(), b.numpy())
+                                              for a, b in zip(got, want)]
+    print(f"[order] nuclear n={n}: " + " ".join(f"{e:.1e}" for e in errs), flush=True)
+    assert errs[0] < 1e-12 and max(errs[1:]) < 1e-9
+
+
+def test_exchange_on_shared_lists_of_a_sorted_list(g, wl, cuda):
+    """RI-K over 72,200 entries (every pair twice, shuffled), its groups in the sort's order: shared
+    node lists against plain records (an aux chunk of 66 cuts their groups), and against the same entries
+    in ascending order. lam = 1e-2 keeps the metric's condition near 1e4, as in test_gpu_node_sets.py."""
+    s = wl.make_small(190, 5, n_atoms=6, seed=4, spread=3.0)
+    t = lambda a: torch.tensor(a, device="cuda").requires_grad_()
+    basis = g.Splat(quat=t(s.quat), log_scale=t(s.log_scale), centers=t(s.centers))
+    C = t(s.C)
+    aux = g.init_product_aux(basis, scales=(0.5, 1.0, 2.0, 4.0))
+    L = g.aux_cholesky(aux, 1e-2)
+    a = np.arange(2 * s.M * s.M) % (s.M * s.M)
+    out = []
+    for order, chunk in ((np.random.default_rng(1).permutation(len(a)), 66),
+                         (np.random.default_rng(1).permutation(len(a)), 0), (np.argsort(a), 0)):
+        i, j = (torch.tensor(x.astype(np.int32)) for x in np.divmod(a[order], s.M))
+        E = g.df_exchange_energy_screened(basis, C, aux, i, j, cholV=L, aux_chunk=chunk)
+        out.append([E.detach().cpu().numpy()] + [x.cpu().numpy() for x in torch.autograd.grad(
+            E, [basis.quat, basis.log_scale, basis.centers, C])])
+    for got in out[1:]:
+        errs = [rel_max(x, y) for x, y in zip(got, out[0])]
+        print("[order] exchange: " + " ".join(f"{e:.1e}" for e in errs), flush=True)
+        assert errs[0] < 1e-10 and max(errs[1:]) < 1e-9
