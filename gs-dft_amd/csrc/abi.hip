@@ -22,8 +22,10 @@ std::vector<EventPair> g_open[kProfCount];     // recorded, not yet read
 std::vector<hipEvent_t> g_pending_start[kProfCount];
 double g_total_ms[kProfCount] = {0};
 int64_t g_launches[kProfCount] = {0};
-unsigned long long* g_work_dev = nullptr;   // kProfCount work counters on g_work_device
+unsigned long long* g_work_dev = nullptr;   // kProfCount x kWorkUnits on g_work_device
 int g_work_device = -1;
+constexpr int kWorkUnits = kWorkSlots * kWorkPad;
+constexpr size_t kWorkBytes = sizeof(unsigned long long) * kWorkUnits;
 }  // namespace
 
 int fail(int code, const char* fmt, ...) {
@@ -70,7 +72,7 @@ unsigned long long* profile_work_counter(int id) {
     if (!g_prof_on || !g_work_dev || id < 0 || id >= kProfCount) return nullptr;
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev != g_work_device) return nullptr;
-    return g_work_dev + id;
+    return g_work_dev + (size_t)kWorkUnits * id;
 }
 
 }  // namespace gsdft
@@ -86,8 +88,8 @@ extern "C" int gsdft_profile_enable(int on) {
     g_prof_on = on != 0;
     if (g_prof_on && !g_work_dev) {
         GSDFT_HIP(hipGetDevice(&g_work_device));
-        GSDFT_HIP(hipMalloc((void**)&g_work_dev, sizeof(unsigned long long) * kProfCount));
-        GSDFT_HIP(hipMemset(g_work_dev, 0, sizeof(unsigned long long) * kProfCount));
+        GSDFT_HIP(hipMalloc((void**)&g_work_dev, kWorkBytes * kProfCount));
+        GSDFT_HIP(hipMemset(g_work_dev, 0, kWorkBytes * kProfCount));
     }
     return GSDFT_OK;
 }
@@ -101,13 +103,14 @@ extern "C" int gsdft_profile_read_work(int id, uint64_t* units, int reset) {
     int dev = -1;
     GSDFT_HIP(hipGetDevice(&dev));
     GSDFT_HIP(hipSetDevice(g_work_device));
-    unsigned long long v = 0;
+    unsigned long long* const from = g_work_dev + (size_t)kWorkUnits * id;
+    std::vector<unsigned long long> v(kWorkUnits);
     hipError_t e = hipDeviceSynchronize();
-    if (e == hipSuccess) e = hipMemcpy(&v, g_work_dev + id, sizeof v, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && reset) e = hipMemset(g_work_dev + id, 0, sizeof v);
+    if (e == hipSuccess) e = hipMemcpy(v.data(), from, kWorkBytes, hipMemcpyDeviceToHost);
+    if (e == hipSuccess && reset) e = hipMemset(from, 0, kWorkBytes);
     (void)hipSetDevice(dev);
     if (e != hipSuccess) return hip_fail(e, "gsdft_profile_read_work");
-    *units = (uint64_t)v;
+    for (int i = 0; i < kWorkSlots; ++i) *units += v[(size_t)kWorkPad * i];
     return GSDFT_OK;
 }
 

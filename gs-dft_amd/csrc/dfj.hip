@@ -16,8 +16,8 @@
 // Work decomposition (no atomics anywhere):
 //   forward  -- one lane per pair slot; the wave walks a block's aux records (uniform node
 //               tables, centre-grouped so the centre terms are shared by the exponent scales);
-//               each lane keeps its partial sums per record in LDS, the block adds them in lane
-//               order, and the per-block partials are summed in fixed order.
+//               each lane keeps its partial sums per record in LDS, the block adds them in a
+//               fixed order, and the per-block partials are summed in fixed order.
 //   reverse  -- one lane per pair slot; the wave walks the aux records the same way, over slabs
 //               of records small enough to stay in L2; each lane accumulates its pair's 25
 //               cotangent moments per slab in registers; the slabs' moments are added in slab
@@ -449,6 +449,12 @@ __device__ __forceinline__ void node_const(double b, double t, double w, double*
 // bit-identical in double precision, and the z-weighted reverse terms move by <= 1.2e-15
 // relative. Checks follow every node from kFirstSkip on, before which z_t <= t^2 |d|^2 stays
 // small for any pair within ~30 Bohr.
+// On shared node lists (nodeset.hip) the loops test z after every second node, from the second on. A
+// list starts at the first node's s = t^2 ~ 1.2e-5 or the next ones' 3e-4, where z passes 36 from 1700 or
+// 330 Bohr on; before that a loop left early has taken every node that still counts. Its nodes stand
+// closer than a function's twenty, so the first one left out is just past 36 rather than well past it:
+// what is left out is at most 6e-16 of (P|a) up to 40 Bohr and 1.1e-15 at 150 (one lane alone, exponents
+// 0.05 to 20, eigenvalues 0.1 to 25; 9e-18 for the twenty).
 constexpr double kSkipZ = 36.0;
 constexpr int kFirstSkip = 5;
 
@@ -523,11 +529,17 @@ __device__ __forceinline__ uint32_t node_loop(Body& body) {
     }
 }
 
-// Profiling only: adds this wave's node evaluations over its live lanes to *work.
+// Profiling only: one wave's node evaluations, from its first lane, into one of the kernel's counters
+// (on one address the waves of the exchange block, 837 k a launch, queued up for 1.9 ms of its 6).
+__device__ __forceinline__ void add_work(unsigned long long* work, uint64_t nodes) {
+    atomicAdd(work + kWorkPad * (blockIdx.x % kWorkSlots), (unsigned long long)nodes);
+}
+
+// Profiling only: adds this wave's node evaluations over its live lanes.
 __device__ __forceinline__ void count_work(unsigned long long* work, bool live, uint32_t nodes) {
     if (!work) return;
     const uint64_t lanes = __builtin_popcountll(__builtin_amdgcn_ballot_w64(live));
-    if ((threadIdx.x & 63) == 0) atomicAdd(work, (unsigned long long)(lanes * nodes));
+    if ((threadIdx.x & 63) == 0) add_work(work, lanes * nodes);
 }
 
 // ------------------------------------------------------------------ forward
@@ -539,7 +551,7 @@ __device__ __forceinline__ void count_work(unsigned long long* work, bool live, 
 // their pair slots (read once into L2) and differ only in their aux records. (One dimension of a
 // grid holds at most 2^32 - 1 work-items: a 1-D grid of both would pass that at 20 M pairs.) The centre-dependent terms (d, Ah d, q0..q2)
 // are formed once per centre and shared by its exponent scales, and the wave's node screen acts on
-// 64 pairs in precision band + Morton order. Each lane keeps its running sums of coef_a F(P, a) for
+// 64 pairs of neighbouring slots (order.hip). Each lane keeps its running sums of coef_a F(P, a) for
 // the block's records in LDS; at the end the 256 lane sums of each record are added in a fixed
 // order and scaled by KN_P (the record's u): partial[g * N + slot]. Twelve records per block keep the
 // LDS at 26 KB, so six workgroups (six waves per SIMD, within the kernel's 60 registers) share a
@@ -662,7 +674,7 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_pairs(int64_t n, int64_t pair
             acc[j][threadIdx.x] = __builtin_fma(F, cf, acc[j][threadIdx.x]);
         }
     }
-    if (work && (threadIdx.x & 63) == 0) atomicAdd(work, (unsigned long long)lane_nodes);
+    if (work && (threadIdx.x & 63) == 0) add_work(work, lane_nodes);
     __syncthreads();
     // sixteen lanes per record: each adds sixteen of the 256 lane sums, then a butterfly
     static_assert(kFwdRecs <= 16, "one record per sixteen lanes of the block");
@@ -822,7 +834,7 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_sets(int64_t n, int64_t pairs
             } while (!last);
         }
     }
-    if (work && (threadIdx.x & 63) == 0) atomicAdd(work, (unsigned long long)lane_nodes);
+    if (work && (threadIdx.x & 63) == 0) add_work(work, lane_nodes);
     __syncthreads();
     const int j = threadIdx.x >> 4, part = threadIdx.x & 15;
     double sum = 0.0;
@@ -2354,7 +2366,7 @@ __global__ __launch_bounds__(256) void k_exch_block_pairs(int64_t n,
 // The same on shared node lists (nodeset.hip, kSetExchange) of four functions each: the sixteen
 // aux slots of a block are four groups, and each node is added to the four functions' sums with
 // the list's weights (KN_P folded in). C20H42: 51.8 -> 44.9 ms a step, the reverse on the same
-// lists 83.8 -> 70.4 ms (three waves per SIMD: 168 registers).
+// lists 83.8 -> 66 (three waves per SIMD: 150 registers).
 template <bool kPair>
 __global__ __launch_bounds__(256) void k_exch_block_sets(int64_t n, const double* __restrict__ rec,
                                                          const int32_t* __restrict__ perm,
@@ -2824,7 +2836,7 @@ int exch_tc_prologue(int64_t M, const double* quat, const double* log_scale,
     GSDFT_HIP(hipGetLastError());
     const int64_t G = (N % M == 0) ? N / M : 1;
     if (exch_shares(w)) {
-        GSDFT_TRY(launch_pair_box(n, nullptr, w.rec, kRec, w.box, s));
+        GSDFT_TRY(launch_pair_box(n, w.rec, kRec, w.box, s));
         GSDFT_TRY(launch_node_sets(N, G, kSetExchange, w.beta, w.kn, aux_centers, nullptr, nullptr,
                                    w.box, w.sets, s));
     } else {
@@ -3545,7 +3557,7 @@ int gamma_run(int64_t M, const double* quat, const double* log_scale, const doub
     const bool sets = use_node_sets(n, G, false) &&
                       ns.stride * ns.groups + kSetSlack + groups * N <= kRec * n;
     if (sets) {
-        GSDFT_TRY(launch_pair_box(n, nullptr, pair_list_order(n) ? w.rec_sorted : w.rec, kRec,
+        GSDFT_TRY(launch_pair_box(n, pair_list_order(n) ? w.rec_sorted : w.rec, kRec,
                                   w.q, s));
     } else {
         k_aux_bwd_prep<<<blocks_2d(N * kNodes), 256, 0, s>>>(N, G, w.beta, w.kn, aux_centers, nullptr,
@@ -3674,7 +3686,7 @@ extern "C" int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_
         const bool sets = use_node_sets(n, G, true) &&
                           ns.stride * ns.groups + kSetSlack <= kAuxRec * N + kAuxRec;
         if (sets) {
-            GSDFT_TRY(launch_pair_box(n, nullptr, pair_list_order(n) ? w.rec_sorted : w.rec, kRec,
+            GSDFT_TRY(launch_pair_box(n, pair_list_order(n) ? w.rec_sorted : w.rec, kRec,
                                   w.q, s));
             GSDFT_TRY(launch_node_sets(N, G, kSetFold, w.beta, w.kn, aux_centers, dgamma, dgamma_scale,
                                        w.q, w.aux, s));

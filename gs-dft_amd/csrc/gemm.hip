@@ -530,7 +530,7 @@ int launch_tiles(int64_t Mr, int64_t Nc, int64_t K, const double* A, int64_t lda
 // C20H42), and a 128-row tile then multiplies rows that are not there. Up to 256 rows the tile is
 // the one that pads least, the larger of equals; beyond that what 128 rows pad is below a third and
 // wider tiles read less. Grid step of C20H42 (81 orbitals: 96 rows in place of 128) 10.58 -> 9.60 ms,
-// of 700 splats with 30 orbitals 1.30 -> 0.94 ms, of 2600 with 150 (two tiles of 96) 15.2 -> 12.1;
+// of 700 splats with 30 orbitals 1.30 -> 0.94 ms, of 2600 with 150 (five tiles of 32) 15.2 -> 12.1;
 // RI-K of C20H42: the k-row products 20.8 -> 18.1 ms.
 inline int dma_row_tiles(int64_t Mr) {
     if (Mr > 2 * kTile) return 4;

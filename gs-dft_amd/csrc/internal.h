@@ -77,8 +77,10 @@ struct ProfileScope {
     ProfileScope(const ProfileScope&) = delete;
     ProfileScope& operator=(const ProfileScope&) = delete;
 };
-// Device counter of work units for kernel id while profiling is on (current device only), else
-// nullptr; kernels given a counter add their executed units to it.
+// Device counters of work units for kernel id while profiling is on (current device only), else
+// nullptr; kernels given them add their executed units to any of the kWorkSlots, kWorkPad apart (a
+// cache line each).
+constexpr int kWorkSlots = 64, kWorkPad = 16;
 unsigned long long* profile_work_counter(int id);
 enum ProfileId { kProfGammaFwd = 0, kProfGammaBwd = 1, kProfScreen = 2, kProfMetric = 3,
                  kProfCholesky = 4, kProfSolve = 5, kProfNucPairs = 6, kProfNucAtoms = 7,
@@ -161,12 +163,12 @@ int launch_pair_groups(int64_t M, int64_t n, const int32_t* pi, const int32_t* p
                        int32_t* grp_first, int32_t* grp_rep, int64_t* n_groups, hipStream_t s);
 
 // nodeset.hip: the reach and widths of n pair records (the first 12 doubles as for
-// launch_pair_order; n_live as there) into scratch[0..7], scratch holding node_set_box_doubles();
+// launch_pair_order) into scratch[0..7], scratch holding node_set_box_doubles();
 // and one node list per group of aux functions in the given form (layout: common.h; dgamma and
 // dscale are read for kSetFold only, whose weights carry dgamma_P dscale kn_P).
 size_t node_set_box_doubles();
-int launch_pair_box(int64_t n, const int64_t* n_live, const double* rec, int rec_stride,
-                    double* scratch, hipStream_t s);
+int launch_pair_box(int64_t n, const double* rec, int rec_stride, double* scratch,
+                    hipStream_t s);
 int launch_node_sets(int64_t N, int64_t G, SetForm form, const double* beta, const double* kn,
                      const double* R, const double* dgamma, const double* dscale,
                      const double* box, double* out, hipStream_t s);

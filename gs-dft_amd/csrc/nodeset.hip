@@ -68,15 +68,13 @@ __device__ __forceinline__ double wave_max(double v) {
 // Largest |P| coordinates and widths of the pair records: per block -min P (3), max P (3),
 // max I2/I3 (at least 1 / the smallest eigenvalue, the squared width), max I1 (at least the
 // largest eigenvalue).
-__global__ __launch_bounds__(256) void k_pair_box(int64_t n, const int64_t* __restrict__ n_live,
-                                                  const double* __restrict__ rec, int rec_stride,
-                                                  double* __restrict__ part) {
+__global__ __launch_bounds__(256) void k_pair_box(int64_t n, const double* __restrict__ rec,
+                                                  int rec_stride, double* __restrict__ part) {
     __shared__ double red[4][8];
-    const int64_t m = n_live ? *n_live : n;
     double v[8];
     for (int c = 0; c < 6; ++c) v[c] = -1e300;
     v[6] = v[7] = 0.0;
-    for (int64_t a = blockIdx.x * (int64_t)256 + threadIdx.x; a < m;
+    for (int64_t a = blockIdx.x * (int64_t)256 + threadIdx.x; a < n;
          a += (int64_t)gridDim.x * 256) {
         const double* r = rec + (int64_t)rec_stride * a;
         for (int c = 0; c < 3; ++c) {
@@ -374,9 +372,9 @@ __global__ __launch_bounds__(kSetThreads) void k_node_sets(
 
 size_t node_set_box_doubles() { return 8 * kBoxBlocks + 8; }
 
-int launch_pair_box(int64_t n, const int64_t* n_live, const double* rec, int rec_stride,
-                    double* scratch, hipStream_t s) {
-    k_pair_box<<<kBoxBlocks, 256, 0, s>>>(n, n_live, rec, rec_stride, scratch + 8);
+int launch_pair_box(int64_t n, const double* rec, int rec_stride, double* scratch,
+                    hipStream_t s) {
+    k_pair_box<<<kBoxBlocks, 256, 0, s>>>(n, rec, rec_stride, scratch + 8);
     k_pair_box_finish<<<1, 64, 0, s>>>(kBoxBlocks, scratch + 8, scratch);
     GSDFT_HIP(hipGetLastError());
     return GSDFT_OK;

@@ -340,7 +340,7 @@ int gsdft_exchange(int64_t M, const double* quat, const double* log_scale, const
  * milliseconds and the launch count since the last reset. gsdft_profile_read_work returns the
  * work units the kernels executed while profiling was on (ids 0, 1, 6-11: quadrature nodes
  * evaluated, summed over live lanes, so at most 20 x (aux functions, nuclei or pairs) x pairs
- * per launch; other ids: 0). Profiling allocates a few bytes of device memory on the device
+ * per launch; other ids: 0). Profiling allocates 120 KiB of device memory on the device
  * current when it is first enabled. */
 int gsdft_profile_enable(int on);
 int gsdft_profile_read(int id, double* total_ms, int64_t* launches, int reset);
