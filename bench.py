@@ -221,22 +221,27 @@ def main() -> int:
         f"{100 * fwd_node_frac:.1f}% of nodes), bwd {bwd_ms:.1f} ms ({bwd_tf / 1e12:.2f} / "
         f"{bwd_exec_tf / 1e12:.2f} TFLOP/s, {100 * bwd_node_frac:.1f}% of nodes), "
         f"solves {solve_ms / max(args.steps, 1):.2f} ms")
+    # the kernel that ran, as profiles/*.json name it: a counter run of another one says nothing here
+    fwd_kernel = "k_gamma_fwd_sets" if fwd_share > 1 else "k_gamma_fwd_pairs"
+    bwd_kernel = "k_gamma_bwd_sets" if bwd_share > 1 else "k_gamma_bwd"
     if bwd_ms >= fwd_ms:
-        dom = ("reverse", "k_gamma_bwd", bwd_ms, FLOPS_BWD, bwd_tf, bwd_exec_tf, bwd_node_frac,
+        dom = ("reverse", bwd_kernel, bwd_ms, FLOPS_BWD, bwd_tf, bwd_exec_tf, bwd_node_frac,
                bwd_fixed, BWD_PER_NODE)
     else:
-        dom = ("forward", "k_gamma_fwd", fwd_ms, FLOPS_FWD, fwd_tf, fwd_exec_tf, fwd_node_frac,
+        dom = ("forward", fwd_kernel, fwd_ms, FLOPS_FWD, fwd_tf, fwd_exec_tf, fwd_node_frac,
                fwd_fixed, fwd_node)
     # HBM bytes of the dominant kernel from the copy-calibrated counter runs of this workload,
     # stored per step together with the kernel's launches per step (the reverse runs its aux
     # slabs in several launches when their moments do not fit one launch's budget).
-    traffic, launches = None, 1
+    counted = s.name if s.eps == 1e-7 else None          # the list the counter runs were taken on
+    traffic, launches, traffic_commit = None, 1, None
     tfile = ROOT / "profiles" / "three_centre_traffic.json"
     if tfile.exists():
-        rec = json.loads(tfile.read_text()).get(s.name, {}).get(dom[1])
+        rec = json.loads(tfile.read_text()).get(counted, {}).get(dom[1])
         if rec:
             launches = int(rec.get("launches_per_step", 1))
             traffic = (rec["fetch_bytes"] + rec["write_bytes"]) / launches
+            traffic_commit = rec["commit"]
 
     # ------------------------------------------------------------------ CPU baseline (oracle)
     cpu = None
@@ -309,7 +314,8 @@ def main() -> int:
         "roofline": {"bound": "valu", "kernel": f"three-centre {dom[0]} ({dom[1]})",
                      "achieved": dom[5] / 1e12, "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s",
                      "frac": dom[5] / PEAK_FP64, "frac_basis": "evaluated nodes",
-                     "traffic": traffic, "launches_per_step": launches,
+                     "traffic": traffic, "traffic_commit": traffic_commit,
+                     "launches_per_step": launches,
                      "flops_per_integral": dom[7], "flops_per_evaluated_node": dom[8],
                      "integrals_per_launch": integrals / launches,
                      "evaluated_nodes_per_launch": dom[6] * NODES * integrals / launches,
@@ -318,7 +324,7 @@ def main() -> int:
                      "algorithmic_achieved": dom[4] / 1e12,
                      "algorithmic_frac": dom[4] / PEAK_FP64,
                      "algorithmic_flops_per_integral": dom[3],
-                     "fp64_counters": counter_record(s.name, dom[1]),
+                     "fp64_counters": counter_record(counted, dom[1]),
                      "note": "FP64 compute bound on the vector ALUs (VALU; MI355X FP64 vector "
                              "peak 78.6 TFLOP/s, no MFMA: the work is elementwise). achieved "
                              "counts the work the kernel has to do: flops_per_integral for "
@@ -733,8 +739,9 @@ def run_exchange(args) -> int:
     dom_alg_tf = dom[3] / (dom[1] * 1e-3)
     # HBM bytes per launch (one aux chunk) of the dominant kernel, from the counter runs
     traffic, counters = None, None
-    tkey = {"three-centre reverse": "k_gamma_bwd_lane_u",
-            "three-centre block": "k_exch_block_pairs"}.get(dom[0].split(" (")[0])
+    tkey = {"three-centre reverse": "k_gamma_bwd_lane_u" + ("_sets" if share > 1 else ""),
+            "three-centre block": "k_exch_block_" + ("sets" if share > 1 else "pairs")}.get(
+                dom[0].split(" (")[0])
     tfile = ROOT / "profiles" / "exchange_traffic.json"
     if tkey and tfile.exists():
         rec = json.loads(tfile.read_text()).get(s.name, {}).get(tkey)
