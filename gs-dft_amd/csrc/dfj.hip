@@ -693,8 +693,8 @@ __global__ __launch_bounds__(256) void k_gamma_fwd_pairs(int64_t n, int64_t pair
 // kFwdRecs records are kFwdRecs / NB groups. Bound by its VALU instructions like
 // k_gamma_fwd_pairs: 26.5 a node (22 + NB; the weights' signs no longer let one ride in the
 // exponent) against 22 for each node of each scale, for about half the nodes (C20H42, 590 k pairs,
-// four scales: 44.5 -> 37.9 ms; water octamer 6.05 -> 4.36). One node a step, with its constants
-// moved between register sets, took 39.1 and 4.62. partial[g * N + slot] is the sum without KN_P
+// four scales: 44.5 -> 38.2 ms; water octamer 6.05 -> 4.5, of which the lists' tail, kSetTail, takes 0.4
+// and 0.1). One node a step, with its constants moved between register sets, took 3% and 6% longer. partial[g * N + slot] is the sum without KN_P
 // (k_slot_sum multiplies it in).
 template <int NB>
 __global__ __launch_bounds__(256) void k_gamma_fwd_sets(int64_t n, int64_t pairs,
@@ -1147,7 +1147,7 @@ __global__ __launch_bounds__(256, kSet && kLaneU ? 3 : kSet ? 4 : 1) void k_gamm
     };
     // kSet: the records are groups of shared node lists (nodeset.hip). With one cotangent per aux
     // function each list's weights are already the sum of its functions' (C20H42, four scales:
-    // 68.4 -> 50.5 ms; water octamer 9.09 -> 5.86; 52.3 and 6.07 with one node a step), with kLaneU
+    // 68.4 -> 48.6 ms; water octamer 9.09 -> 5.8; 4% longer with one node a step), with kLaneU
     // the lane forms them node by node from its four cotangents.
     if constexpr (kSet) {
         for (int64_t p = p0; p < p1; ++p) {

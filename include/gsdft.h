@@ -159,7 +159,7 @@ int gsdft_gamma(int64_t M, const double* quat, const double* log_scale, const do
  * cannot allocate device memory (HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc). Sizes whose gsdft_gamma workspace exceeds 64 MiB (gsdft_gamma_workspace_size) are
  * refused with GSDFT_ERR_ARG before any launch: the water octamer (M = 600, N_aux = 2,400,
- * n = 166,915 pairs, 49.8 MiB) fits, C20H42 (n = 590,298, 179 MiB) does not.
+ * n = 166,915 pairs, 49.4 MiB) fits, C20H42 (n = 590,298, 174 MiB) does not.
  * Every call on one GPU shares that GPU's scratch and leaves its contents behind, so calls that
  * overlap on one GPU (several streams or host threads at once) race; serialise them. */
 int gsdft_gamma_noalloc(int64_t M, const double* quat, const double* log_scale,
@@ -175,10 +175,11 @@ int gsdft_gamma_noalloc(int64_t M, const double* quat, const double* log_scale,
  * gs_dft/coulomb/ri.py:436-469, :190-222, gs_dft/coulomb/stream.py:203-215 and
  * gs_dft/basis/spectral.py:33-40,72-82 (gs_dft/ks/train.py:367-373 holds the aux constant).
  * The pass is cut into slabs of at most 4096 aux functions, so that each slab's records stay in
- * one XCD's L2 while the workgroups running together walk it; the workspace holds 200 bytes per
+ * one XCD's L2 while the workgroups running together walk it, and into more on lists that leave few
+ * workgroups; the workspace holds 200 bytes per
  * pair for the slabs of one launch (all of them while that fits in 5 GiB, else as many as fit and
  * at least one, the launches adding their moments to running sums): 4.5 GB for 11.2 M pairs and
- * 80,000 aux functions, 4.1 GB for 20.6 M. */
+ * 80,000 aux functions, 4.1 GB for 20.6 M, 0.94 GB for 590 k and 8,000 (8 slabs). */
 int gsdft_gamma_vjp_workspace_size(int64_t M, int64_t k, int64_t N, int64_t n, size_t* bytes);
 int gsdft_gamma_vjp(int64_t M, const double* quat, const double* log_scale,
                     const double* centers, int64_t k, const double* C, const double* occ,
@@ -228,7 +229,8 @@ int gsdft_external_energy(int64_t M, const double* quat, const double* log_scale
  * (a|b) the pair-pair Coulomb integral at the reference's 20-node rule, and J (n) = sum_b (a|b)
  * Pw_b (0 on zero-weight entries). Optional: the gradients w.r.t. quat, log_scale, centers and
  * C (all four, with the pair index of the same n entries; grads = 1 in the workspace query).
- * O(n^2) work. Replaces screened_coulomb_energy / full_eri_block_schur and JAX's reverse pass
+ * O(n^2) work; workspace with gradients 1.3 GB at 28 k pairs, 7.5 GB at 167 k, 9.5 GB at 590 k.
+ * Replaces screened_coulomb_energy / full_eri_block_schur and JAX's reverse pass
  * through them, gs_dft/coulomb/stream.py:249-281,296-320 (ScreenedExactCoulomb,
  * gs_dft/ks/terms.py:193-205). */
 int gsdft_exact_coulomb_workspace_size(int64_t M, int64_t k, int64_t n, int grads,

@@ -288,9 +288,10 @@ def test_streamed_exact_term_equals_the_screened_full_list(g, wl, cuda):
 @pytest.mark.parametrize("M,n_atoms", [(60, 3), (190, 6), (330, 9)])
 def test_exact_slab_lengths(g, wl, orc, cuda, M, n_atoms):
     """The symmetric passes shorten their ket slabs on short lists (768 kets down to 48): lists of
-    1.8 k, 17 k and 46 k pairs run on different slab lengths, with ragged last slabs and bra groups.
-    The energy-only pass agrees with the reverse's E_J, and J on sampled pairs, the last ones and
-    the ones at 256-bra edges included, with oracle rows (1e-12, the bar of the full-size test)."""
+    1.8 k, 17 k and 46 k pairs run on different slab lengths, with ragged last slabs and bra groups,
+    the longest in two bands of 32768 bras. The energy-only pass agrees with the reverse's E_J, and J
+    on sampled pairs, the last ones and the ones at 256-bra and band edges included (these lists keep
+    their order), with oracle rows (1e-12, the bar of the full-size test)."""
     s = wl.make_small(M, 5, n_atoms=n_atoms, seed=8, spread=2.5)
     pi, pj, w, _ = orc.neighbor_pairs(s.quat, s.log_scale, s.centers, s.eps, None, True)
     n = len(pi)
@@ -304,7 +305,7 @@ def test_exact_slab_lengths(g, wl, orc, cuda, M, n_atoms):
         J = _np(g.screened_coulomb_J(basis, C, s.occ, pi, pj, valid=w))
     rel = abs(E_fwd.item() - E_rev.item()) / abs(E_rev.item())
     Pw = w * np.sum(s.occ[None, :] * s.C[pi] * s.C[pj], axis=1)
-    sel = np.unique([0, 255, 256, n // 2, n - 257, n - 1])
+    sel = np.unique([0, 255, 256, n // 2, n - 257, n - 1, min(32767, n - 1), min(32768, n - 1)])
     rows = orc.eri_block(s.quat, s.log_scale, s.centers, pi[sel], pj[sel], pi, pj)
     bound = 1e-12 * (np.abs(rows) @ np.abs(Pw))
     err = float(np.max(np.abs(J[sel] - rows @ Pw) / bound))

@@ -1,5 +1,5 @@
 """Slot order of the pairs. Lists of up to 65,536 entries keep their own order where it runs over i in
-ascending order and are put into the order of the slot keys otherwise; longer lists are always sorted.
+ascending order and are brought into ascending i otherwise; longer lists are sorted by the slot keys.
 A wave leaves a node loop when all of its 64 pairs are out of reach, so on a long molecule the nodes
 evaluated show whether neighbours share waves: the same pairs shuffled may not cost more than a tenth
 more nodes than ascending (in shuffled order they cost 1.3 to 2 times as many).
